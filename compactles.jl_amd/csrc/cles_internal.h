@@ -62,7 +62,7 @@ struct LineDev {
     int periodic;
     int closed;     // both edges closed (one rank, non-periodic)
     int P;          // chunks per line (power of two)
-    int nsteps;     // log2(P)
+    int nsteps;     // PCR steps: log2(P), or fewer where the later blocks are below rounding
     int m;          // base chunk length
     int extra;      // first `extra` chunks have length m + 1
     const double *coef64;  // [0..8) ci, [8] a0, [16..80) clo[8][8], [80..144) chi[8][8]

@@ -1,0 +1,28 @@
+"""GPU parity of the line operators at the sizes where a kernel or a plan
+changes form: truncated reductions, chunk capacities, uneven chunks, ragged
+lane counts.  Against the oracle's apply_along! on the same seeded inputs, with
+the operators' bar: FP64 normwise <= 1e-12, FP32 <= 2e-5."""
+import numpy as np
+import pytest
+
+import helpers as Hh
+from test_gpu_operators import _gpu_apply, _oracle_apply, ctx  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("name", ["lele_d1_6", "lele_d1_10", "compact_filter"])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("dim,n", [(1, (1000, 5, 3)), (2, (6, 900, 2)), (3, (7, 2, 520))])
+def test_truncated_reduction(ctx, name, periodic, dim, n):  # noqa: F811
+    """Lines long enough that the reduction stops before log2(chunks) steps:
+    a random line, and one spike of 1e8 over a random line (the interface values
+    then span eight decades; the bar is relative to the largest value)."""
+    f = Hh.random_field(n, seed=21)
+    g = f.copy()
+    at = [0, 0, 0]
+    at[dim - 1] = n[dim - 1] // 3
+    g[tuple(at)] = 1e8
+    for a in (f, g):
+        ref = _oracle_apply(name, dim, n, periodic, 0.01, a)
+        assert Hh.relerr(_gpu_apply(ctx, name, dim, n, periodic, 0.01, a), ref) <= 1e-12
