@@ -71,6 +71,9 @@ struct LineDev {
     const float *row32;
     const double *pcr;     // per step s, chunk k: alpha, beta (B*B each, row-major);
                            // then per chunk the final inverse block
+    int cap;               // chunk capacity of the kernels: 8, 16 or 32 >= the longest chunk
+    const double *rowu64;  // per-chunk blocks [(k * nrow + field) * cap + t] of the row constants; rows
+    const float *rowu32;   //   past a chunk's length are zero, and so is its last row's coupling C
     const double *rowt64;  // chunk-major copy of the per-row constants (ragged plans):
     const float *rowt32;   //   [(field * RAG_MAX_CHUNK + t) * P + k] = row of point t of chunk k
 };
@@ -94,7 +97,7 @@ struct HostPlan {
 struct LineTables {
     LineDev dev{};
     std::vector<unsigned char> image;
-    size_t o_coef32 = 0, o_row64 = 0, o_row32 = 0, o_pcr = 0, o_rowt64 = 0, o_rowt32 = 0;
+    size_t o_coef32 = 0, o_row64 = 0, o_row32 = 0, o_pcr = 0, o_rowu64 = 0, o_rowu32 = 0, o_rowt64 = 0, o_rowt32 = 0;
 };
 // chunk_major: also store the chunk-major row tables of the ragged kernel
 // (RAG_MAX_CHUNK rows per chunk; max_chunk must not exceed it).

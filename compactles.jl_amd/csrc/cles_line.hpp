@@ -19,6 +19,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "cles_internal.h"
 
 // Multiply-adds in the line kernels are written as explicit fma where they
@@ -723,21 +725,406 @@ __device__ __forceinline__ double corrected(const LineDev &p, int g, T y, const 
 }
 
 // ---------------------------------------------------------------------------
-// y / z sweeps: lanes along x, one chunk row per load instruction.
-// Line dimension stride sd, outer dimension stride so; block = Lx lanes x P
-// chunks.  UNI: Lx == 64, so each wave holds one chunk and every per-row
-// constant is wave-uniform (scalar loads).
+// y / z sweeps, one chunk per wave: 64 lanes along x with V adjacent lines per
+// lane, so a row is one contiguous segment of 64 V values and every per-row
+// constant is wave-uniform.
+//
+// Bound: HBM for FP64 and large FP32 grids, instruction issue before that.  The
+// row constants come from per-chunk blocks padded with zeros (LineDev::rowu64),
+// so the sweeps run CL unconditional steps: a row past the chunk's length only
+// multiplies by zeros, and the last row's coupling is stored as zero.  Every
+// window load is unconditional too, from the row wrapped or clamped into the
+// line (scalar arithmetic), and the closure rows, the zero halo of a closed
+// line and the ends of a chunk shorter than CL are fixed up in branches that
+// only their own waves take.  FULL: every chunk holds CL points.
+//
+// V = 2 (float): two lines per lane make the row segments 512 bytes, as for
+// double, and halve the instructions per point.
+//
+// The C6 store kernel of 32-point chunks went from 4777 to 1237 instructions
+// (2375 with uneven chunks).  Measured before / after, one pass: C6 gradient of
+// 384^3 FP32 665 / 578 us, in-place C8 filter of 256 x 255 x 257 FP64 185 / 176
+// us, C10 gradient of 250 x 199 x 180 FP32 256 / 224 us; 40 Taylor-Green steps
+// at 64^3 FP64 31.9 / 28.7 ms, 120 x 97 x 81 FP32 81.8 / 73.4 ms.
 // ---------------------------------------------------------------------------
-template <typename T, int Q, int M, int SYM, int EPI, bool UNI, int CL = MC, bool NTS = false>
-__global__ void __launch_bounds__(UNI && Q == 1 ? 1024 : 512, UNI ? (Q == 2 ? 4 : 1) : 3) k_line_yz(LineDev p, const T *__restrict__ f, int sd, int64_t so,
+// Blocks are dispatched round-robin over the 8 XCDs, each with its own L2;
+// renumbered so that every XCD sweeps one contiguous slab.  For y sweeps, whose
+// blocks share memory rows, this is the better order (four-field C6 derivative
+// at 256^3 FP64: 226 us round-robin, 201 us in slabs); z sweeps, whose
+// neighbouring blocks are adjacent in memory, keep the dispatch order (a copy
+// with their access pattern takes 196 us so and 208 us in slabs).
+__device__ __forceinline__ unsigned xcd_slab(unsigned b, unsigned nb)
+{
+    const unsigned nfull = nb & ~7u;
+    return b < nfull ? (b & 7u) * (nfull >> 3) + (b >> 3) : b;
+}
+
+// Loads through the constant address space: wave-uniform addresses become
+// scalar loads wherever they stand (tables are never written by a kernel).
+template <typename T> __device__ __forceinline__ T cload(const T *ptr)
+{
+    return *(const __attribute__((address_space(4))) T *)ptr;
+}
+template <typename T> __device__ __forceinline__ const T *rowup(const LineDev &p);
+template <> __device__ __forceinline__ const double *rowup<double>(const LineDev &p) { return p.rowu64; }
+template <> __device__ __forceinline__ const float *rowup<float>(const LineDev &p) { return p.rowu32; }
+
+// V adjacent values as one access; elements are only element-aligned (odd
+// strides and halos), which the memory unit takes for global accesses.
+template <typename T, int V> struct Pack {
+    typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+};
+template <int V, typename T> __device__ __forceinline__ void vload(const T *ptr, T (&v)[V])
+{
+    if constexpr (V == 1) {
+        v[0] = *ptr;
+    } else {
+        const typename Pack<T, V>::type x = *(const typename Pack<T, V>::type *)ptr;
+#pragma unroll
+        for (int i = 0; i < V; i++) v[i] = x[i];
+    }
+}
+template <int V, bool NT, typename T> __device__ __forceinline__ void vstore(T *ptr, const T (&v)[V])
+{
+    if constexpr (V == 1) {
+        if constexpr (NT) __builtin_nontemporal_store(v[0], ptr);
+        else *ptr = v[0];
+    } else {
+        typename Pack<T, V>::type x;
+#pragma unroll
+        for (int i = 0; i < V; i++) x[i] = v[i];
+        if constexpr (NT) __builtin_nontemporal_store(x, (typename Pack<T, V>::type *)ptr);
+        else *(typename Pack<T, V>::type *)ptr = x;
+    }
+}
+
+// The epilogue of NB rows of V adjacent points: element o[i] .. o[i] + V - 1
+// takes v[.][i].  Every input is loaded before any output is stored.  Row i is
+// stored where ok[i] (wave-uniform); the offsets of other rows are in bounds.
+template <typename T, int EPI, int NB, int V, bool NT>
+__device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&o)[NB], const T (&v)[V][NB],
+                                              const bool (&ok)[NB])
+{
+    if constexpr (EPI == EPI_ART_MULTI) {
+        if (e.kind == EPI_ART_MUBETA) epilogue_rows<T, EPI_ART_MUBETA, NB, V, NT>(e, o, v, ok);
+        else if (e.kind == EPI_ART_KAPPA) epilogue_rows<T, EPI_ART_KAPPA, NB, V, NT>(e, o, v, ok);
+        else epilogue_rows<T, EPI_ART_D, NB, V, NT>(e, o, v, ok);
+        return;
+    }
+    if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_NEG) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (!ok[i]) continue;
+            T x[V];
+#pragma unroll
+            for (int j = 0; j < V; j++) x[j] = EPI == EPI_STORE_NEG ? -v[j][i] : v[j][i];
+            vstore<V, NT>((T *)e.out + o[i], x);
+        }
+    } else if constexpr (EPI == EPI_SUB) {
+        T a[NB][V];
+#pragma unroll
+        for (int i = 0; i < NB; i++) vload<V>((const T *)e.out + o[i], a[i]);
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (!ok[i]) continue;
+#pragma unroll
+            for (int j = 0; j < V; j++) a[i][j] = a[i][j] - v[j][i];
+            vstore<V, false>((T *)e.out + o[i], a[i]);
+        }
+    } else if constexpr (EPI == EPI_LSRK) {
+        const T *acc = (const T *)e.a0;
+        T a[NB][V];
+        double du[NB][V], q[NB][V];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (acc) vload<V>(acc + o[i], a[i]);
+            vload<V>((const double *)e.du + o[i], du[i]);
+            vload<V>((const double *)e.Q + o[i], q[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (!ok[i]) continue;
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                const double dq = acc ? (double)(a[i][j] - v[j][i]) : -(double)v[j][i];
+                du[i][j] = fma(e.dt, dq, e.c0 * du[i][j]);
+                q[i][j] = fma(e.c1, du[i][j], q[i][j]);
+            }
+            vstore<V, false>(e.du + o[i], du[i]);
+            vstore<V, false>(e.Q + o[i], q[i]);
+        }
+    } else if constexpr (EPI == EPI_ART_MUBETA) {
+        T r[NB][V];
+#pragma unroll
+        for (int i = 0; i < NB; i++) vload<V>((const T *)e.a0 + o[i], r[i]);
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (!ok[i]) continue;
+            T mu[V], be[V];
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                const T rs = r[i][j] * (v[j][i] > T(0) ? v[j][i] : T(0));
+                mu[j] = (T)e.c0 * rs;
+                be[j] = (T)e.c1 * rs;
+            }
+            vstore<V, false>((T *)e.out + o[i], mu);
+            vstore<V, false>((T *)e.out2 + o[i], be);
+        }
+    } else if constexpr (EPI == EPI_ART_KAPPA) {
+        T r[NB][V], cc[NB][V], tt[NB][V];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            vload<V>((const T *)e.a0 + o[i], r[i]);
+            vload<V>((const T *)e.a1 + o[i], cc[i]);
+            vload<V>((const T *)e.a2 + o[i], tt[i]);
+        }
+        const T eps = sizeof(T) == 8 ? (T)2.220446049250313e-16 : (T)1.1920929e-07f;
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (!ok[i]) continue;
+            T ka[V];
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                const T scale = r[i][j] * cc[i][j] / (tt[i][j] > eps ? tt[i][j] : eps);
+                ka[j] = (T)e.c0 * scale * (v[j][i] > T(0) ? v[j][i] : T(0));
+            }
+            vstore<V, false>((T *)e.out + o[i], ka);
+        }
+    } else if constexpr (EPI == EPI_ART_D) {
+        T cc[NB][V];
+#pragma unroll
+        for (int i = 0; i < NB; i++) vload<V>((const T *)e.a1 + o[i], cc[i]);
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (!ok[i]) continue;
+            T dd[V];
+#pragma unroll
+            for (int j = 0; j < V; j++) dd[j] = (T)e.c0 * cc[i][j] * (v[j][i] > T(0) ? v[j][i] : T(0));
+            vstore<V, false>((T *)e.out + o[i], dd);
+        }
+    } else {
+        // gated kinds: the flag and dt of the launch, or of each point's instance
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            int64_t oj[NB];
+            T vj[NB];
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                oj[i] = o[i] + j;
+                vj[i] = v[j][i];
+            }
+            epilogue_batch<T, EPI, NB, false>(e, oj, vj, ok);
+        }
+    }
+}
+
+template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V, bool NTS>
+__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
+k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
+           LineFields mf)
+{
+    select_field<T, EPI>(mf, f, e);
+    extern __shared__ double smem[];
+    constexpr int B = 2 * Q, NROW = Q == 1 ? (int)R1_N : (int)R2_N;
+    const int P = p.P, n = p.n;
+    const int NT = 64 * P;
+    const int lane = (int)(threadIdx.x & 63);
+    const int k = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned blk = slabs ? xcd_slab(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int xb = blk % nxb;
+    const int64_t ob = blk / nxb;
+    const int x0 = (xb * 64 + lane) * V;
+    const bool valid = x0 < nlane;                  // nlane is a multiple of V
+    const int xi = valid ? x0 : nlane - V;
+    const int64_t off = ob * so;
+    const T *fl = f + off;
+    const int s = FULL ? k * CL : k * p.m + min(k, p.extra);
+    const int len = FULL ? CL : p.m + (k < p.extra ? 1 : 0);
+    const bool lo = p.closed && k == 0, hi = p.closed && k == P - 1;
+
+    T fv[V][CL + 2 * M];
+#pragma unroll
+    for (int t = -M; t < CL + M; t++) {
+        // the wrapped row, or for a closed line any row of it (fixed up below)
+        int r = s + t;
+        if (t < 0) r = r < 0 ? r + n : r;
+        if (!FULL || t >= CL) r = r >= n ? r - n : r;
+        if (!FULL) r = r >= n ? n - 1 : r;          // rows past a short last chunk
+        T x[V];
+        vload<V>(fl + (int64_t)r * sd + xi, x);
+#pragma unroll
+        for (int j = 0; j < V; j++) fv[j][t + M] = x[j];
+    }
+    if (lo) {
+#pragma unroll
+        for (int t = 0; t < M; t++)
+#pragma unroll
+            for (int j = 0; j < V; j++) fv[j][t] = T(0);
+    }
+    if (hi) {
+#pragma unroll
+        for (int t = 0; t < CL + M; t++)
+#pragma unroll
+            for (int j = 0; j < V; j++) fv[j][t + M] = t >= len ? T(0) : fv[j][t + M];
+    }
+
+    const T *cf = coefp<T>(p);
+    T d[V][CL];
+    {
+        T ci[M];
+#pragma unroll
+        for (int m = 0; m < M; m++) ci[m] = cload(cf + COEF_CI + m);
+        const T a0 = cload(cf + COEF_A0);
+#pragma unroll
+        for (int j = 0; j < V; j++)
+#pragma unroll
+            for (int t = 0; t < CL; t++) d[j][t] = rhs_row<T, M, SYM>(fv[j], t + M, ci, a0);
+    }
+    if (lo) {
+#pragma unroll
+        for (int t = 0; t < NCMAX; t++) {
+            if (t >= p.nc) continue;
+            const T *cr = cf + COEF_CLO + t * 8;
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                T acc = cload(cr) * fv[j][M];
+#pragma unroll
+                for (int kap = 1; kap < 8; kap++) acc = fma(cload(cr + kap), fv[j][kap + M], acc);
+                d[j][t] = acc;
+            }
+        }
+    }
+    if (hi) {
+        T fe[V][8];
+#pragma unroll
+        for (int kap = 0; kap < 8; kap++) {
+            T x[V];
+            vload<V>(fl + (int64_t)(kap < n ? n - 1 - kap : 0) * sd + xi, x);
+#pragma unroll
+            for (int j = 0; j < V; j++) fe[j][kap] = kap < n ? x[j] : T(0);
+        }
+#pragma unroll
+        for (int jr = 0; jr < NCMAX; jr++) {
+            if (jr >= p.nc) continue;
+            const T *cr = cf + COEF_CHI + jr * 8;
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                T acc = cload(cr) * fe[j][0];
+#pragma unroll
+                for (int kap = 1; kap < 8; kap++) acc = fma(cload(cr + kap), fe[j][kap], acc);
+#pragma unroll
+                for (int t = 0; t < CL; t++) d[j][t] = t == len - 1 - jr ? acc : d[j][t];
+            }
+        }
+    }
+
+    // chunk sweeps (src/tridiag.jl:46-57, src/banded.jl:63-80)
+    const T *rw = rowup<T>(p) + (size_t)k * NROW * CL;
+    if constexpr (Q == 1) {
+        const T *rl = rw + R1_L * CL, *rdi = rw + R1_DINV * CL, *rc = rw + R1_C * CL;
+#pragma unroll
+        for (int t = 1; t < CL; t++)
+#pragma unroll
+            for (int j = 0; j < V; j++) d[j][t] = fma(-cload(rl + t), d[j][t - 1], d[j][t]);
+#pragma unroll
+        for (int j = 0; j < V; j++) d[j][CL - 1] *= cload(rdi + CL - 1);
+#pragma unroll
+        for (int t = CL - 2; t >= 0; t--)
+#pragma unroll
+            for (int j = 0; j < V; j++) d[j][t] = fma(-cload(rc + t), d[j][t + 1], d[j][t]) * cload(rdi + t);
+    } else {
+        const T *l1 = rw + R2_L1 * CL, *l2 = rw + R2_L2 * CL, *u0 = rw + R2_U0INV * CL, *u1 = rw + R2_U1 * CL,
+                *u2 = rw + R2_U2 * CL;
+#pragma unroll
+        for (int t = 0; t < CL - 1; t++)
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                d[j][t + 1] = fma(-cload(l1 + t), d[j][t], d[j][t + 1]);
+                if (t + 2 < CL) d[j][t + 2] = fma(-cload(l2 + t), d[j][t], d[j][t + 2]);
+            }
+#pragma unroll
+        for (int t = CL - 1; t >= 0; t--)
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                T acc = d[j][t];
+                if (t + 1 < CL) acc = fma(-cload(u1 + t), d[j][t + 1], acc);
+                if (t + 2 < CL) acc = fma(-cload(u2 + t), d[j][t + 2], acc);
+                d[j][t] = acc * cload(u0 + t);
+            }
+    }
+
+    // the reduced system, each of the V lines in its own part of the buffers
+    double tp[V][Q], hn[V][Q];
+#pragma unroll
+    for (int j = 0; j < V; j++) {
+        double r[B];
+#pragma unroll
+        for (int i = 0; i < Q; i++) {
+            r[i] = (double)d[j][i];
+            r[Q + i] = (double)d[j][CL - Q + i];
+        }
+        if constexpr (!FULL) {
+#pragma unroll
+            for (int i = 0; i < Q; i++) {
+                T x = d[j][0];
+#pragma unroll
+                for (int t = 1; t < CL; t++) x = t == len - Q + i ? d[j][t] : x;
+                r[Q + i] = (double)x;
+            }
+        }
+        reduced_solve<Q>(p, smem + (size_t)j * 2 * B * NT, NT, 64, k, lane, r, tp[j], hn[j]);
+    }
+    if (!valid) return;
+
+    // spike correction, FP64 as the reduced system
+    const double *rv = p.rowu64 + (size_t)k * NROW * CL;
+    // the Runge-Kutta epilogues hold three inputs per point: four rows at a
+    // time where eight would spill
+    constexpr int NB = (EPI == EPI_LSRK || EPI == EPI_LSRK_DEV) && (CL > 16 || V > 1) ? 4 : 8;
+#pragma unroll
+    for (int b = 0; b < CL; b += NB) {
+        int64_t o[NB];
+        T v[V][NB];
+        bool ok[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const int t = b + i;
+            ok[i] = FULL || t < len;
+            const int r = FULL ? s + t : min(s + t, n - 1);
+            o[i] = off + (int64_t)r * sd + xi;
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                double acc;
+                if constexpr (Q == 1) {
+                    acc = fma(cload(rv + R1_W * CL + t), hn[j][0], cload(rv + R1_V * CL + t) * tp[j][0]);
+                } else {
+                    acc = cload(rv + R2_V0 * CL + t) * tp[j][0];
+                    acc = fma(cload(rv + R2_W0 * CL + t), hn[j][0], acc);
+                    acc = fma(cload(rv + R2_V1 * CL + t), tp[j][1], acc);
+                    acc = fma(cload(rv + R2_W1 * CL + t), hn[j][1], acc);
+                }
+                v[j][i] = (T)((double)d[j][t] - acc);
+            }
+        }
+        epilogue_rows<T, EPI, NB, V, NTS>(e, o, v, ok);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// y / z sweeps on narrow blocks: lanes along x.
+// Line dimension stride sd, outer dimension stride so; block = Lx lanes x P
+// chunks, several chunks per wave: narrow x extents (2-D grids), and lines
+// with too many chunks for 64 lanes.
+// ---------------------------------------------------------------------------
+template <typename T, int Q, int M, int SYM, int EPI, int CL>
+__global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restrict__ f, int sd, int64_t so,
                                                   int nlane, int nxb, int Lx, EpiArgs e, LineFields mf)
 {
     select_field<T, EPI>(mf, f, e);
     extern __shared__ double smem[];
     const int NT = Lx * p.P;
-    const int lane = UNI ? (int)(threadIdx.x & 63) : (int)(threadIdx.x % Lx);
-    int k = UNI ? (int)(threadIdx.x >> 6) : (int)(threadIdx.x / Lx);
-    if constexpr (UNI) k = __builtin_amdgcn_readfirstlane(k);
+    const int lane = (int)(threadIdx.x % Lx);
+    const int k = (int)(threadIdx.x / Lx);
     const int xb = blockIdx.x % nxb;
     const int64_t ob = blockIdx.x / nxb;
     const int xi = xb * Lx + lane;
@@ -749,44 +1136,25 @@ __global__ void __launch_bounds__(UNI && Q == 1 ? 1024 : 512, UNI ? (Q == 2 ? 4 
     const int len = p.m + (k < p.extra ? 1 : 0);
 
     T fv[CL + 2 * M];
-    if constexpr (UNI) {
-        // one chunk per wave: the branches below are uniform
+    // lanes of one wave own different chunks, so branching per load
+    // would diverge: every load is unconditional, from the wrapped row
+    // clamped into the line (and the last lane of the row set for lanes
+    // past it), and its value selected afterwards
+    const T *fa = f + (int64_t)(valid ? xi : nlane - 1) + ob * so;
 #pragma unroll
-        for (int t = -M; t < CL + M; t++) {
-            T val = T(0);
-            if (valid && t < len + M) {
-                int r = s + t;
-                bool ok = true;
-                if (r < 0) {
-                    if (p.periodic) r += n; else ok = false;
-                } else if (r >= n) {
-                    if (p.periodic) r -= n; else ok = false;
-                }
-                if (ok) val = fl[r * sd];
-            }
-            fv[t + M] = val;
+    for (int t = -M; t < CL + M; t++) {
+        int r = s + t;
+        bool ok = valid && t < len + M;
+        if (r < 0) {
+            ok = ok && p.periodic;
+            r += n;
+        } else if (r >= n) {
+            ok = ok && p.periodic;
+            r -= n;
         }
-    } else {
-        // lanes of one wave own different chunks, so branching per load
-        // would diverge: every load is unconditional, from the wrapped row
-        // clamped into the line (and the last lane of the row set for lanes
-        // past it), and its value selected afterwards
-        const T *fa = f + (int64_t)(valid ? xi : nlane - 1) + ob * so;
-#pragma unroll
-        for (int t = -M; t < CL + M; t++) {
-            int r = s + t;
-            bool ok = valid && t < len + M;
-            if (r < 0) {
-                ok = ok && p.periodic;
-                r += n;
-            } else if (r >= n) {
-                ok = ok && p.periodic;
-                r -= n;
-            }
-            const int rc = r < 0 ? 0 : (r > n - 1 ? n - 1 : r);
-            const T val = fa[(int64_t)rc * sd];
-            fv[t + M] = ok ? val : T(0);
-        }
+        const int rc = r < 0 ? 0 : (r > n - 1 ? n - 1 : r);
+        const T val = fa[(int64_t)rc * sd];
+        fv[t + M] = ok ? val : T(0);
     }
     T fe[8];
 #pragma unroll
@@ -800,8 +1168,8 @@ __global__ void __launch_bounds__(UNI && Q == 1 ? 1024 : 512, UNI ? (Q == 2 ? 4 
     Chunk<T, Q, M, SYM, CL> ch;
     ch.rhs(p, k, len, fv, fe);
     // grouped row loads where they fit the 128 registers of a 1024-thread
-    // block (chunks of up to 16 points); wave-uniform rows (UNI) are scalar loads
-    constexpr bool GRP = !UNI && CL <= 16;
+    // block (chunks of up to 16 points)
+    constexpr bool GRP = CL <= 16;
     constexpr int G = CL <= 8 ? CL : 4;
     if constexpr (GRP)
         solve_grouped<T, Q, CL, G>(ch.d, len, RowsClamped<T>{rowp<T>(p), n, s});
@@ -809,7 +1177,7 @@ __global__ void __launch_bounds__(UNI && Q == 1 ? 1024 : 512, UNI ? (Q == 2 ? 4 
         ch.solve(p, s, len);
     double r[2 * Q], tp[Q], hn[Q];
     ch.ends(len, r);
-    reduced_solve<Q, !UNI && Q == 1 && sizeof(T) == 8>(p, smem, NT, Lx, k, lane, r, tp, hn);
+    reduced_solve<Q, Q == 1 && sizeof(T) == 8>(p, smem, NT, Lx, k, lane, r, tp, hn);
     if (!valid) return;
     if constexpr (GRP) {
         correct_grouped<T, Q, CL, G>(ch.d, len, RowsClamped<double>{p.row64, n, s}, tp, hn);
@@ -832,7 +1200,7 @@ __global__ void __launch_bounds__(UNI && Q == 1 ? 1024 : 512, UNI ? (Q == 2 ? 4 
             o[i] = off + (int64_t)(s + b + i) * sd;
             v[i] = ch.d[b + i];
         }
-        epilogue_batch<T, EPI, NB, NTS>(e, o, v, ok);
+        epilogue_batch<T, EPI, NB>(e, o, v, ok);
     }
 }
 
@@ -1414,33 +1782,49 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         const int64_t nouter = dim == 2 ? v.n[2] : v.n[1];
         if ((int64_t)(p.n - 1) * sd > INT32_MAX) throw Error{CLES_ERR_UNSUPPORTED, "array too large for 32-bit line offsets"};
         if (nlane >= 48 && 64 * P <= maxNT) {
-            const int Lx = 64, NT = 64 * P;
-            const int nxb = (int)((nlane + Lx - 1) / Lx);
-            const size_t shm = (size_t)2 * B * NT * sizeof(double);
+            const int NT = 64 * P;
             // The z sweep's plain stores take the non-temporal hint when the launch
             // writes more than the 256 MB Infinity Cache holds (the outputs are
             // evicted before they are read again); the x and y sweeps measured
             // faster without it.
-            const bool narrow = p.m + (p.extra ? 1 : 0) <= 16;
-            bool nts = false;
+            const bool nts = dim == 3 && (EPI == EPI_STORE || EPI == EPI_STORE_NEG) &&
+                             (double)v.n[0] * v.n[1] * v.n[2] * sizeof(T) * nf > 256.0 * 1024 * 1024;
+            const bool full = p.extra == 0 && p.m == p.cap;
+            auto go = [&](auto kern, int V) {
+                const int nxb = (int)((nlane + 64 * V - 1) / (64 * V));
+                const size_t shm = (size_t)2 * B * NT * V * sizeof(double);
+                hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf), dim3(NT), shm, st, p, f, (int)sd, so,
+                                   (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf);
+            };
+            auto pick = [&](auto cl, auto vv, auto nt) {
+                if (full) go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, true, vv.value, nt.value>, vv.value);
+                else go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, false, vv.value, nt.value>, vv.value);
+            };
+            using std::integral_constant;
+            auto capd = [&](auto vv, auto nt) {
+                if (p.cap == 8) pick(integral_constant<int, 8>{}, vv, nt);
+                else if (p.cap == 16) pick(integral_constant<int, 16>{}, vv, nt);
+                else pick(integral_constant<int, MC>{}, vv, nt);
+            };
+            // two lines per lane in FP32 where the launch still has two blocks
+            // per CU (the row width must be even)
+            bool two = false;
+            if constexpr (sizeof(T) == 4 && Q == 1)
+                two = nlane % 2 == 0 && ((nlane + 127) / 128) * nouter * (int64_t)nf >= 512;
             if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_NEG) {
-                nts = dim == 3 && (double)v.n[0] * v.n[1] * v.n[2] * sizeof(T) * nf > 256.0 * 1024 * 1024;
-                if (nts && narrow)
-                    hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, true, 16, true>), dim3((unsigned)(nxb * nouter), nf),
-                                       dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
-                else if (nts)
-                    hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, true, MC, true>), dim3((unsigned)(nxb * nouter), nf),
-                                       dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
+                if (nts) {
+                    if constexpr (sizeof(T) == 4 && Q == 1) {
+                        if (two) capd(integral_constant<int, 2>{}, std::true_type{});
+                    }
+                    if (!two) capd(integral_constant<int, 1>{}, std::true_type{});
+                }
             }
-            if (!nts && p.m + (p.extra ? 1 : 0) <= 8)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, true, 8>), dim3((unsigned)(nxb * nouter), nf), dim3(NT),
-                                   shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
-            else if (!nts && narrow)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, true, 16>), dim3((unsigned)(nxb * nouter), nf), dim3(NT),
-                                   shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
-            else if (!nts)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, true>), dim3((unsigned)(nxb * nouter), nf), dim3(NT),
-                                   shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
+            if (!nts) {
+                if constexpr (sizeof(T) == 4 && Q == 1) {
+                    if (two) capd(integral_constant<int, 2>{}, std::false_type{});
+                }
+                if (!two) capd(integral_constant<int, 1>{}, std::false_type{});
+            }
         } else {
             int Lx = 64;
             while (Lx * P > 512 && Lx > 1) Lx /= 2;
@@ -1454,13 +1838,13 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             const size_t shm = (size_t)2 * B * NT * sizeof(double);
             const int cl = p.m + (p.extra ? 1 : 0);
             if (cl <= 8)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, false, 8>), dim3((unsigned)(nxb * nouter), nf),
+                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 8>), dim3((unsigned)(nxb * nouter), nf),
                                    dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
             else if (cl <= 16)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, false, 16>), dim3((unsigned)(nxb * nouter), nf),
+                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 16>), dim3((unsigned)(nxb * nouter), nf),
                                    dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
             else
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, false>), dim3((unsigned)(nxb * nouter), nf),
+                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, MC>), dim3((unsigned)(nxb * nouter), nf),
                                    dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
         }
     }

@@ -417,7 +417,22 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
                     rowt[((size_t)f * RAG_MAX_CHUNK + t) * P + k] = row[(size_t)f * n + cstart(k) + t];
     }
 
-    // host image: coef64 | coef32 | row64 | row32 | pcr | rowt64 | rowt32 (256-byte aligned parts)
+    // per-chunk blocks padded to the kernels' capacity (LineDev::rowu64); the
+    // ragged plans do not use them
+    const int longest = m + (extra ? 1 : 0);
+    const int cap = longest <= 8 ? 8 : longest <= 16 ? 16 : 32;
+    std::vector<double> rowu;
+    if (!chunk_major) {
+        rowu.assign((size_t)P * nrow * cap, 0.0);
+        for (int k = 0; k < P; k++)
+            for (int f = 0; f < nrow; f++)
+                for (int t = 0; t < clen(k); t++) {
+                    if (q == 1 && f == R1_C && t == clen(k) - 1) continue;
+                    rowu[((size_t)k * nrow + f) * cap + t] = row[(size_t)f * n + cstart(k) + t];
+                }
+    }
+
+    // host image: coef64 | coef32 | row64 | row32 | pcr | rowu64 | rowu32 | rowt64 | rowt32 (256-byte aligned parts)
     size_t b_coef64 = COEF_N * sizeof(double), b_coef32 = COEF_N * sizeof(float);
     size_t b_row64 = row.size() * sizeof(double), b_row32 = row.size() * sizeof(float);
     size_t b_pcr = pcr.size() * sizeof(double);
@@ -427,10 +442,18 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     out.o_row64 = out.o_coef32 + al(b_coef32);
     out.o_row32 = out.o_row64 + al(b_row64);
     out.o_pcr = out.o_row32 + al(b_row32);
-    out.o_rowt64 = out.o_pcr + al(std::max<size_t>(b_pcr, 8));
+    const size_t b_rowu64 = rowu.size() * sizeof(double), b_rowu32 = rowu.size() * sizeof(float);
+    out.o_rowu64 = out.o_pcr + al(std::max<size_t>(b_pcr, 8));
+    out.o_rowu32 = out.o_rowu64 + al(b_rowu64);
+    out.o_rowt64 = out.o_rowu32 + al(b_rowu32);
     out.o_rowt32 = out.o_rowt64 + al(b_rowt64);
     const size_t total = out.o_rowt32 + al(b_rowt32);
     out.image.assign(total, 0);
+    if (!rowu.empty()) {
+        std::vector<float> rowu32(rowu.begin(), rowu.end());
+        std::memcpy(out.image.data() + out.o_rowu64, rowu.data(), b_rowu64);
+        std::memcpy(out.image.data() + out.o_rowu32, rowu32.data(), b_rowu32);
+    }
     if (!rowt.empty()) {
         std::vector<float> rowt32(rowt.begin(), rowt.end());
         std::memcpy(out.image.data() + out.o_rowt64, rowt.data(), b_rowt64);
@@ -447,6 +470,7 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     L0.n = n; L0.q = q; L0.M = M; L0.sym = s.symmetric ? 1 : 0; L0.nc = closed ? nc : 0;
     L0.periodic = periodic ? 1 : 0; L0.closed = closed ? 1 : 0;
     L0.P = P; L0.nsteps = nsteps; L0.m = m; L0.extra = extra;
+    L0.cap = cap;
 }
 
 void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base)
@@ -457,6 +481,8 @@ void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base)
     dev.row64 = (const double *)(base + t.o_row64);
     dev.row32 = (const float *)(base + t.o_row32);
     dev.pcr = (const double *)(base + t.o_pcr);
+    dev.rowu64 = (const double *)(base + t.o_rowu64);
+    dev.rowu32 = (const float *)(base + t.o_rowu32);
     dev.rowt64 = t.o_rowt64 != t.o_rowt32 ? (const double *)(base + t.o_rowt64) : nullptr;
     dev.rowt32 = t.o_rowt64 != t.o_rowt32 ? (const float *)(base + t.o_rowt32) : nullptr;
 }

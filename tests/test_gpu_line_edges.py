@@ -26,3 +26,22 @@ def test_truncated_reduction(ctx, name, periodic, dim, n):  # noqa: F811
     for a in (f, g):
         ref = _oracle_apply(name, dim, n, periodic, 0.01, a)
         assert Hh.relerr(_gpu_apply(ctx, name, dim, n, periodic, 0.01, a), ref) <= 1e-12
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("lanes,line,outer", [(48, 16, 3), (64, 9, 2), (65, 33, 2), (127, 64, 2), (130, 20, 1),
+                                              (50, 33, 512), (128, 64, 513), (130, 11, 300)])
+def test_wave_uniform_yz(ctx, dtype, bar, periodic, lanes, line, outer):  # noqa: F811
+    """The one-chunk-per-wave y / z sweeps: whole and short chunks of every
+    capacity, partial lane blocks, and (FP32, even rows, >= 512 blocks) two
+    lines per lane; C6, C10 and the filter."""
+    for name in ("lele_d1_6", "lele_d1_10", "compact_filter"):
+        for dim in (2, 3):
+            n = (lanes, line, outer) if dim == 2 else (lanes, outer, line)
+            f = Hh.random_field(n, seed=31)
+            if dtype == np.float32:
+                f = f.astype(np.float32).astype(np.float64)
+            ref = _oracle_apply(name, dim, n, periodic, 0.1, f)
+            got = _gpu_apply(ctx, name, dim, n, periodic, 0.1, f, dtype=dtype)
+            assert Hh.relerr(got, ref) <= bar, (name, dim)
