@@ -74,6 +74,8 @@ struct LineDev {
     int cap;               // chunk capacity of the kernels: 8, 16 or 32 >= the longest chunk
     const double *rowu64;  // per-chunk blocks [(k * nrow + field) * cap + t] of the row constants; rows
     const float *rowu32;   //   past a chunk's length are zero, and so is its last row's coupling C
+    const double *rowv64;  // the same constants, chunks adjacent: [(field * cap + t) * P + k]
+    const float *rowv32;
     const double *rowt64;  // chunk-major copy of the per-row constants (ragged plans):
     const float *rowt32;   //   [(field * RAG_MAX_CHUNK + t) * P + k] = row of point t of chunk k
 };
@@ -97,7 +99,8 @@ struct HostPlan {
 struct LineTables {
     LineDev dev{};
     std::vector<unsigned char> image;
-    size_t o_coef32 = 0, o_row64 = 0, o_row32 = 0, o_pcr = 0, o_rowu64 = 0, o_rowu32 = 0, o_rowt64 = 0, o_rowt32 = 0;
+    size_t o_coef32 = 0, o_row64 = 0, o_row32 = 0, o_pcr = 0, o_rowu64 = 0, o_rowu32 = 0, o_rowv64 = 0, o_rowv32 = 0,
+           o_rowt64 = 0, o_rowt32 = 0;
 };
 // chunk_major: also store the chunk-major row tables of the ragged kernel
 // (RAG_MAX_CHUNK rows per chunk; max_chunk must not exceed it).

@@ -1332,13 +1332,18 @@ constexpr int XCL = 16;
 // PF: each step's coefficient blocks are loaded one step ahead (per-lane
 // chunk indices kc, whose blocks are vector loads), so their latency overlaps
 // the previous step's shuffles and products.
-template <int Q, bool PF = false>
+// UNI: kc is wave-uniform (scalar loads).
+template <int Q, bool PF = false, bool UNI = false>
 __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int kc, int base, double (&r)[2 * Q],
                                                    double (&tp)[Q], double (&hn)[Q])
 {
     constexpr int B = 2 * Q;
     const int P = p.P;
     const double *pc = p.pcr;
+    auto ld = [](const double *q) {
+        if constexpr (UNI) return cload(q);
+        else return gload(q);
+    };
     if constexpr (PF) {
         constexpr int C = 2 * B * B;
         // one PCR step: multiplies by the blocks in cur and loads the next
@@ -1418,8 +1423,8 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
                 double acc = r[i];
 #pragma unroll
                 for (int j = 0; j < B; j++) {
-                    acc = fma(gload(al + i * B + j), rm[j], acc);
-                    acc = fma(gload(be + i * B + j), rp[j], acc);
+                    acc = fma(ld(al + i * B + j), rm[j], acc);
+                    acc = fma(ld(be + i * B + j), rp[j], acc);
                 }
                 r[i] = acc;
             }
@@ -1431,7 +1436,7 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
     for (int i = 0; i < B; i++) {
         double acc = 0.0;
 #pragma unroll
-        for (int j = 0; j < B; j++) acc = fma(gload(mi + i * B + j), r[j], acc);
+        for (int j = 0; j < B; j++) acc = fma(ld(mi + i * B + j), r[j], acc);
         z[i] = acc;
     }
     int kprev = k - 1, knext = k + 1;
@@ -1454,128 +1459,321 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
     }
 }
 
-// One wave per block.  The wave's 64/P lines are staged in LDS (a pad slot
-// after every XC points keeps the chunk-strided reads conflict-free), so
-// global loads and stores are contiguous 512-byte rows.  XC is the chunk
-// capacity (8 or 16): the sweeps run XC steps, so chunks of at most 8 points
-// take the 8-step kernel.
 template <int XC = XCL>
 __device__ __forceinline__ int xw_slot(int x) { return x + x / XC; }
 
-template <typename T, int Q, int M, int SYM, int EPI, bool UNIROW, int XC>
+template <typename T> __device__ __forceinline__ const T *rowvp(const LineDev &p);
+template <> __device__ __forceinline__ const double *rowvp<double>(const LineDev &p) { return p.rowv64; }
+template <> __device__ __forceinline__ const float *rowvp<float>(const LineDev &p) { return p.rowv32; }
+
+// The zero-padded plan rows of one chunk: a block of its own read through
+// scalar loads (every chunk of the wave has the same rows) ...
+template <typename T, int CAP> struct RowsBlock {
+    const T *base;
+    __device__ __forceinline__ T operator()(int f, int t) const { return cload(base + f * CAP + t); }
+    template <typename D> __device__ __forceinline__ void fence(const D &) {}
+};
+// ... or per lane, with the rows of adjacent chunks in adjacent words
+template <typename T, int CAP> struct RowsLane {
+    const T *base;
+    int P;
+    __device__ __forceinline__ T operator()(int f, int t) const { return gload(base + (f * CAP + t) * P); }
+    template <typename D> __device__ __forceinline__ void fence(const D &dep)
+    {
+        asm volatile("" : "+v"(base) : "v"(dep));
+    }
+};
+
+// Chunk sweeps over all CL rows (rows past the chunk's length hold zeros and
+// multiply by zeros), the rows read G at a time as in solve_grouped.
+template <typename T, int Q, int CL, int G, typename Rows>
+__device__ __forceinline__ void solve_padded(T (&d)[CL], Rows R)
+{
+    constexpr int NG = CL / G;
+    constexpr int NL = Q, NU = Q == 1 ? 2 : 3;
+    const int fl[2] = {Q == 1 ? (int)R1_L : (int)R2_L1, (int)R2_L2};
+    const int fu[3] = {Q == 1 ? (int)R1_DINV : (int)R2_U0INV, Q == 1 ? (int)R1_C : (int)R2_U1, (int)R2_U2};
+    T c[NL][G], nx[NL][G];
+#pragma unroll
+    for (int f = 0; f < NL; f++)
+#pragma unroll
+        for (int i = 0; i < G; i++) c[f][i] = R(fl[f], i);
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        if (g + 1 < NG) {
+            if (g > 0) R.fence(d[g * G - 1]);
+#pragma unroll
+            for (int f = 0; f < NL; f++)
+#pragma unroll
+                for (int i = 0; i < G; i++) nx[f][i] = R(fl[f], (g + 1) * G + i);
+        }
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            const int t = g * G + i;
+            if constexpr (Q == 1) {
+                if (t >= 1) d[t] = fma(-c[0][i], d[t - 1], d[t]);
+            } else {
+                if (t + 1 < CL) d[t + 1] = fma(-c[0][i], d[t], d[t + 1]);
+                if (t + 2 < CL) d[t + 2] = fma(-c[1][i], d[t], d[t + 2]);
+            }
+        }
+        if (g + 1 < NG) {
+#pragma unroll
+            for (int f = 0; f < NL; f++)
+#pragma unroll
+                for (int i = 0; i < G; i++) c[f][i] = nx[f][i];
+        }
+    }
+    T u[NU][G], nu[NU][G];
+    R.fence(d[CL - 1]);
+#pragma unroll
+    for (int f = 0; f < NU; f++)
+#pragma unroll
+        for (int i = 0; i < G; i++) u[f][i] = R(fu[f], (NG - 1) * G + i);
+#pragma unroll
+    for (int g = NG - 1; g >= 0; g--) {
+        if (g > 0) {
+            if (g < NG - 1) R.fence(d[(g + 1) * G]);
+#pragma unroll
+            for (int f = 0; f < NU; f++)
+#pragma unroll
+                for (int i = 0; i < G; i++) nu[f][i] = R(fu[f], (g - 1) * G + i);
+        }
+#pragma unroll
+        for (int i = G - 1; i >= 0; i--) {
+            const int t = g * G + i;
+            T acc = d[t];
+            if (t + 1 < CL) acc = fma(-u[1][i], d[t + 1 < CL ? t + 1 : t], acc);
+            if constexpr (Q == 2)
+                if (t + 2 < CL) acc = fma(-u[2][i], d[t + 2 < CL ? t + 2 : t], acc);
+            d[t] = acc * u[0][i];
+        }
+        if (g > 0) {
+#pragma unroll
+            for (int f = 0; f < NU; f++)
+#pragma unroll
+                for (int i = 0; i < G; i++) u[f][i] = nu[f][i];
+        }
+    }
+}
+
+// One wave per block, 64/P lines staged in LDS (a pad slot after every XC
+// points keeps the chunk-strided reads conflict-free), so global loads and
+// stores are contiguous.  XC is the chunk capacity (8 or 16).
+//
+// Bound: instruction issue before HBM, so every row costs as few instructions
+// as it can.  A line's points are dealt to LPL = 8..64 lanes (the power of two
+// that holds the line, at most a wave), 64 / LPL lines at a time, so no element
+// index is divided by the line length; WIDE (LPL = 64): one line at a time,
+// its offset in scalar registers.  The tile row holds the M halo points at both
+// ends (wrapped copies, or zeros at closed ends), so window reads need no wrap
+// test.  The row constants are zero-padded to XC rows (LineDev::rowu64, rowv64),
+// so the sweeps run without length tests.  UNIROW: periodic line of equal
+// chunks, whose factors, spikes and PCR blocks are those of chunk 0 (scalar
+// loads).  FULL: those chunks hold XC points, which fixes every LDS offset at
+// compile time.
+//
+// The FP32 C6 kernel of equal 12-point chunks went from 7416 to 2224
+// instructions.  Measured before / after, one pass (three sweeps): C6 gradient
+// of 384^3 FP32 578 / 390 us, C10 gradient of 250 x 199 x 180 FP32 between
+// walls 224 / 126 us; 40 Taylor-Green steps at 64^3 FP64 28.7 / 25.6 ms, at
+// 120 x 97 x 81 FP32 73.4 / 62.4 ms.
+template <typename T, int Q, int M, int SYM, int EPI, bool UNIROW, int XC, bool FULL, bool WIDE>
 __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz, int ny,
-                                                int64_t nlines, int TS, EpiArgs e, LineFields mf)
+                                                int64_t nlines, int TS, int lsh, EpiArgs e, LineFields mf)
 {
     select_field<T, EPI>(mf, f, e);
     extern __shared__ double smem[];
     T *tile = (T *)smem;
-    const int P = p.P;
-    const int n = p.n;
+    const int P = p.P, n = p.n;
     const int lane = threadIdx.x;
-    const int nl = 64 / P;           // lines staged by the wave
+    const int nl = 64 / P;                       // lines of the wave
+    // element i of this lane: point x = xl + q lpl of line lj < nl, walked
+    // segment by segment (at most XC elements)
+    const int lpl = WIDE ? 64 : 1 << lsh, grp = 64 / lpl;
+    const int seg = (n + lpl - 1) / lpl;
+    const int lsub = WIDE ? 0 : lane >> lsh, xl = lane & (lpl - 1);
+    // lane l holds the offset of line l (the first one's for lines that do not
+    // exist); WIDE reads it into scalar registers
     const int64_t l0 = (int64_t)blockIdx.x * nl;
-    // stage the lines: lane-element i of the block's nl*n points is line lj,
-    // point x (shifts when n is a power of two >= 64, else a division); every
-    // load is issued before the LDS writes.
-    const int cnt = (nl * n + 63) / 64;
-    const bool pow2 = n >= 64 && (n & (n - 1)) == 0;
-    const int sh = pow2 ? __builtin_ctz((unsigned)(n >> 6)) : 0;
-    const int j0 = (int)(l0 % ny), k0 = (int)(l0 / ny);
-    auto line_of = [&](int i, int &lj, int &x) {
-        if (pow2) {
-            lj = i >> sh;
-            x = lane + 64 * (i & ((1 << sh) - 1));
-        } else {
-            const int q = lane + 64 * i;
-            lj = q / n;
-            x = q - lj * n;
-        }
-    };
+    const int left = (int)(nlines - l0 < nl ? nlines - l0 : nl);   // lines that exist, >= 1
+    int olo, ohi;
+    {
+        // a launch holds fewer than 2^32 threads, hence fewer lines
+        const uint32_t l = (uint32_t)l0 + (uint32_t)(lane < left ? lane : 0);
+        const uint32_t kk = l / (uint32_t)ny;
+        const int64_t off = (int64_t)(l - kk * (uint32_t)ny) * sy + (int64_t)kk * sz;
+        olo = (int)(uint32_t)off;
+        ohi = (int)(off >> 32);
+    }
     auto line_off = [&](int lj) -> int64_t {
-        int j = j0 + lj, k = k0;
-        while (j >= ny) {
-            j -= ny;
-            k++;
+        uint32_t a;
+        int b;
+        if constexpr (WIDE) {
+            a = (uint32_t)__builtin_amdgcn_readlane(olo, lj);
+            b = __builtin_amdgcn_readlane(ohi, lj);
+        } else {
+            a = (uint32_t)__shfl(olo, lj, 64);
+            b = __shfl(ohi, lj, 64);
         }
-        return (int64_t)j * sy + (int64_t)k * sz;
+        return (int64_t)(((uint64_t)(uint32_t)b << 32) | a);
+    };
+    struct Walk {
+        int q, lj;
+    };
+    auto next = [&](Walk &w) {
+        const bool turn = w.q + 1 == seg;
+        w.q = turn ? 0 : w.q + 1;
+        w.lj += turn ? grp : 0;
     };
     {
         T tmp[XC];
+        Walk w{0, lsub};
 #pragma unroll
         for (int i = 0; i < XC; i++) {
-            tmp[i] = T(0);
-            int lj, x;
-            line_of(i, lj, x);
-            if (i < cnt && lj < nl && l0 + lj < nlines) tmp[i] = f[line_off(lj) + x];
+            const int x = xl + w.q * lpl;
+            tmp[i] = f[line_off(w.lj) + (x < n ? x : n - 1)];
+            next(w);
         }
+        // the M halo points at both ends of each line: wrapped copies, or zeros
+        for (int h0 = 0; h0 < nl * 2 * M; h0 += 64) {
+            const int h = h0 + lane;
+            const int lj = h / (2 * M), hx = h % (2 * M);
+            T v = T(0);
+            if (p.periodic) {
+                const uint32_t a = (uint32_t)__shfl(olo, lj & 63, 64);
+                const uint32_t b = (uint32_t)__shfl(ohi, lj & 63, 64);
+                v = f[(int64_t)(((uint64_t)b << 32) | a) + (hx < M ? n - M + hx : hx - M)];
+            }
+            if (lj < nl) tile[lj * TS + xw_slot<XC>(hx < M ? hx : hx + n)] = v;
+        }
+        w = Walk{0, lsub};
 #pragma unroll
         for (int i = 0; i < XC; i++) {
-            int lj, x;
-            line_of(i, lj, x);
-            if (i < cnt && lj < nl) tile[lj * TS + xw_slot<XC>(x)] = tmp[i];
+            const int x = xl + w.q * lpl;
+            if (w.lj < nl && x < n) tile[w.lj * TS + xw_slot<XC>(x + M)] = tmp[i];
+            next(w);
         }
     }
     __syncthreads();
     const int k = lane & (P - 1);
-    const int base = (lane / P) * P;
-    const int s = k * p.m + min(k, p.extra);
-    const int len = p.m + (k < p.extra ? 1 : 0);
-    const int rs = UNIROW ? 0 : s;
-    const int kc = UNIROW ? 0 : k;
-    T res[XC];
+    const int li = lane / P;
+    const int s = FULL ? k * XC : k * p.m + min(k, p.extra);
+    const int len = FULL ? XC : p.m + (k < p.extra ? 1 : 0);
+    T *trow = tile + li * TS;
+    // slot of window point t (halo included), t = 0 .. XC + 2 M - 1
+    auto slot = [&](int t) { return FULL ? k * (XC + 1) + t + t / XC : xw_slot<XC>(s + t); };
+    T d[XC];
     {
-        const T *trow = tile + (lane / P) * TS;
         T fv[XC + 2 * M];
 #pragma unroll
-        for (int t = -M; t < XC + M; t++) {
-            T val = T(0);
-            if (t < len + M) {
-                int r = s + t;
-                bool ok = true;
-                if (r < 0) {
-                    if (p.periodic) r += n; else ok = false;
-                } else if (r >= n) {
-                    if (p.periodic) r -= n; else ok = false;
-                }
-                if (ok) val = trow[xw_slot<XC>(r)];
-            }
-            fv[t + M] = val;
+        for (int t = 0; t < XC + 2 * M; t++) fv[t] = trow[slot(t)];
+        const T *cf = coefp<T>(p);
+        T ci[M];
+#pragma unroll
+        for (int m = 0; m < M; m++) ci[m] = cload(cf + COEF_CI + m);
+        const T a0 = cload(cf + COEF_A0);
+        // rows past the chunk's length start and stay zero; a chunk holds more
+        // than half the capacity 16
+#pragma unroll
+        for (int t = 0; t < XC; t++) {
+            d[t] = rhs_row<T, M, SYM>(fv, t + M, ci, a0);
+            if (!FULL && t >= (XC > 8 ? XC / 2 : 1)) d[t] = t < len ? d[t] : T(0);
         }
-        T fe[8];
+        if (!UNIROW && p.closed) {
 #pragma unroll
-        for (int kap = 0; kap < 8; kap++) fe[kap] = (p.closed && kap < n) ? trow[xw_slot<XC>(n - 1 - kap)] : T(0);
-        Chunk<T, Q, M, SYM, XC> ch;
-        ch.rhs(p, k, len, fv, fe);
-        solve_grouped<T, Q, XC, 8>(ch.d, len, RowsClamped<T>{rowp<T>(p), n, rs});
-        double r[2 * Q], tp[Q], hn[Q];
-        ch.ends(len, r);
-        reduced_solve_wave<Q, !UNIROW && Q == 1 && sizeof(T) == 8>(p, k, kc, base, r, tp, hn);
-        correct_grouped<T, Q, XC, 8>(ch.d, len, RowsClamped<double>{p.row64, n, rs}, tp, hn);
+            for (int t = 0; t < NCMAX; t++) {
+                if (t >= p.nc) continue;
+                const T *cr = cf + COEF_CLO + t * 8;
+                T acc = cload(cr) * fv[M];
 #pragma unroll
-        for (int t = 0; t < XC; t++) res[t] = ch.d[t];
+                for (int kap = 1; kap < 8; kap++) {
+                    // points past a line shorter than the stencil take a zero weight
+                    const T fk = kap < n ? fv[kap + M] : T(0);
+                    acc = fma(cload(cr + kap), fk, acc);
+                }
+                d[t] = k == 0 ? acc : d[t];
+            }
+            T fe[8];
+#pragma unroll
+            for (int kap = 0; kap < 8; kap++) fe[kap] = kap < n ? trow[xw_slot<XC>(n - 1 - kap + M)] : T(0);
+            // the last chunk holds m points (the longer ones come first)
+#pragma unroll
+            for (int t = 0; t < XC; t++) {
+                const int jr = p.m - 1 - t;
+                if (jr < 0 || jr >= p.nc) continue;
+                const T *cr = cf + COEF_CHI + jr * 8;
+                T acc = cload(cr) * fe[0];
+#pragma unroll
+                for (int kap = 1; kap < 8; kap++) acc = fma(cload(cr + kap), fe[kap], acc);
+                d[t] = k == P - 1 ? acc : d[t];
+            }
+        }
     }
-    __syncthreads();   // all window reads done before the tile is overwritten
-    {
-        T *wrow = tile + (lane / P) * TS;
+    // rows per group of per-lane loads: four where two groups of eight spill
+    constexpr int G = !UNIROW && XC > 8 && (Q == 2 || sizeof(T) == 8) ? 4 : 8;
+    if constexpr (UNIROW) solve_padded<T, Q, XC, G>(d, RowsBlock<T, XC>{rowup<T>(p)});
+    else solve_padded<T, Q, XC, G>(d, RowsLane<T, XC>{rowvp<T>(p) + k, P});
+    double r[2 * Q], tp[Q], hn[Q];
 #pragma unroll
-        for (int t = 0; t < XC; t++)
-            if (t < len) wrow[xw_slot<XC>(s + t)] = res[t];
+    for (int i = 0; i < Q; i++) {
+        r[i] = (double)d[i];
+        T x = d[FULL ? XC - Q + i : 0];
+        if constexpr (!FULL) {
+#pragma unroll
+            for (int t = 1; t < XC; t++) x = t == len - Q + i ? d[t] : x;
+        }
+        r[Q + i] = (double)x;
     }
+    reduced_solve_wave<Q, !UNIROW && Q == 1 && sizeof(T) == 8, UNIROW>(p, k, UNIROW ? 0 : k, li * P, r, tp, hn);
+    // spike correction; each result goes back to the tile (every window read
+    // of the wave is done: the wave runs in step)
     __syncthreads();
+    auto correct = [&](auto R) {
+#pragma unroll
+        for (int g = 0; g < XC / G; g++) {
+            if (g > 0) R.fence(d[g * G - 1]);
+            double c[2 * Q][G];
+#pragma unroll
+            for (int i = 0; i < G; i++) {
+                c[0][i] = R(Q == 1 ? (int)R1_V : (int)R2_V0, g * G + i);
+                c[1][i] = R(Q == 1 ? (int)R1_W : (int)R2_W0, g * G + i);
+                if constexpr (Q == 2) {
+                    c[2][i] = R(R2_V1, g * G + i);
+                    c[3][i] = R(R2_W1, g * G + i);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < G; i++) {
+                const int t = g * G + i;
+                double acc = fma(c[1][i], hn[0], c[0][i] * tp[0]);
+                if constexpr (Q == 2) {
+                    acc = fma(c[2][i], tp[1], acc);
+                    acc = fma(c[3][i], hn[1], acc);
+                }
+                d[t] = (T)((double)d[t] - acc);
+                if (FULL || t < (XC > 8 ? XC / 2 : 1) || t < len) trow[slot(t + M)] = d[t];
+            }
+        }
+    };
+    if constexpr (UNIROW) correct(RowsBlock<double, XC>{p.rowu64});
+    else correct(RowsLane<double, XC>{p.rowv64 + k, P});
+    __syncthreads();
+    Walk w{0, lsub};
 #pragma unroll
     for (int b = 0; b < XC; b += 8) {
         int64_t o[8];
-        T v[8];
+        T v[1][8];
         bool ok[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            int lj, x;
-            line_of(b + i, lj, x);
-            ok[i] = (b + i) < cnt && lj < nl && l0 + lj < nlines;
-            o[i] = ok[i] ? line_off(lj) + x : 0;
-            v[i] = ok[i] ? tile[lj * TS + xw_slot<XC>(x)] : T(0);
+            const int x = xl + w.q * lpl, xc = x < n ? x : n - 1;
+            ok[i] = w.lj < left && x < n;
+            o[i] = line_off(w.lj) + xc;
+            v[0][i] = tile[(w.lj < nl ? w.lj : 0) * TS + xw_slot<XC>(xc + M)];
+            next(w);
         }
-        epilogue_batch<T, EPI, 8>(e, o, v, ok);
+        epilogue_rows<T, EPI, 8, 1, false>(e, o, v, ok);
     }
 }
 
@@ -1727,19 +1925,25 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         const int nl = 64 / P;
         const int64_t nblk = (nlines + nl - 1) / nl;
         const bool uni = p.periodic && p.extra == 0;
+        int lsh = 3;   // lanes per line: the power of two that holds it, 8 .. 64
+        while ((1 << lsh) < p.n && lsh < 6) lsh++;
         auto go = [&](auto kern, int xc) {
-            const int TS = p.n + p.n / xc + 1;
+            const int y = p.n + 2 * M + xc;
+            const int TS = y + y / xc + 1;
             const size_t shm = (size_t)nl * TS * sizeof(T);
             hipLaunchKernelGGL(kern, dim3((unsigned)nblk, nf), dim3(64), shm, st, p, f, v.s[1], v.s[2], (int)v.n[1],
-                               nlines, TS, e, mf);
+                               nlines, TS, lsh, e, mf);
         };
-        if (p.m + (p.extra ? 1 : 0) <= 8) {
-            if (uni) go(k_line_xw<T, Q, M, SYM, EPI, true, 8>, 8);
-            else go(k_line_xw<T, Q, M, SYM, EPI, false, 8>, 8);
-        } else {
-            if (uni) go(k_line_xw<T, Q, M, SYM, EPI, true, XCL>, XCL);
-            else go(k_line_xw<T, Q, M, SYM, EPI, false, XCL>, XCL);
-        }
+        auto pick = [&](auto xcv) {
+            constexpr int XC = xcv.value;
+            if (uni && lsh == 6 && p.m == XC) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, true, true>, XC);
+            else if (uni && lsh == 6) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, false, true>, XC);
+            else if (uni) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, false, false>, XC);
+            else if (lsh == 6) go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, true>, XC);
+            else go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, false>, XC);
+        };
+        if (p.cap == 8) pick(std::integral_constant<int, 8>{});
+        else pick(std::integral_constant<int, XCL>{});
     } else if (dim == 1) {
         const size_t tile_row = (size_t)(p.n + 1) * sizeof(T);
         const int64_t nlines = v.n[1] * v.n[2];

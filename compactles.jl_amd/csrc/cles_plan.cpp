@@ -421,18 +421,22 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     // ragged plans do not use them
     const int longest = m + (extra ? 1 : 0);
     const int cap = longest <= 8 ? 8 : longest <= 16 ? 16 : 32;
-    std::vector<double> rowu;
+    std::vector<double> rowu, rowv;
     if (!chunk_major) {
         rowu.assign((size_t)P * nrow * cap, 0.0);
+        rowv.assign((size_t)P * nrow * cap, 0.0);
         for (int k = 0; k < P; k++)
             for (int f = 0; f < nrow; f++)
                 for (int t = 0; t < clen(k); t++) {
                     if (q == 1 && f == R1_C && t == clen(k) - 1) continue;
-                    rowu[((size_t)k * nrow + f) * cap + t] = row[(size_t)f * n + cstart(k) + t];
+                    const double c = row[(size_t)f * n + cstart(k) + t];
+                    rowu[((size_t)k * nrow + f) * cap + t] = c;
+                    rowv[((size_t)f * cap + t) * P + k] = c;
                 }
     }
 
-    // host image: coef64 | coef32 | row64 | row32 | pcr | rowu64 | rowu32 | rowt64 | rowt32 (256-byte aligned parts)
+    // host image: coef64 | coef32 | row64 | row32 | pcr | rowu64 | rowu32 | rowv64 | rowv32 | rowt64 | rowt32
+    // (256-byte aligned parts)
     size_t b_coef64 = COEF_N * sizeof(double), b_coef32 = COEF_N * sizeof(float);
     size_t b_row64 = row.size() * sizeof(double), b_row32 = row.size() * sizeof(float);
     size_t b_pcr = pcr.size() * sizeof(double);
@@ -445,7 +449,9 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     const size_t b_rowu64 = rowu.size() * sizeof(double), b_rowu32 = rowu.size() * sizeof(float);
     out.o_rowu64 = out.o_pcr + al(std::max<size_t>(b_pcr, 8));
     out.o_rowu32 = out.o_rowu64 + al(b_rowu64);
-    out.o_rowt64 = out.o_rowu32 + al(b_rowu32);
+    out.o_rowv64 = out.o_rowu32 + al(b_rowu32);
+    out.o_rowv32 = out.o_rowv64 + al(b_rowu64);
+    out.o_rowt64 = out.o_rowv32 + al(b_rowu32);
     out.o_rowt32 = out.o_rowt64 + al(b_rowt64);
     const size_t total = out.o_rowt32 + al(b_rowt32);
     out.image.assign(total, 0);
@@ -453,6 +459,9 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
         std::vector<float> rowu32(rowu.begin(), rowu.end());
         std::memcpy(out.image.data() + out.o_rowu64, rowu.data(), b_rowu64);
         std::memcpy(out.image.data() + out.o_rowu32, rowu32.data(), b_rowu32);
+        std::vector<float> rowv32(rowv.begin(), rowv.end());
+        std::memcpy(out.image.data() + out.o_rowv64, rowv.data(), b_rowu64);
+        std::memcpy(out.image.data() + out.o_rowv32, rowv32.data(), b_rowu32);
     }
     if (!rowt.empty()) {
         std::vector<float> rowt32(rowt.begin(), rowt.end());
@@ -483,6 +492,8 @@ void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base)
     dev.pcr = (const double *)(base + t.o_pcr);
     dev.rowu64 = (const double *)(base + t.o_rowu64);
     dev.rowu32 = (const float *)(base + t.o_rowu32);
+    dev.rowv64 = (const double *)(base + t.o_rowv64);
+    dev.rowv32 = (const float *)(base + t.o_rowv32);
     dev.rowt64 = t.o_rowt64 != t.o_rowt32 ? (const double *)(base + t.o_rowt64) : nullptr;
     dev.rowt32 = t.o_rowt64 != t.o_rowt32 ? (const float *)(base + t.o_rowt32) : nullptr;
 }

@@ -45,3 +45,22 @@ def test_wave_uniform_yz(ctx, dtype, bar, periodic, lanes, line, outer):  # noqa
             ref = _oracle_apply(name, dim, n, periodic, 0.1, f)
             got = _gpu_apply(ctx, name, dim, n, periodic, 0.1, f, dtype=dtype)
             assert Hh.relerr(got, ref) <= bar, (name, dim)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("line", [9, 16, 17, 24, 32, 33, 40, 63, 64, 65, 100, 128, 129, 250, 256, 257, 384, 512, 1000,
+                                  1024])
+def test_wave_local_x(ctx, dtype, bar, periodic, line):  # noqa: F811
+    """The wave-local x sweep: 8 to 64 lanes per line, whole and short chunks of
+    both capacities, line counts that leave waves partly empty, padded and
+    unpadded rows; every scheme."""
+    for name in ("lele_d1_6", "pade_d1_4", "lele_d1_10", "compact_filter"):
+        for ny, nz, padded in ((5, 3, True), (1, 1, False), (3, 7, False), (67, 2, True)):
+            n = (line, ny, nz)
+            f = Hh.random_field(n, seed=41)
+            if dtype == np.float32:
+                f = f.astype(np.float32).astype(np.float64)
+            ref = _oracle_apply(name, 1, n, periodic, 0.1, f)
+            got = _gpu_apply(ctx, name, 1, n, periodic, 0.1, f, dtype=dtype, padded=padded)
+            assert Hh.relerr(got, ref) <= bar, (name, n)
