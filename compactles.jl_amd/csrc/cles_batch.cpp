@@ -72,6 +72,9 @@ struct cles_batch {
     int64_t *step = nullptr, *nmax = nullptr, *step0 = nullptr;
     int *status = nullptr, *active = nullptr, *stepped = nullptr, *filt = nullptr, *cnt = nullptr;
     int *host_cnt = nullptr;
+    // one instance's state on its way to or from the host
+    std::mutex io_mu;
+    cles::PinnedBuf io_buf;
 
     // CLES_RUN_STEP_GRAPH: GRAPH_ITERS run! iterations captured once and
     // replayed; the captured kernels record dts into gdts (nrec = g_nrec)
@@ -709,36 +712,48 @@ int cles_batch_shape(cles_batch *b, int64_t *count, int64_t *total_points, int *
     })
 }
 
+// One instance's components between the device and the padded host layout,
+// through pinned memory that one kernel reads or writes over the link (a copy
+// per component costs a launch and a pageable staging pass each).
+static void move_instance(cles_batch *b, int64_t i, double *Qh, const int64_t padded[3], const int halo[3], bool down)
+{
+    CLES_REQUIRE(b && Qh && padded && halo, "NULL argument");
+    cles::check_inst(b, i);
+    CLES_REQUIRE(halo[0] >= 0 && padded[0] >= b->n[i] + 2 * (int64_t)halo[0], "padded extents smaller than n + 2*halo");
+    CLES_REQUIRE(padded[1] == 1 && padded[2] == 1 && halo[1] == 0 && halo[2] == 0,
+                 "a batch instance is laid out as (n + 2*halo, 1, 1) with halo (H, 0, 0)");
+    const int64_t NP = padded[0];
+    const size_t n = (size_t)b->n[i];
+    double *dev = b->Q + b->off[i], *host = Qh + halo[0];
+    std::lock_guard<std::mutex> lk(b->io_mu);
+    CLES_HIP(hipSetDevice(b->ctx->device));
+    const int nmax = *std::max_element(b->n.begin(), b->n.end());
+    double *buf = (double *)b->io_buf.get(sizeof(double) * (size_t)nmax * b->C);
+    if (!b->io_buf.pinned) {
+        for (int c = 0; c < b->C; c++) {
+            double *h = host + c * NP, *d = dev + (size_t)c * b->N;
+            if (down) CLES_HIP(hipMemcpyAsync(h, d, sizeof(double) * n, hipMemcpyDeviceToHost, b->st()));
+            else CLES_HIP(hipMemcpyAsync(d, h, sizeof(double) * n, hipMemcpyHostToDevice, b->st()));
+        }
+        CLES_HIP(hipStreamSynchronize(b->st()));
+        return;
+    }
+    if (!down)
+        for (int c = 0; c < b->C; c++) std::memcpy(buf + (size_t)c * n, host + c * NP, sizeof(double) * n);
+    cles::launch_batch_io(dev, b->N, buf, (int64_t)n, b->C, down, b->st());
+    CLES_HIP(hipStreamSynchronize(b->st()));
+    if (down)
+        for (int c = 0; c < b->C; c++) std::memcpy(host + c * NP, buf + (size_t)c * n, sizeof(double) * n);
+}
+
 int cles_batch_upload(cles_batch *b, int64_t i, const double *Qh, const int64_t padded[3], const int halo[3])
 {
-    CLES_TRY({
-        CLES_REQUIRE(b && Qh && padded && halo, "NULL argument");
-        cles::check_inst(b, i);
-        CLES_REQUIRE(halo[0] >= 0 && padded[0] >= b->n[i] + 2 * (int64_t)halo[0], "padded extents smaller than n + 2*halo");
-        CLES_REQUIRE(padded[1] == 1 && padded[2] == 1 && halo[1] == 0 && halo[2] == 0,
-                     "a batch instance is laid out as (n + 2*halo, 1, 1) with halo (H, 0, 0)");
-        const int64_t NP = padded[0] * padded[1] * padded[2];
-        for (int c = 0; c < b->C; c++)
-            CLES_HIP(hipMemcpyAsync(b->Q + (size_t)c * b->N + b->off[i], Qh + c * NP + halo[0],
-                                    sizeof(double) * b->n[i], hipMemcpyHostToDevice, b->st()));
-        CLES_HIP(hipStreamSynchronize(b->st()));
-    })
+    CLES_TRY({ move_instance(b, i, const_cast<double *>(Qh), padded, halo, false); })
 }
 
 int cles_batch_download(cles_batch *b, int64_t i, double *Qh, const int64_t padded[3], const int halo[3])
 {
-    CLES_TRY({
-        CLES_REQUIRE(b && Qh && padded && halo, "NULL argument");
-        cles::check_inst(b, i);
-        CLES_REQUIRE(halo[0] >= 0 && padded[0] >= b->n[i] + 2 * (int64_t)halo[0], "padded extents smaller than n + 2*halo");
-        CLES_REQUIRE(padded[1] == 1 && padded[2] == 1 && halo[1] == 0 && halo[2] == 0,
-                     "a batch instance is laid out as (n + 2*halo, 1, 1) with halo (H, 0, 0)");
-        const int64_t NP = padded[0] * padded[1] * padded[2];
-        for (int c = 0; c < b->C; c++)
-            CLES_HIP(hipMemcpyAsync(Qh + c * NP + halo[0], b->Q + (size_t)c * b->N + b->off[i],
-                                    sizeof(double) * b->n[i], hipMemcpyDeviceToHost, b->st()));
-        CLES_HIP(hipStreamSynchronize(b->st()));
-    })
+    CLES_TRY({ move_instance(b, i, Qh, padded, halo, true); })
 }
 
 namespace {

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -126,6 +128,42 @@ void free_line_plan(HostPlan &hp);
 struct View3 {
     int64_t n[3];
     int64_t s[3];
+};
+
+// ---------------------------------------------------------------------------
+// Host transfers (cles_stage.cpp)
+// ---------------------------------------------------------------------------
+// A pinned host buffer that grows on demand (pageable where no pinned memory
+// is to be had: `pinned` tells).
+struct PinnedBuf {
+    void *ptr = nullptr;
+    size_t cap = 0;
+    bool pinned = false;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf &) = delete;
+    PinnedBuf &operator=(const PinnedBuf &) = delete;
+    ~PinnedBuf();
+    void *get(size_t bytes);
+    void release();
+};
+// Pinned staging of one owner (at most 6 x 2 buffers of 4 MB, or of a row that
+// is longer), freed with it; transfers of one stage run one at a time.
+struct HostStage {
+    ~HostStage();
+    // Moves ncomp components of contiguous device rows (component c, plane k,
+    // row j at dev + n0 (j + n1 (k + n2 c))) to or from host rows at host +
+    // c comp_stride + j s[1] + k s[2] (host_view: extents and strides), after
+    // the work queued on st; complete on return.
+    void transfer(bool down, int device, hipStream_t st, double *dev, const View3 &host_view, int64_t ncomp,
+                  int64_t comp_stride, double *host);
+
+private:
+    struct Lane {
+        PinnedBuf buf[2];
+        hipEvent_t ev[2] = {nullptr, nullptr};
+    };
+    std::mutex mu;
+    std::vector<std::unique_ptr<Lane>> lanes;
 };
 
 // ---------------------------------------------------------------------------

@@ -279,6 +279,9 @@ void launch_extrapolate(const PlaneArgs &a, double *Q, hipStream_t st);
 template <typename W>
 void launch_integral(const DiagArgs<W> &a, int kind, double *part, int nb, double scale, double *out,
                      hipStream_t st);
+// the C components (stride N) of n device points to or from pinned host memory
+// (contiguous components)
+void launch_batch_io(double *dev, int64_t N, double *host, int64_t n, int C, bool down, hipStream_t st);
 void launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
 template <typename Dst, typename Src> void launch_convert(Dst *d, const Src *s, int64_t N, hipStream_t st);
 

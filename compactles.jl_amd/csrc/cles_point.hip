@@ -1788,6 +1788,23 @@ void launch_integral(const DiagArgs<W> &a, int kind, double *part, int nb, doubl
     CHECK_LAUNCH();
 }
 
+// One thread per value; a component is contiguous on both sides, so the link
+// sees whole cache lines.
+__global__ void __launch_bounds__(TPB) k_batch_io(double *dev, int64_t N, double *host, int64_t n, bool down)
+{
+    const int64_t I = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    if (I >= n) return;
+    double *d = dev + (int64_t)blockIdx.y * N + I, *h = host + (int64_t)blockIdx.y * n + I;
+    if (down) *h = *d;
+    else *d = *h;
+}
+
+void launch_batch_io(double *dev, int64_t N, double *host, int64_t n, int C, bool down, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_batch_io, dim3(nblocks(n), (unsigned)C), dim3(TPB), 0, st, dev, N, host, n, down);
+    CHECK_LAUNCH();
+}
+
 void launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
 {
     const uintptr_t a = (uintptr_t)dst | (uintptr_t)src;

@@ -81,6 +81,7 @@ struct cles_solver {
     bool nsd_merged = false;
     void *flux[3][CLES_MAXSP + 4] = {};
     double *part = nullptr, *scal = nullptr;   // reduction partials, device scalars
+    cles::HostStage stage;                     // state transfers
     int nred = 1024;
     double *host_scal = nullptr;               // pinned
     double t = 0, tstage = 0, dt_prev = 0, rate_prev = 0;
@@ -1726,40 +1727,28 @@ static void check_layout(const cles_solver *s, const int64_t padded[3], const in
             throw cles::Error{CLES_ERR_INVALID, "padded extents smaller than n + 2*halo"};
 }
 
+// the padded host layout of the state (decomposition.jl:129-134)
+static void move_state(cles_solver *s, double *Qh, const int64_t padded[3], const int halo[3], bool down)
+{
+    CLES_REQUIRE(s && Qh && padded && halo, "NULL argument");
+    check_layout(s, padded, halo);
+    cles::View3 v;
+    for (int k = 0; k < 3; k++) v.n[k] = s->n[k];
+    v.s[0] = 1;
+    v.s[1] = padded[0];
+    v.s[2] = padded[0] * padded[1];
+    s->stage.transfer(down, s->ctx->device, s->st(), s->Q, v, s->C, padded[0] * padded[1] * padded[2],
+                      Qh + halo[0] + padded[0] * (halo[1] + padded[1] * halo[2]));
+}
+
 int cles_solver_upload(cles_solver *s, const double *Qh, const int64_t padded[3], const int halo[3])
 {
-    CLES_TRY({
-        CLES_REQUIRE(s && Qh && padded && halo, "NULL argument");
-        check_layout(s, padded, halo);
-        const int64_t P0 = padded[0], P1 = padded[1], NP = padded[0] * padded[1] * padded[2];
-        std::vector<double> buf((size_t)s->N * s->C);
-        for (int c = 0; c < s->C; c++)
-            for (int64_t k = 0; k < s->n[2]; k++)
-                for (int64_t j = 0; j < s->n[1]; j++)
-                    std::memcpy(&buf[(size_t)c * s->N + (size_t)s->n[0] * (j + s->n[1] * k)],
-                                Qh + c * NP + halo[0] + P0 * ((j + halo[1]) + P1 * (k + halo[2])),
-                                sizeof(double) * s->n[0]);
-        CLES_HIP(hipMemcpyAsync(s->Q, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice, s->st()));
-        CLES_HIP(hipStreamSynchronize(s->st()));
-    })
+    CLES_TRY({ move_state(s, const_cast<double *>(Qh), padded, halo, false); })
 }
 
 int cles_solver_download(cles_solver *s, double *Qh, const int64_t padded[3], const int halo[3])
 {
-    CLES_TRY({
-        CLES_REQUIRE(s && Qh && padded && halo, "NULL argument");
-        check_layout(s, padded, halo);
-        std::vector<double> buf((size_t)s->N * s->C);
-        CLES_HIP(hipMemcpyAsync(buf.data(), s->Q, buf.size() * sizeof(double), hipMemcpyDeviceToHost, s->st()));
-        CLES_HIP(hipStreamSynchronize(s->st()));
-        const int64_t P0 = padded[0], P1 = padded[1], NP = padded[0] * padded[1] * padded[2];
-        for (int c = 0; c < s->C; c++)
-            for (int64_t k = 0; k < s->n[2]; k++)
-                for (int64_t j = 0; j < s->n[1]; j++)
-                    std::memcpy(Qh + c * NP + halo[0] + P0 * ((j + halo[1]) + P1 * (k + halo[2])),
-                                &buf[(size_t)c * s->N + (size_t)s->n[0] * (j + s->n[1] * k)],
-                                sizeof(double) * s->n[0]);
-    })
+    CLES_TRY({ move_state(s, Qh, padded, halo, true); })
 }
 
 int cles_solver_get_field(cles_solver *s, const char *name, double *host)
