@@ -45,6 +45,7 @@ struct cles_batch {
     cles::LineDev *dplans = nullptr, *fplans = nullptr;
     int *order_d = nullptr, *items_d = nullptr, *order_f = nullptr, *items_f = nullptr;
     int nitems_d = 0, nitems_f = 0, nshort_d = 0, nshort_f = 0;
+    int pmin_d[2] = {64, 64}, pmin_f[2] = {64, 64};   // fewest chunks per line: short, long items
     int dq = 1, dM = 2, dsym = 0, fq = 1, fM = 4, fsym = 1;
 
     // geometry on the device
@@ -143,12 +144,14 @@ struct PlanSet {
     std::vector<LineDev> dev;                       // per instance, pointers are blob offsets
     std::vector<int> order, items;
     int nshort = 0;                                 // leading items of the short class
+    int pmin[2] = {64, 64};                         // fewest chunks per line: short, long items
 };
 
 void build_plan_set(PlanSet &ps, std::vector<unsigned char> &blob, const cles_scheme_desc &s,
                     const std::vector<int> &n, const std::vector<double> &h, int periodic)
 {
     const int64_t count = (int64_t)n.size();
+    RowPool pool;   // chunk blocks of every instance: the lines differ in length, their inner chunks do not
     std::map<std::pair<int, double>, std::pair<LineDev, size_t>> cache;   // (n, h) -> (dev, blob offset)
     ps.dev.resize(count);
     std::vector<int> P(count);
@@ -162,7 +165,7 @@ void build_plan_set(PlanSet &ps, std::vector<unsigned char> &blob, const cles_sc
             // per wave and sweeps half as long); longer ones into up to 32
             LineTables t;
             const int mc = n[i] <= 64 * RAG_SHORT_CHUNK ? RAG_SHORT_CHUNK : RAG_MAX_CHUNK;
-            build_line_tables(t, s, n[i], periodic, h[i], mc, 1, true);
+            build_line_tables(t, s, n[i], periodic, h[i], mc, 1, &pool);
             if (t.dev.P > 64)
                 throw Error{CLES_ERR_UNSUPPORTED, "batched instances are limited to " +
                                                       std::to_string(64 * RAG_MAX_CHUNK) + " points"};
@@ -172,15 +175,26 @@ void build_plan_set(PlanSet &ps, std::vector<unsigned char> &blob, const cles_sc
             // offsets relative to the blob; rebased after upload
             d.coef64 = (const double *)(uintptr_t)(base);
             d.coef32 = (const float *)(uintptr_t)(base + t.o_coef32);
-            d.row64 = (const double *)(uintptr_t)(base + t.o_row64);
-            d.row32 = (const float *)(uintptr_t)(base + t.o_row32);
             d.pcr = (const double *)(uintptr_t)(base + t.o_pcr);
-            d.rowt64 = (const double *)(uintptr_t)(base + t.o_rowt64);
-            d.rowt32 = (const float *)(uintptr_t)(base + t.o_rowt32);
+            d.blk = (const int *)(uintptr_t)(base + t.o_blk);
             it = cache.emplace(key, std::make_pair(d, base)).first;
         }
         ps.dev[i] = it->second.first;
         P[i] = ps.dev[i].P;
+    }
+    const std::vector<float> rows32(pool.rows.begin(), pool.rows.end());
+    auto append = [&](const void *src, size_t bytes) {
+        const size_t base = (blob.size() + 255) & ~(size_t)255;
+        blob.resize(base + bytes);
+        std::memcpy(blob.data() + base, src, bytes);
+        return base;
+    };
+    const size_t o64 = append(pool.rows.data(), pool.rows.size() * sizeof(double));
+    const size_t o32 = append(rows32.data(), rows32.size() * sizeof(float));
+    blob.resize((blob.size() + 255) & ~(size_t)255);
+    for (LineDev &d : ps.dev) {
+        d.rows64 = (const double *)(uintptr_t)o64;
+        d.rows32 = (const float *)(uintptr_t)o32;
     }
     // instances grouped by class (short first), then chunk count; one wave
     // holds 64/P of them
@@ -204,6 +218,7 @@ void build_plan_set(PlanSet &ps, std::vector<unsigned char> &blob, const cles_sc
         ps.items.push_back((int)k);
         ps.items.push_back(cnt);
         if (ck == 0) ps.nshort++;
+        ps.pmin[ck] = std::min(ps.pmin[ck], Pk);
         k += cnt;
     }
 }
@@ -213,11 +228,10 @@ void rebase(std::vector<LineDev> &v, unsigned char *base)
     for (LineDev &d : v) {
         d.coef64 = (const double *)(base + (uintptr_t)d.coef64);
         d.coef32 = (const float *)(base + (uintptr_t)d.coef32);
-        d.row64 = (const double *)(base + (uintptr_t)d.row64);
-        d.row32 = (const float *)(base + (uintptr_t)d.row32);
         d.pcr = (const double *)(base + (uintptr_t)d.pcr);
-        d.rowt64 = (const double *)(base + (uintptr_t)d.rowt64);
-        d.rowt32 = (const float *)(base + (uintptr_t)d.rowt32);
+        d.blk = (const int *)(base + (uintptr_t)d.blk);
+        d.rows64 = (const double *)(base + (uintptr_t)d.rows64);
+        d.rows32 = (const float *)(base + (uintptr_t)d.rows32);
     }
 }
 
@@ -254,6 +268,7 @@ struct BImpl {
         r.items = filter ? b.items_f : b.items_d;
         r.nitems = filter ? b.nitems_f : b.nitems_d;
         r.nshort = filter ? b.nshort_f : b.nshort_d;
+        for (int i = 0; i < 2; i++) r.pmin[i] = filter ? b.pmin_f[i] : b.pmin_d[i];
         r.dt = dtv;
         r.mask = mask;
         r.q = filter ? b.fq : b.dq;
@@ -604,6 +619,10 @@ int cles_batch_create(cles_ctx *ctx, const cles_solver_desc *desc, int64_t count
             b->items_d = b->upload_vec(pd.items);
             b->nitems_d = (int)(pd.items.size() / 3);
             b->nshort_d = pd.nshort;
+            for (int k = 0; k < 2; k++) {
+                b->pmin_d[k] = pd.pmin[k];
+                b->pmin_f[k] = pf.pmin[k];
+            }
             b->order_f = b->upload_vec(pf.order);
             b->items_f = b->upload_vec(pf.items);
             b->nitems_f = (int)(pf.items.size() / 3);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -69,17 +70,17 @@ struct LineDev {
     int extra;      // first `extra` chunks have length m + 1
     const double *coef64;  // [0..8) ci, [8] a0, [16..80) clo[8][8], [80..144) chi[8][8]
     const float *coef32;
-    const double *row64;   // per-row constants, [field * n + g]
-    const float *row32;
     const double *pcr;     // per step s, chunk k: alpha, beta (B*B each, row-major);
                            // then per chunk the final inverse block
-    int cap;               // chunk capacity of the kernels: 8, 16 or 32 >= the longest chunk
-    const double *rowu64;  // per-chunk blocks [(k * nrow + field) * cap + t] of the row constants; rows
-    const float *rowu32;   //   past a chunk's length are zero, and so is its last row's coupling C
-    const double *rowv64;  // the same constants, chunks adjacent: [(field * cap + t) * P + k]
-    const float *rowv32;
-    const double *rowt64;  // chunk-major copy of the per-row constants (ragged plans):
-    const float *rowt32;   //   [(field * RAG_MAX_CHUNK + t) * P + k] = row of point t of chunk k
+    int cap;               // chunk capacity of the kernels: 8, 16 or 32 >= the longest chunk (ragged: 16 or 32)
+    // Row constants: one block [field * cap + t] per distinct chunk, rows past
+    // the chunk's length zero and its last row's coupling C zero (q = 1); chunk
+    // k has the block at rows64 + blk[k].  Chunks inside a line factorise alike,
+    // so a line has at most a few blocks however many chunks it is split into,
+    // and they stay in the nearest cache.
+    const double *rows64;
+    const float *rows32;
+    const int *blk;
 };
 
 constexpr int RAG_MAX_CHUNK = 32;   // points per thread in the ragged kernel
@@ -101,11 +102,16 @@ struct HostPlan {
 struct LineTables {
     LineDev dev{};
     std::vector<unsigned char> image;
-    size_t o_coef32 = 0, o_row64 = 0, o_row32 = 0, o_pcr = 0, o_rowu64 = 0, o_rowu32 = 0, o_rowv64 = 0, o_rowv32 = 0,
-           o_rowt64 = 0, o_rowt32 = 0;
+    size_t o_coef32 = 0, o_pcr = 0, o_blk = 0, o_rows64 = 0, o_rows32 = 0;
 };
-// chunk_major: also store the chunk-major row tables of the ragged kernel
-// (RAG_MAX_CHUNK rows per chunk; max_chunk must not exceed it).
+// Distinct chunk blocks, shared by the plans that are built with one pool.
+struct RowPool {
+    std::map<std::string, int> at;   // a block's bytes -> its offset in `rows`
+    std::vector<double> rows;
+};
+// pool: where the chunk blocks go (the ragged batches share one over all
+// instances; the caller uploads it and binds rows64 / rows32); NULL: the
+// image holds the plan's own.
 // lo_fold (0: none, +1 / -1: the solution parity sigma_g) replaces the low
 // edge's closure by a parity fold on a half-offset grid (operators.jl:59-69,
 // operators_banded.jl:55-64): the LHS coupling to ghost unknown j < 0 moves to
@@ -114,7 +120,7 @@ struct LineTables {
 // for derivatives), carried as synthesised closure rows.
 // hi_fold does the same at the high edge (ghost n + j mirrors n - 1 - j).
 void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int periodic, double h, int max_chunk,
-                       int dim, bool chunk_major = false, int lo_fold = 0, int hi_fold = 0);
+                       int dim, RowPool *pool = nullptr, int lo_fold = 0, int hi_fold = 0);
 void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base);
 
 // Builds the device tables for one (scheme, n, periodic, h).  Throws Error.
@@ -247,6 +253,7 @@ struct RagLines {
     const int *order;        // instances grouped by chunk count
     const int *items;        // 3 ints per work item
     int nitems;
+    int pmin[2];             // fewest chunks per line of the short / long items (LDS size)
     int nshort;              // items [0, nshort) hold lines of chunks of at most RAG_SHORT_CHUNK points
     const double *dt;        // per-instance dt for the LSRK epilogue (NULL: epi.dt)
     const int *mask;         // per-instance: nonzero applies the epilogue (NULL: all)

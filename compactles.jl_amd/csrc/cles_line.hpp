@@ -19,6 +19,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "cles_internal.h"
@@ -45,9 +46,35 @@ template <typename T> __device__ __forceinline__ T gload(const T *ptr)
 template <typename T> __device__ __forceinline__ const T *coefp(const LineDev &p);
 template <> __device__ __forceinline__ const double *coefp<double>(const LineDev &p) { return p.coef64; }
 template <> __device__ __forceinline__ const float *coefp<float>(const LineDev &p) { return p.coef32; }
-template <typename T> __device__ __forceinline__ const T *rowp(const LineDev &p);
-template <> __device__ __forceinline__ const double *rowp<double>(const LineDev &p) { return p.row64; }
-template <> __device__ __forceinline__ const float *rowp<float>(const LineDev &p) { return p.row32; }
+template <typename T> __device__ __forceinline__ const T *rowsp(const LineDev &p);
+template <> __device__ __forceinline__ const double *rowsp<double>(const LineDev &p) { return p.rows64; }
+template <> __device__ __forceinline__ const float *rowsp<float>(const LineDev &p) { return p.rows32; }
+
+// Loads through the constant address space: wave-uniform addresses become
+// scalar loads wherever they stand (tables are never written by a kernel).
+template <typename T> __device__ __forceinline__ T cload(const T *ptr)
+{
+    return *(const __attribute__((address_space(4))) T *)ptr;
+}
+
+// One chunk's block of row constants (LineDev::rows64): row t of field f, read
+// by scalar loads (UNI: the wave has one chunk) or per lane (the lanes of a wave
+// share a few blocks, so a load is a few broadcasts at constant offsets).
+// fence(v) makes per-lane loads that follow wait for v: an empty asm statement
+// through which the base pointer depends on it, which keeps the compiler from
+// issuing every group of rows at once (and spilling them).
+template <typename T, int CAP, bool UNI> struct Rows {
+    const T *base;
+    __device__ __forceinline__ T operator()(int f, int t) const
+    {
+        if constexpr (UNI) return cload(base + f * CAP + t);
+        else return gload(base + f * CAP + t);
+    }
+    template <typename D> __device__ __forceinline__ void fence(const D &dep)
+    {
+        if constexpr (!UNI) asm volatile("" : "+v"(base) : "v"(dep));
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Epilogues
@@ -262,321 +289,202 @@ __device__ __forceinline__ T rhs_row(const T (&fv)[W], int c, const T (&ci)[M], 
     return acc;
 }
 
-template <typename T, int Q, int M, int SYM, int CL = MC>
-struct Chunk {
-    static constexpr int B = 2 * Q;
-    T d[CL];
-
-    // RHS of every row of the chunk from the window fv[t + M] = f[s + t]
-    // (closure rows from fv (low edge, s = 0) and fe[kap] = f[n-1-kap]).
-    __device__ __forceinline__ void rhs(const LineDev &p, int k, int len, const T (&fv)[CL + 2 * M],
-                                        const T (&fe)[8])
-    {
-        const T *cf = coefp<T>(p);
-        T ci[M];
+// RHS of every row of a chunk from its window fv[t + M] = f[s + t]; rows past
+// the chunk's length are zero.  At a closed line's ends (first, last: the lane
+// holds that chunk) the closure rows replace the first and last nc rows, from
+// fv and from fe[kap] = f[n - 1 - kap].  tmin: the fewest points of a chunk of
+// this launch that the compiler may count on.  MUNI: p.m is wave-uniform (the
+// last chunk holds p.m points, so its closure rows sit at wave-uniform t).
+template <typename T, int M, int SYM, int CL, bool FULL, bool MUNI, int TMIN>
+__device__ __forceinline__ void chunk_rhs(const LineDev &p, const T (&fv)[CL + 2 * M], const T (&fe)[8], bool first,
+                                          bool last, int len, T (&d)[CL])
+{
+    const T *cf = coefp<T>(p);
+    auto ld = [](const T *q) {
+        if constexpr (MUNI) return cload(q);
+        else return gload(q);
+    };
+    T ci[M];
 #pragma unroll
-        for (int m = 0; m < M; m++) ci[m] = cf[COEF_CI + m];
-        const T a0 = cf[COEF_A0];
-        const bool lo = p.closed && k == 0;
-        const bool hi = p.closed && k == p.P - 1;
+    for (int m = 0; m < M; m++) ci[m] = ld(cf + COEF_CI + m);
+    const T a0 = ld(cf + COEF_A0);
+#pragma unroll
+    for (int t = 0; t < CL; t++) {
+        d[t] = rhs_row<T, M, SYM>(fv, t + M, ci, a0);
+        if (!FULL && t >= TMIN) d[t] = t < len ? d[t] : T(0);
+    }
+    if (!p.closed) return;
+#pragma unroll
+    for (int t = 0; t < NCMAX; t++) {
+        if (t >= p.nc) continue;
+        const T *cr = cf + COEF_CLO + t * 8;
+        T acc = ld(cr) * fv[M];
+#pragma unroll
+        for (int kap = 1; kap < 8; kap++) {
+            // points past a line shorter than the stencil take a zero weight
+            const T fk = kap < p.n ? fv[kap + M] : T(0);
+            acc = fma(ld(cr + kap), fk, acc);
+        }
+        d[t] = first ? acc : d[t];
+    }
+    if constexpr (MUNI) {
 #pragma unroll
         for (int t = 0; t < CL; t++) {
-            T acc = rhs_row<T, M, SYM>(fv, t + M, ci, a0);
-            if (t < NCMAX) {
-                if (lo && t < p.nc) {
-                    const T *cr = cf + COEF_CLO + t * 8;
-                    acc = cr[0] * fv[M];
+            const int jr = p.m - 1 - t;
+            if (jr < 0 || jr >= p.nc) continue;
+            const T *cr = cf + COEF_CHI + jr * 8;
+            T acc = ld(cr) * fe[0];
 #pragma unroll
-                    for (int kap = 1; kap < 8; kap++) acc = fma(cr[kap], fv[kap + M], acc);
-                }
-            }
-            if (hi) {
-                const int jr = len - 1 - t;
-                if (jr >= 0 && jr < p.nc) {
-                    const T *cr = cf + COEF_CHI + jr * 8;
-                    acc = cr[0] * fe[0];
-#pragma unroll
-                    for (int kap = 1; kap < 8; kap++) acc = fma(cr[kap], fe[kap], acc);
-                }
-            }
-            d[t] = acc;
-        }
-    }
-
-    // chunk-local forward/backward sweeps
-    __device__ __forceinline__ void solve(const LineDev &p, int rs, int len)
-    {
-        const int n = p.n;
-        const T *rw = rowp<T>(p);
-        if constexpr (Q == 1) {
-            const T *rl = rw + (size_t)R1_L * n + rs;
-            const T *rdi = rw + (size_t)R1_DINV * n + rs;
-            const T *rc = rw + (size_t)R1_C * n + rs;
-#pragma unroll
-            for (int t = 1; t < CL; t++)
-                if (t < len) d[t] = fma(-rl[t], d[t - 1], d[t]);
-#pragma unroll
-            for (int t = CL - 1; t >= 0; t--) {
-                if (t < len) {
-                    const T nxt = d[t + 1 < CL ? t + 1 : CL - 1];
-                    d[t] = (t == len - 1) ? d[t] * rdi[t] : fma(-rc[t], nxt, d[t]) * rdi[t];
-                }
-            }
-        } else {
-            const T *l1 = rw + (size_t)R2_L1 * n + rs;
-            const T *l2 = rw + (size_t)R2_L2 * n + rs;
-            const T *u0 = rw + (size_t)R2_U0INV * n + rs;
-            const T *u1 = rw + (size_t)R2_U1 * n + rs;
-            const T *u2 = rw + (size_t)R2_U2 * n + rs;
-#pragma unroll
-            for (int t = 0; t < CL - 1; t++) {
-                if (t < len - 1) {
-                    const T xt = d[t];
-                    d[t + 1] = fma(-l1[t], xt, d[t + 1]);
-                    if (t + 2 < CL)
-                        if (t < len - 2) d[t + 2 < CL ? t + 2 : t] = fma(-l2[t], xt, d[t + 2 < CL ? t + 2 : t]);
-                }
-            }
-#pragma unroll
-            for (int t = CL - 1; t >= 0; t--) {
-                if (t < len) {
-                    T acc = d[t];
-                    if (t + 1 < CL)
-                        if (t + 1 < len) acc = fma(-u1[t], d[t + 1 < CL ? t + 1 : t], acc);
-                    if (t + 2 < CL)
-                        if (t + 2 < len) acc = fma(-u2[t], d[t + 2 < CL ? t + 2 : t], acc);
-                    d[t] = acc * u0[t];
-                }
-            }
-        }
-    }
-
-    __device__ __forceinline__ void ends(int len, double (&r)[B]) const
-    {
-#pragma unroll
-        for (int i = 0; i < Q; i++) r[i] = (double)d[i];
-#pragma unroll
-        for (int t = 0; t < CL; t++)
-#pragma unroll
-            for (int i = 0; i < Q; i++)
-                if (t == len - Q + i) r[Q + i] = (double)d[t];
-    }
-};
-
-// Chunk sweeps and spike correction with the row constants read G rows at a
-// time: the loads of group g + 1 are issued once the arithmetic of group g - 1
-// is done and before that of group g, so each group waits for one round trip
-// (instead of every row waiting for its own inside the dependency chain) while
-// only two groups of rows are held in registers.  Rows::fence(v) is an empty
-// asm statement that makes the table pointer depend on v, which keeps the
-// compiler from issuing a group's loads earlier than that.  Rows(field, t)
-// must be in bounds for every t < CL (rows past the chunk's length read
-// padding or a clamped row); rows t >= len are left unchanged through
-// selects, so the arithmetic of rows t < len is that of Chunk::solve /
-// corrected(), operation for operation.
-template <typename T, int Q, int CL, int G, typename Rows>
-__device__ __forceinline__ void solve_grouped(T (&d)[CL], int len, Rows R)
-{
-    static_assert(CL % G == 0, "group size must divide the chunk length");
-    constexpr int NG = CL / G;
-    if constexpr (Q == 1) {
-        T cur[G], nxt[G];
-#pragma unroll
-        for (int i = 0; i < G; i++) cur[i] = R(R1_L, i);
-#pragma unroll
-        for (int g = 0; g < NG; g++) {
-            if (g + 1 < NG) {
-                if (g > 0) R.fence(d[g * G - 1]);
-#pragma unroll
-                for (int i = 0; i < G; i++) nxt[i] = R(R1_L, (g + 1) * G + i);
-            }
-#pragma unroll
-            for (int i = 0; i < G; i++) {
-                const int t = g * G + i;
-                if (t >= 1) {
-                    const T nv = fma(-cur[i], d[t - 1], d[t]);
-                    d[t] = t < len ? nv : d[t];
-                }
-            }
-            if (g + 1 < NG) {
-#pragma unroll
-                for (int i = 0; i < G; i++) cur[i] = nxt[i];
-            }
-        }
-        T cc[G], cd[G], nc[G], nd[G];
-        R.fence(d[CL - 1]);
-#pragma unroll
-        for (int i = 0; i < G; i++) {
-            cc[i] = R(R1_C, (NG - 1) * G + i);
-            cd[i] = R(R1_DINV, (NG - 1) * G + i);
-        }
-#pragma unroll
-        for (int g = NG - 1; g >= 0; g--) {
-            if (g > 0) {
-                if (g < NG - 1) R.fence(d[(g + 1) * G]);
-#pragma unroll
-                for (int i = 0; i < G; i++) {
-                    nc[i] = R(R1_C, (g - 1) * G + i);
-                    nd[i] = R(R1_DINV, (g - 1) * G + i);
-                }
-            }
-#pragma unroll
-            for (int i = G - 1; i >= 0; i--) {
-                const int t = g * G + i;
-                const T nx = d[t + 1 < CL ? t + 1 : CL - 1];
-                const T v = (t == len - 1) ? d[t] * cd[i] : fma(-cc[i], nx, d[t]) * cd[i];
-                d[t] = t < len ? v : d[t];
-            }
-            if (g > 0) {
-#pragma unroll
-                for (int i = 0; i < G; i++) {
-                    cc[i] = nc[i];
-                    cd[i] = nd[i];
-                }
-            }
+            for (int kap = 1; kap < 8; kap++) acc = fma(ld(cr + kap), fe[kap], acc);
+            d[t] = last ? acc : d[t];
         }
     } else {
-        T a1[G], a2[G], b1[G], b2[G];
 #pragma unroll
-        for (int i = 0; i < G; i++) {
-            a1[i] = R(R2_L1, i);
-            a2[i] = R(R2_L2, i);
-        }
+        for (int jr = 0; jr < NCMAX; jr++) {
+            if (jr >= p.nc) continue;
+            const T *cr = cf + COEF_CHI + jr * 8;
+            T acc = ld(cr) * fe[0];
 #pragma unroll
-        for (int g = 0; g < NG; g++) {
-            if (g + 1 < NG) {
-                if (g > 0) R.fence(d[g * G - 1]);
+            for (int kap = 1; kap < 8; kap++) acc = fma(ld(cr + kap), fe[kap], acc);
+            const int at = last ? len - 1 - jr : -1;
 #pragma unroll
-                for (int i = 0; i < G; i++) {
-                    b1[i] = R(R2_L1, (g + 1) * G + i);
-                    b2[i] = R(R2_L2, (g + 1) * G + i);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < G; i++) {
-                const int t = g * G + i;
-                if (t < CL - 1) {
-                    const T xt = d[t];
-                    const T n1 = fma(-a1[i], xt, d[t + 1]);
-                    d[t + 1] = t < len - 1 ? n1 : d[t + 1];
-                    if (t + 2 < CL) {
-                        const T n2 = fma(-a2[i], xt, d[t + 2 < CL ? t + 2 : t]);
-                        d[t + 2 < CL ? t + 2 : t] = t < len - 2 ? n2 : d[t + 2 < CL ? t + 2 : t];
-                    }
-                }
-            }
-            if (g + 1 < NG) {
-#pragma unroll
-                for (int i = 0; i < G; i++) {
-                    a1[i] = b1[i];
-                    a2[i] = b2[i];
-                }
-            }
-        }
-        T u0[G], u1[G], u2[G], w0[G], w1[G], w2[G];
-        R.fence(d[CL - 1]);
-#pragma unroll
-        for (int i = 0; i < G; i++) {
-            u0[i] = R(R2_U0INV, (NG - 1) * G + i);
-            u1[i] = R(R2_U1, (NG - 1) * G + i);
-            u2[i] = R(R2_U2, (NG - 1) * G + i);
-        }
-#pragma unroll
-        for (int g = NG - 1; g >= 0; g--) {
-            if (g > 0) {
-                if (g < NG - 1) R.fence(d[(g + 1) * G]);
-#pragma unroll
-                for (int i = 0; i < G; i++) {
-                    w0[i] = R(R2_U0INV, (g - 1) * G + i);
-                    w1[i] = R(R2_U1, (g - 1) * G + i);
-                    w2[i] = R(R2_U2, (g - 1) * G + i);
-                }
-            }
-#pragma unroll
-            for (int i = G - 1; i >= 0; i--) {
-                const int t = g * G + i;
-                T acc = d[t];
-                if (t + 1 < CL) {
-                    const T x1 = fma(-u1[i], d[t + 1 < CL ? t + 1 : t], acc);
-                    acc = t + 1 < len ? x1 : acc;
-                }
-                if (t + 2 < CL) {
-                    const T x2 = fma(-u2[i], d[t + 2 < CL ? t + 2 : t], acc);
-                    acc = t + 2 < len ? x2 : acc;
-                }
-                d[t] = t < len ? acc * u0[i] : d[t];
-            }
-            if (g > 0) {
-#pragma unroll
-                for (int i = 0; i < G; i++) {
-                    u0[i] = w0[i];
-                    u1[i] = w1[i];
-                    u2[i] = w2[i];
-                }
-            }
+            for (int t = 0; t < CL; t++) d[t] = t == at ? acc : d[t];
         }
     }
 }
 
-// x = y - V tail_prev - W head_next for every row of the chunk, the FP64 spike
-// rows read in groups as above (Rows64(field, t) in bounds for t < CL).
-template <typename T, int Q, int CL, int G, typename Rows64>
-__device__ __forceinline__ void correct_grouped(T (&d)[CL], int len, Rows64 R, const double (&tp)[Q],
-                                                const double (&hn)[Q])
+// Chunk sweeps (src/tridiag.jl:46-57, src/banded.jl:63-80) over all CL rows:
+// rows past the chunk's length hold zeros and multiply by zeros.  The row
+// constants are read G rows at a time: the loads of group g + 1 are issued once
+// the arithmetic of group g - 1 is done and before that of group g, so each
+// group waits for one round trip while two groups are held in registers.
+template <typename T, int Q, int CL, int G, typename Rows>
+__device__ __forceinline__ void solve_padded(T (&d)[CL], Rows R)
 {
     constexpr int NG = CL / G;
-    constexpr int NF = 2 * Q;
-    const int fld[4] = {Q == 1 ? (int)R1_V : (int)R2_V0, Q == 1 ? (int)R1_W : (int)R2_W0,
-                        Q == 1 ? 0 : (int)R2_V1, Q == 1 ? 0 : (int)R2_W1};
-    double cur[NF][G], nxt[NF][G];
+    constexpr int NL = Q, NU = Q == 1 ? 2 : 3;
+    const int fl[2] = {Q == 1 ? (int)R1_L : (int)R2_L1, (int)R2_L2};
+    const int fu[3] = {Q == 1 ? (int)R1_DINV : (int)R2_U0INV, Q == 1 ? (int)R1_C : (int)R2_U1, (int)R2_U2};
+    T c[NL][G], nx[NL][G];
 #pragma unroll
-    for (int f = 0; f < NF; f++)
+    for (int f = 0; f < NL; f++)
 #pragma unroll
-        for (int i = 0; i < G; i++) cur[f][i] = R(fld[f], i);
+        for (int i = 0; i < G; i++) c[f][i] = R(fl[f], i);
 #pragma unroll
     for (int g = 0; g < NG; g++) {
         if (g + 1 < NG) {
             if (g > 0) R.fence(d[g * G - 1]);
 #pragma unroll
-            for (int f = 0; f < NF; f++)
+            for (int f = 0; f < NL; f++)
 #pragma unroll
-                for (int i = 0; i < G; i++) nxt[f][i] = R(fld[f], (g + 1) * G + i);
+                for (int i = 0; i < G; i++) nx[f][i] = R(fl[f], (g + 1) * G + i);
         }
 #pragma unroll
         for (int i = 0; i < G; i++) {
             const int t = g * G + i;
-            double acc = fma(cur[1][i], hn[0], cur[0][i] * tp[0]);
-            if constexpr (Q == 2) {
-                acc = fma(cur[2][i], tp[1], acc);
-                acc = fma(cur[3][i], hn[1], acc);
+            if constexpr (Q == 1) {
+                if (t >= 1) d[t] = fma(-c[0][i], d[t - 1], d[t]);
+            } else {
+                if (t + 1 < CL) d[t + 1] = fma(-c[0][i], d[t], d[t + 1]);
+                if (t + 2 < CL) d[t + 2] = fma(-c[1][i], d[t], d[t + 2]);
             }
-            const T c = (T)((double)d[t] - acc);
-            d[t] = t < len ? c : d[t];
         }
         if (g + 1 < NG) {
 #pragma unroll
-            for (int f = 0; f < NF; f++)
+            for (int f = 0; f < NL; f++)
 #pragma unroll
-                for (int i = 0; i < G; i++) cur[f][i] = nxt[f][i];
+                for (int i = 0; i < G; i++) c[f][i] = nx[f][i];
+        }
+    }
+    T u[NU][G], nu[NU][G];
+    R.fence(d[CL - 1]);
+#pragma unroll
+    for (int f = 0; f < NU; f++)
+#pragma unroll
+        for (int i = 0; i < G; i++) u[f][i] = R(fu[f], (NG - 1) * G + i);
+#pragma unroll
+    for (int g = NG - 1; g >= 0; g--) {
+        if (g > 0) {
+            if (g < NG - 1) R.fence(d[(g + 1) * G]);
+#pragma unroll
+            for (int f = 0; f < NU; f++)
+#pragma unroll
+                for (int i = 0; i < G; i++) nu[f][i] = R(fu[f], (g - 1) * G + i);
+        }
+#pragma unroll
+        for (int i = G - 1; i >= 0; i--) {
+            const int t = g * G + i;
+            T acc = d[t];
+            if (t + 1 < CL) acc = fma(-u[1][i], d[t + 1 < CL ? t + 1 : t], acc);
+            if constexpr (Q == 2)
+                if (t + 2 < CL) acc = fma(-u[2][i], d[t + 2 < CL ? t + 2 : t], acc);
+            d[t] = acc * u[0][i];
+        }
+        if (g > 0) {
+#pragma unroll
+            for (int f = 0; f < NU; f++)
+#pragma unroll
+                for (int i = 0; i < G; i++) u[f][i] = nu[f][i];
         }
     }
 }
 
-// Row-major plan rows of the chunk starting at s (row index clamped to the line)
-template <typename T>
-struct RowsClamped {
-    const T *base;
-    int n, s;
-    __device__ __forceinline__ T operator()(int f, int t) const
-    {
-        const int g = s + t < n ? s + t : n - 1;
-        return gload(base + (size_t)f * n + g);
+// The 2Q end values of a chunk of len points (TMIN as in chunk_rhs).
+template <typename T, int Q, int CL, bool FULL, int TMIN>
+__device__ __forceinline__ void chunk_ends(const T (&d)[CL], int len, double (&r)[2 * Q])
+{
+#pragma unroll
+    for (int i = 0; i < Q; i++) {
+        r[i] = (double)d[i];
+        if constexpr (FULL) {
+            r[Q + i] = (double)d[CL - Q + i];
+        } else {
+            constexpr int T0 = TMIN - Q > 0 ? TMIN - Q : 0;
+            T x = d[T0];
+#pragma unroll
+            for (int t = T0 + 1; t < CL; t++) {
+                // the value is read before the choice: a choice between
+                // addresses would put the whole chunk into scratch memory
+                const T y = d[t];
+                x = t == len - Q + i ? y : x;
+            }
+            r[Q + i] = (double)x;
+        }
     }
-    template <typename D> __device__ __forceinline__ void fence(const D &dep)
-    {
-        asm volatile("" : "+v"(base) : "v"(dep));
+}
+
+// x = y - V tail_prev - W head_next (src/tridiag.jl:159-168, src/banded.jl:
+// 371-382) for every row, the FP64 spike rows read G at a time; put(t, value)
+// takes each row.
+template <typename T, int Q, int CL, int G, typename R64, typename Put>
+__device__ __forceinline__ void correct_padded(T (&d)[CL], R64 R, const double (&tp)[Q], const double (&hn)[Q], Put put)
+{
+#pragma unroll
+    for (int g = 0; g < CL / G; g++) {
+        if (g > 0) R.fence(d[g * G - 1]);
+        double c[2 * Q][G];
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            c[0][i] = R(Q == 1 ? (int)R1_V : (int)R2_V0, g * G + i);
+            c[1][i] = R(Q == 1 ? (int)R1_W : (int)R2_W0, g * G + i);
+            if constexpr (Q == 2) {
+                c[2][i] = R(R2_V1, g * G + i);
+                c[3][i] = R(R2_W1, g * G + i);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            const int t = g * G + i;
+            double acc = fma(c[1][i], hn[0], c[0][i] * tp[0]);
+            if constexpr (Q == 2) {
+                acc = fma(c[2][i], tp[1], acc);
+                acc = fma(c[3][i], hn[1], acc);
+            }
+            d[t] = (T)((double)d[t] - acc);
+            put(t, d[t]);
+        }
     }
-};
+}
 
 // Reduced interface system: block PCR across the P chunks of each line
 // (slot = chunk * nl + line-in-block), then fetch the previous chunk's tail
@@ -707,30 +615,13 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
     }
 }
 
-template <typename T, int Q>
-__device__ __forceinline__ double corrected(const LineDev &p, int g, T y, const double (&tp)[Q],
-                                            const double (&hn)[Q])
-{
-    const int n = p.n;
-    const double *rw = p.row64;
-    if constexpr (Q == 1) {
-        return (double)y - fma(rw[(size_t)R1_W * n + g], hn[0], rw[(size_t)R1_V * n + g] * tp[0]);
-    } else {
-        double acc = rw[(size_t)R2_V0 * n + g] * tp[0];
-        acc = fma(rw[(size_t)R2_W0 * n + g], hn[0], acc);
-        acc = fma(rw[(size_t)R2_V1 * n + g], tp[1], acc);
-        acc = fma(rw[(size_t)R2_W1 * n + g], hn[1], acc);
-        return (double)y - acc;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // y / z sweeps, one chunk per wave: 64 lanes along x with V adjacent lines per
 // lane, so a row is one contiguous segment of 64 V values and every per-row
 // constant is wave-uniform.
 //
 // Bound: HBM for FP64 and large FP32 grids, instruction issue before that.  The
-// row constants come from per-chunk blocks padded with zeros (LineDev::rowu64),
+// row constants come from chunk blocks padded with zeros (LineDev::rows64),
 // so the sweeps run CL unconditional steps: a row past the chunk's length only
 // multiplies by zeros, and the last row's coupling is stored as zero.  Every
 // window load is unconditional too, from the row wrapped or clamped into the
@@ -758,16 +649,6 @@ __device__ __forceinline__ unsigned xcd_slab(unsigned b, unsigned nb)
     const unsigned nfull = nb & ~7u;
     return b < nfull ? (b & 7u) * (nfull >> 3) + (b >> 3) : b;
 }
-
-// Loads through the constant address space: wave-uniform addresses become
-// scalar loads wherever they stand (tables are never written by a kernel).
-template <typename T> __device__ __forceinline__ T cload(const T *ptr)
-{
-    return *(const __attribute__((address_space(4))) T *)ptr;
-}
-template <typename T> __device__ __forceinline__ const T *rowup(const LineDev &p);
-template <> __device__ __forceinline__ const double *rowup<double>(const LineDev &p) { return p.rowu64; }
-template <> __device__ __forceinline__ const float *rowup<float>(const LineDev &p) { return p.rowu32; }
 
 // V adjacent values as one access; elements are only element-aligned (odd
 // strides and halos), which the memory unit takes for global accesses.
@@ -925,7 +806,7 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
 {
     select_field<T, EPI>(mf, f, e);
     extern __shared__ double smem[];
-    constexpr int B = 2 * Q, NROW = Q == 1 ? (int)R1_N : (int)R2_N;
+    constexpr int B = 2 * Q;
     const int P = p.P, n = p.n;
     const int NT = 64 * P;
     const int lane = (int)(threadIdx.x & 63);
@@ -1019,7 +900,8 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
     }
 
     // chunk sweeps (src/tridiag.jl:46-57, src/banded.jl:63-80)
-    const T *rw = rowup<T>(p) + (size_t)k * NROW * CL;
+    const int rows = cload(p.blk + k);
+    const T *rw = rowsp<T>(p) + rows;
     if constexpr (Q == 1) {
         const T *rl = rw + R1_L * CL, *rdi = rw + R1_DINV * CL, *rc = rw + R1_C * CL;
 #pragma unroll
@@ -1077,7 +959,7 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
     if (!valid) return;
 
     // spike correction, FP64 as the reduced system
-    const double *rv = p.rowu64 + (size_t)k * NROW * CL;
+    const double *rv = p.rows64 + rows;
     // the Runge-Kutta epilogues hold three inputs per point: four rows at a
     // time where eight would spill
     constexpr int NB = (EPI == EPI_LSRK || EPI == EPI_LSRK_DEV) && (CL > 16 || V > 1) ? 4 : 8;
@@ -1130,7 +1012,6 @@ __global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restri
     const int xi = xb * Lx + lane;
     const bool valid = xi < nlane;
     const int64_t off = (int64_t)xi + ob * so;
-    const T *fl = f + off;
     const int n = p.n;
     const int s = k * p.m + min(k, p.extra);
     const int len = p.m + (k < p.extra ? 1 : 0);
@@ -1159,162 +1040,155 @@ __global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restri
     T fe[8];
 #pragma unroll
     for (int kap = 0; kap < 8; kap++) fe[kap] = T(0);
-    if (p.closed && k == p.P - 1 && valid) {
+    if (p.closed) {
 #pragma unroll
         for (int kap = 0; kap < 8; kap++)
-            if (kap < n) fe[kap] = fl[(n - 1 - kap) * sd];
+            if (kap < n) fe[kap] = fa[(int64_t)(n - 1 - kap) * sd];
     }
 
-    Chunk<T, Q, M, SYM, CL> ch;
-    ch.rhs(p, k, len, fv, fe);
-    // grouped row loads where they fit the 128 registers of a 1024-thread
-    // block (chunks of up to 16 points)
-    constexpr bool GRP = CL <= 16;
+    constexpr int TMIN = CL == 8 ? 1 : CL / 2;
     constexpr int G = CL <= 8 ? CL : 4;
-    if constexpr (GRP)
-        solve_grouped<T, Q, CL, G>(ch.d, len, RowsClamped<T>{rowp<T>(p), n, s});
-    else
-        ch.solve(p, s, len);
+    T d[CL];
+    chunk_rhs<T, M, SYM, CL, false, true, TMIN>(p, fv, fe, k == 0, k == p.P - 1, len, d);
+    const int blk = p.blk[k];
+    solve_padded<T, Q, CL, G>(d, Rows<T, CL, false>{rowsp<T>(p) + blk});
     double r[2 * Q], tp[Q], hn[Q];
-    ch.ends(len, r);
+    chunk_ends<T, Q, CL, false, TMIN>(d, len, r);
     reduced_solve<Q, Q == 1 && sizeof(T) == 8>(p, smem, NT, Lx, k, lane, r, tp, hn);
     if (!valid) return;
-    if constexpr (GRP) {
-        correct_grouped<T, Q, CL, G>(ch.d, len, RowsClamped<double>{p.row64, n, s}, tp, hn);
-    } else {
-#pragma unroll
-        for (int t = 0; t < CL; t++)
-            if (t < len) ch.d[t] = (T)corrected<T, Q>(p, s + t, ch.d[t], tp, hn);
-    }
+    correct_padded<T, Q, CL, G>(d, Rows<double, CL, false>{p.rows64 + blk}, tp, hn, [](int, T) {});
     // the device-dt LSRK epilogue (per-point gate and dt beside three
     // inputs) goes four points at a time at the full capacity (no spills)
     constexpr int NB = EPI == EPI_LSRK_DEV && CL > 16 ? 4 : 8;
 #pragma unroll
     for (int b = 0; b < CL; b += NB) {
         int64_t o[NB];
-        T v[NB];
+        T v[1][NB];
         bool ok[NB];
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             ok[i] = b + i < len;
-            o[i] = off + (int64_t)(s + b + i) * sd;
-            v[i] = ch.d[b + i];
+            o[i] = off + (int64_t)(ok[i] ? s + b + i : s) * sd;
+            v[0][i] = d[b + i];
         }
-        epilogue_batch<T, EPI, NB>(e, o, v, ok);
+        epilogue_rows<T, EPI, NB, 1, false>(e, o, v, ok);
     }
 }
 
 // ---------------------------------------------------------------------------
-// x sweep: Lt whole lines staged in LDS (row stride n + 1), threads own
-// (line, chunk) pairs, tid = line + Lt * chunk.  Lines are indexed
-// l = j + ny*k over the y-z plane.  UNI: Lt == 64 (one chunk per wave).
+// x sweep, block-wide: lines of more than 64 chunks (or of chunks longer than
+// 16 points).  The block stages Lt whole lines in LDS with the M halo points at
+// both ends; thread li P + k owns chunk k of line li, so the lanes of a wave
+// hold adjacent chunks; results return through the tile.  As in the wave-local
+// sweep, no element index is divided by the line length, window reads need no
+// wrap test and the sweeps run on zero-padded rows.  60 steps of the 1024 x 512
+// shock / interface FP64 and the state's return, this kernel and the narrow y
+// sweep on row-major tables / on shared chunk blocks: 84.6 / 80.5 ms.
 // ---------------------------------------------------------------------------
-template <typename T, int Q, int M, int SYM, int EPI, bool UNI, int CL = MC>
-__global__ void __launch_bounds__(UNI && Q == 1 ? 1024 : 512, !UNI && CL <= 8 && Q == 1 ? 5 : 1) k_line_x(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz,
-                                                 int ny, int64_t nlines, int Lt, EpiArgs e, LineFields mf)
+template <int XC> __device__ __forceinline__ int xw_slot(int x) { return x + x / XC; }
+
+template <typename T, int Q, int M, int SYM, int EPI, int CL>
+__global__ void __launch_bounds__(512, CL <= 8 && Q == 1 ? 4 : 1)
+k_line_x(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz, int ny, int64_t nlines, int Lt, int TS, bool overlay,
+         EpiArgs e, LineFields mf)
 {
     select_field<T, EPI>(mf, f, e);
     extern __shared__ double smem[];
-    const int n = p.n;
-    const int TS = n + 1;
-    const int NT = Lt * p.P;
+    const int n = p.n, P = p.P;
+    const int NT = Lt * P;
     T *tile = (T *)smem;
-    double *buf = smem + (((size_t)Lt * TS * sizeof(T) + 7) / 8);
+    // overlay: the exchange buffers share the tile's memory, between barriers
+    // of their own (lines that leave no room for both)
+    double *buf = overlay ? smem : smem + (((size_t)Lt * TS * sizeof(T) + 7) / 8);
     const int tid = threadIdx.x;
     const int64_t l0 = (int64_t)blockIdx.x * Lt;
-
-    if constexpr (!UNI && CL <= 8) {
-        // element q = tid + NT i of the block's Lt lines is line q / n, point
-        // q % n; a thread holds at most ceil(n / P) <= CL of them, and all its
-        // loads are issued before the LDS writes
-        const int nel = Lt * n;
-        const int j0 = (int)(l0 % ny), k0 = (int)(l0 / ny);
-        T tmp[CL];
-        int dst[CL];
+    const int left = (int)(nlines - l0 < Lt ? nlines - l0 : Lt);   // lines that exist, >= 1
+    const int seg = (n + NT - 1) / NT;
+    // element i of this thread: point x = tid + q NT of line lj, segment by segment
+    struct Walk {
+        int q, lj;
+    };
+    auto next = [&](Walk &w) {
+        const bool turn = w.q + 1 == seg;
+        w.q = turn ? 0 : w.q + 1;
+        w.lj += turn ? 1 : 0;
+    };
+    // a launch holds fewer than 2^32 threads, hence fewer lines
+    auto line_off = [&](int lj) -> int64_t {
+        const uint32_t l = (uint32_t)l0 + (uint32_t)(lj < left ? lj : 0);
+        const uint32_t kk = l / (uint32_t)ny;
+        return (int64_t)(l - kk * (uint32_t)ny) * sy + (int64_t)kk * sz;
+    };
+    {
+        Walk w{0, 0};
+        for (int e0 = 0; e0 < Lt * seg; e0 += CL) {
+            T tmp[CL];
+            Walk u = w;
 #pragma unroll
-        for (int i = 0; i < CL; i++) {
-            const int q = tid + NT * i;
-            const int lj = q / n, x = q - lj * n;
-            int j = j0 + lj, kk = k0;
-            while (j >= ny) {
-                j -= ny;
-                kk++;
+            for (int i = 0; i < CL; i++) {
+                const int x = tid + u.q * NT;
+                tmp[i] = f[line_off(u.lj) + (x < n ? x : n - 1)];
+                next(u);
             }
-            const bool ok = q < nel && l0 + lj < nlines;
-            tmp[i] = ok ? f[(int64_t)j * sy + (int64_t)kk * sz + x] : T(0);
-            dst[i] = q < nel ? lj * TS + x : -1;
-        }
 #pragma unroll
-        for (int i = 0; i < CL; i++)
-            if (dst[i] >= 0) tile[dst[i]] = tmp[i];
-    } else {
-        for (int li = 0; li < Lt; li++) {
-            const int64_t l = l0 + li;
-            if (l >= nlines) break;
-            const T *src = f + (l % ny) * sy + (l / ny) * sz;
-            for (int i = tid; i < n; i += NT) tile[li * TS + i] = src[i];
+            for (int i = 0; i < CL; i++) {
+                const int x = tid + w.q * NT;
+                if (w.lj < Lt && x < n) tile[w.lj * TS + xw_slot<CL>(x + M)] = tmp[i];
+                next(w);
+            }
+        }
+        for (int h = tid; h < Lt * 2 * M; h += NT) {
+            const int lj = h / (2 * M), hx = h % (2 * M);
+            T v = T(0);
+            if (p.periodic) v = f[line_off(lj) + (hx < M ? n - M + hx : hx - M)];
+            tile[lj * TS + xw_slot<CL>(hx < M ? hx : hx + n)] = v;
         }
     }
     __syncthreads();
 
-    const int li = UNI ? (tid & 63) : (tid % Lt);
-    int k = UNI ? (tid >> 6) : (tid / Lt);
-    if constexpr (UNI) k = __builtin_amdgcn_readfirstlane(k);
+    const int k = tid & (P - 1), li = tid / P;
     const int s = k * p.m + min(k, p.extra);
     const int len = p.m + (k < p.extra ? 1 : 0);
-    const T *trow = tile + li * TS;
-    T fv[CL + 2 * M];
+    T *trow = tile + li * TS;
+    constexpr int TMIN = CL == 8 ? 1 : CL / 2;
+    constexpr int G = CL <= 8 ? 8 : 4;
+    T d[CL];
+    {
+        T fv[CL + 2 * M], fe[8];
 #pragma unroll
-    for (int t = -M; t < CL + M; t++) {
-        T val = T(0);
-        if (t < len + M) {
-            int r = s + t;
-            bool ok = true;
-            if (r < 0) {
-                if (p.periodic) r += n; else ok = false;
-            } else if (r >= n) {
-                if (p.periodic) r -= n; else ok = false;
-            }
-            if (ok) val = trow[r];
-        }
-        fv[t + M] = val;
+        for (int t = 0; t < CL + 2 * M; t++) fv[t] = trow[xw_slot<CL>(s + t)];
+#pragma unroll
+        for (int kap = 0; kap < 8; kap++)
+            fe[kap] = p.closed && kap < n ? trow[xw_slot<CL>(n - 1 - kap + M)] : T(0);
+        chunk_rhs<T, M, SYM, CL, false, true, TMIN>(p, fv, fe, k == 0, k == P - 1, len, d);
     }
-    T fe[8];
-#pragma unroll
-    for (int kap = 0; kap < 8; kap++) fe[kap] = (p.closed && kap < n) ? trow[n - 1 - kap] : T(0);
-
-    Chunk<T, Q, M, SYM, CL> ch;
-    ch.rhs(p, k, len, fv, fe);
-    // grouped row loads where they fit the 128 registers of a 1024-thread
-    // block (chunks of up to 16 points); wave-uniform rows (UNI) are scalar loads
-    constexpr bool GRP = !UNI && CL <= 16;
-    constexpr int G = CL <= 8 ? CL : 4;
-    if constexpr (GRP)
-        solve_grouped<T, Q, CL, G>(ch.d, len, RowsClamped<T>{rowp<T>(p), n, s});
-    else
-        ch.solve(p, s, len);
+    const int blk = p.blk[k];
+    solve_padded<T, Q, CL, G>(d, Rows<T, CL, false>{rowsp<T>(p) + blk});
     double r[2 * Q], tp[Q], hn[Q];
-    ch.ends(len, r);
-    reduced_solve<Q, !UNI && Q == 1>(p, buf, NT, Lt, k, li, r, tp, hn);
-    // every thread has finished reading the tile before the first reduced-solve barrier
-    T *wrow = tile + li * TS;
-    if constexpr (GRP) {
-        correct_grouped<T, Q, CL, G>(ch.d, len, RowsClamped<double>{p.row64, n, s}, tp, hn);
-#pragma unroll
-        for (int t = 0; t < CL; t++)
-            if (t < len) wrow[s + t] = ch.d[t];
-    } else {
-#pragma unroll
-        for (int t = 0; t < CL; t++)
-            if (t < len) wrow[s + t] = (T)corrected<T, Q>(p, s + t, ch.d[t], tp, hn);
-    }
+    chunk_ends<T, Q, CL, false, TMIN>(d, len, r);
+    if (overlay) __syncthreads();
+    reduced_solve<Q, Q == 1>(p, buf, NT, Lt, k, li, r, tp, hn);
+    // every thread has finished reading the tile before the reduced solve's barrier
+    if (overlay) __syncthreads();
+    correct_padded<T, Q, CL, G>(d, Rows<double, CL, false>{p.rows64 + blk}, tp, hn, [&](int t, T v) {
+        if (t < TMIN || t < len) trow[xw_slot<CL>(s + t + M)] = v;
+    });
     __syncthreads();
 
-    for (int lj = 0; lj < Lt; lj++) {
-        const int64_t l = l0 + lj;
-        if (l >= nlines) break;
-        const int64_t off = (l % ny) * sy + (l / ny) * sz;
-        for (int i = tid; i < n; i += NT) epilogue<T, EPI>(e, off + i, (double)tile[lj * TS + i]);
+    Walk w{0, 0};
+    for (int e0 = 0; e0 < Lt * seg; e0 += 8) {
+        int64_t o[8];
+        T v[1][8];
+        bool ok[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int x = tid + w.q * NT, xc = x < n ? x : n - 1;
+            ok[i] = w.lj < left && x < n;
+            o[i] = line_off(w.lj) + xc;
+            v[0][i] = tile[(w.lj < Lt ? w.lj : 0) * TS + xw_slot<CL>(xc + M)];
+            next(w);
+        }
+        epilogue_rows<T, EPI, 8, 1, false>(e, o, v, ok);
     }
 }
 
@@ -1459,104 +1333,6 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
     }
 }
 
-template <int XC = XCL>
-__device__ __forceinline__ int xw_slot(int x) { return x + x / XC; }
-
-template <typename T> __device__ __forceinline__ const T *rowvp(const LineDev &p);
-template <> __device__ __forceinline__ const double *rowvp<double>(const LineDev &p) { return p.rowv64; }
-template <> __device__ __forceinline__ const float *rowvp<float>(const LineDev &p) { return p.rowv32; }
-
-// The zero-padded plan rows of one chunk: a block of its own read through
-// scalar loads (every chunk of the wave has the same rows) ...
-template <typename T, int CAP> struct RowsBlock {
-    const T *base;
-    __device__ __forceinline__ T operator()(int f, int t) const { return cload(base + f * CAP + t); }
-    template <typename D> __device__ __forceinline__ void fence(const D &) {}
-};
-// ... or per lane, with the rows of adjacent chunks in adjacent words
-template <typename T, int CAP> struct RowsLane {
-    const T *base;
-    int P;
-    __device__ __forceinline__ T operator()(int f, int t) const { return gload(base + (f * CAP + t) * P); }
-    template <typename D> __device__ __forceinline__ void fence(const D &dep)
-    {
-        asm volatile("" : "+v"(base) : "v"(dep));
-    }
-};
-
-// Chunk sweeps over all CL rows (rows past the chunk's length hold zeros and
-// multiply by zeros), the rows read G at a time as in solve_grouped.
-template <typename T, int Q, int CL, int G, typename Rows>
-__device__ __forceinline__ void solve_padded(T (&d)[CL], Rows R)
-{
-    constexpr int NG = CL / G;
-    constexpr int NL = Q, NU = Q == 1 ? 2 : 3;
-    const int fl[2] = {Q == 1 ? (int)R1_L : (int)R2_L1, (int)R2_L2};
-    const int fu[3] = {Q == 1 ? (int)R1_DINV : (int)R2_U0INV, Q == 1 ? (int)R1_C : (int)R2_U1, (int)R2_U2};
-    T c[NL][G], nx[NL][G];
-#pragma unroll
-    for (int f = 0; f < NL; f++)
-#pragma unroll
-        for (int i = 0; i < G; i++) c[f][i] = R(fl[f], i);
-#pragma unroll
-    for (int g = 0; g < NG; g++) {
-        if (g + 1 < NG) {
-            if (g > 0) R.fence(d[g * G - 1]);
-#pragma unroll
-            for (int f = 0; f < NL; f++)
-#pragma unroll
-                for (int i = 0; i < G; i++) nx[f][i] = R(fl[f], (g + 1) * G + i);
-        }
-#pragma unroll
-        for (int i = 0; i < G; i++) {
-            const int t = g * G + i;
-            if constexpr (Q == 1) {
-                if (t >= 1) d[t] = fma(-c[0][i], d[t - 1], d[t]);
-            } else {
-                if (t + 1 < CL) d[t + 1] = fma(-c[0][i], d[t], d[t + 1]);
-                if (t + 2 < CL) d[t + 2] = fma(-c[1][i], d[t], d[t + 2]);
-            }
-        }
-        if (g + 1 < NG) {
-#pragma unroll
-            for (int f = 0; f < NL; f++)
-#pragma unroll
-                for (int i = 0; i < G; i++) c[f][i] = nx[f][i];
-        }
-    }
-    T u[NU][G], nu[NU][G];
-    R.fence(d[CL - 1]);
-#pragma unroll
-    for (int f = 0; f < NU; f++)
-#pragma unroll
-        for (int i = 0; i < G; i++) u[f][i] = R(fu[f], (NG - 1) * G + i);
-#pragma unroll
-    for (int g = NG - 1; g >= 0; g--) {
-        if (g > 0) {
-            if (g < NG - 1) R.fence(d[(g + 1) * G]);
-#pragma unroll
-            for (int f = 0; f < NU; f++)
-#pragma unroll
-                for (int i = 0; i < G; i++) nu[f][i] = R(fu[f], (g - 1) * G + i);
-        }
-#pragma unroll
-        for (int i = G - 1; i >= 0; i--) {
-            const int t = g * G + i;
-            T acc = d[t];
-            if (t + 1 < CL) acc = fma(-u[1][i], d[t + 1 < CL ? t + 1 : t], acc);
-            if constexpr (Q == 2)
-                if (t + 2 < CL) acc = fma(-u[2][i], d[t + 2 < CL ? t + 2 : t], acc);
-            d[t] = acc * u[0][i];
-        }
-        if (g > 0) {
-#pragma unroll
-            for (int f = 0; f < NU; f++)
-#pragma unroll
-                for (int i = 0; i < G; i++) u[f][i] = nu[f][i];
-        }
-    }
-}
-
 // One wave per block, 64/P lines staged in LDS (a pad slot after every XC
 // points keeps the chunk-strided reads conflict-free), so global loads and
 // stores are contiguous.  XC is the chunk capacity (8 or 16).
@@ -1567,8 +1343,8 @@ __device__ __forceinline__ void solve_padded(T (&d)[CL], Rows R)
 // index is divided by the line length; WIDE (LPL = 64): one line at a time,
 // its offset in scalar registers.  The tile row holds the M halo points at both
 // ends (wrapped copies, or zeros at closed ends), so window reads need no wrap
-// test.  The row constants are zero-padded to XC rows (LineDev::rowu64, rowv64),
-// so the sweeps run without length tests.  UNIROW: periodic line of equal
+// test.  The row constants are zero-padded to XC rows (LineDev::rows64), so the
+// sweeps run without length tests.  UNIROW: periodic line of equal
 // chunks, whose factors, spikes and PCR blocks are those of chunk 0 (scalar
 // loads).  FULL: those chunks hold XC points, which fixes every LDS offset at
 // compile time.
@@ -1663,101 +1439,32 @@ __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restric
     T *trow = tile + li * TS;
     // slot of window point t (halo included), t = 0 .. XC + 2 M - 1
     auto slot = [&](int t) { return FULL ? k * (XC + 1) + t + t / XC : xw_slot<XC>(s + t); };
+    constexpr int TMIN = XC == 8 ? 1 : XC / 2;
     T d[XC];
     {
-        T fv[XC + 2 * M];
+        T fv[XC + 2 * M], fe[8];
 #pragma unroll
         for (int t = 0; t < XC + 2 * M; t++) fv[t] = trow[slot(t)];
-        const T *cf = coefp<T>(p);
-        T ci[M];
 #pragma unroll
-        for (int m = 0; m < M; m++) ci[m] = cload(cf + COEF_CI + m);
-        const T a0 = cload(cf + COEF_A0);
-        // rows past the chunk's length start and stay zero; a chunk holds more
-        // than half the capacity 16
-#pragma unroll
-        for (int t = 0; t < XC; t++) {
-            d[t] = rhs_row<T, M, SYM>(fv, t + M, ci, a0);
-            if (!FULL && t >= (XC > 8 ? XC / 2 : 1)) d[t] = t < len ? d[t] : T(0);
-        }
-        if (!UNIROW && p.closed) {
-#pragma unroll
-            for (int t = 0; t < NCMAX; t++) {
-                if (t >= p.nc) continue;
-                const T *cr = cf + COEF_CLO + t * 8;
-                T acc = cload(cr) * fv[M];
-#pragma unroll
-                for (int kap = 1; kap < 8; kap++) {
-                    // points past a line shorter than the stencil take a zero weight
-                    const T fk = kap < n ? fv[kap + M] : T(0);
-                    acc = fma(cload(cr + kap), fk, acc);
-                }
-                d[t] = k == 0 ? acc : d[t];
-            }
-            T fe[8];
-#pragma unroll
-            for (int kap = 0; kap < 8; kap++) fe[kap] = kap < n ? trow[xw_slot<XC>(n - 1 - kap + M)] : T(0);
-            // the last chunk holds m points (the longer ones come first)
-#pragma unroll
-            for (int t = 0; t < XC; t++) {
-                const int jr = p.m - 1 - t;
-                if (jr < 0 || jr >= p.nc) continue;
-                const T *cr = cf + COEF_CHI + jr * 8;
-                T acc = cload(cr) * fe[0];
-#pragma unroll
-                for (int kap = 1; kap < 8; kap++) acc = fma(cload(cr + kap), fe[kap], acc);
-                d[t] = k == P - 1 ? acc : d[t];
-            }
-        }
+        for (int kap = 0; kap < 8; kap++)
+            fe[kap] = !UNIROW && p.closed && kap < n ? trow[xw_slot<XC>(n - 1 - kap + M)] : T(0);
+        LineDev pr = p;
+        if constexpr (UNIROW) pr.closed = 0;   // periodic: no closure code
+        chunk_rhs<T, M, SYM, XC, FULL, true, TMIN>(pr, fv, fe, k == 0, k == P - 1, len, d);
     }
     // rows per group of per-lane loads: four where two groups of eight spill
     constexpr int G = !UNIROW && XC > 8 && (Q == 2 || sizeof(T) == 8) ? 4 : 8;
-    if constexpr (UNIROW) solve_padded<T, Q, XC, G>(d, RowsBlock<T, XC>{rowup<T>(p)});
-    else solve_padded<T, Q, XC, G>(d, RowsLane<T, XC>{rowvp<T>(p) + k, P});
+    const int blk = UNIROW ? cload(p.blk) : p.blk[k];
+    solve_padded<T, Q, XC, G>(d, Rows<T, XC, UNIROW>{rowsp<T>(p) + blk});
     double r[2 * Q], tp[Q], hn[Q];
-#pragma unroll
-    for (int i = 0; i < Q; i++) {
-        r[i] = (double)d[i];
-        T x = d[FULL ? XC - Q + i : 0];
-        if constexpr (!FULL) {
-#pragma unroll
-            for (int t = 1; t < XC; t++) x = t == len - Q + i ? d[t] : x;
-        }
-        r[Q + i] = (double)x;
-    }
+    chunk_ends<T, Q, XC, FULL, TMIN>(d, len, r);
     reduced_solve_wave<Q, !UNIROW && Q == 1 && sizeof(T) == 8, UNIROW>(p, k, UNIROW ? 0 : k, li * P, r, tp, hn);
     // spike correction; each result goes back to the tile (every window read
     // of the wave is done: the wave runs in step)
     __syncthreads();
-    auto correct = [&](auto R) {
-#pragma unroll
-        for (int g = 0; g < XC / G; g++) {
-            if (g > 0) R.fence(d[g * G - 1]);
-            double c[2 * Q][G];
-#pragma unroll
-            for (int i = 0; i < G; i++) {
-                c[0][i] = R(Q == 1 ? (int)R1_V : (int)R2_V0, g * G + i);
-                c[1][i] = R(Q == 1 ? (int)R1_W : (int)R2_W0, g * G + i);
-                if constexpr (Q == 2) {
-                    c[2][i] = R(R2_V1, g * G + i);
-                    c[3][i] = R(R2_W1, g * G + i);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < G; i++) {
-                const int t = g * G + i;
-                double acc = fma(c[1][i], hn[0], c[0][i] * tp[0]);
-                if constexpr (Q == 2) {
-                    acc = fma(c[2][i], tp[1], acc);
-                    acc = fma(c[3][i], hn[1], acc);
-                }
-                d[t] = (T)((double)d[t] - acc);
-                if (FULL || t < (XC > 8 ? XC / 2 : 1) || t < len) trow[slot(t + M)] = d[t];
-            }
-        }
-    };
-    if constexpr (UNIROW) correct(RowsBlock<double, XC>{p.rowu64});
-    else correct(RowsLane<double, XC>{p.rowv64 + k, P});
+    correct_padded<T, Q, XC, G>(d, Rows<double, XC, UNIROW>{p.rows64 + blk}, tp, hn, [&](int t, T v) {
+        if (FULL || t < TMIN || t < len) trow[slot(t + M)] = v;
+    });
     __syncthreads();
     Walk w{0, lsub};
 #pragma unroll
@@ -1777,12 +1484,12 @@ __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restric
     }
 }
 
-// x sweep for lines of exactly 16 P points in equal 16-point chunks (the
-// production grids): the same algorithm as k_line_xw with the line length,
+// x sweep for periodic lines of exactly 16 P points in equal 16-point chunks
+// (the production grids): the same algorithm as k_line_xw with the line length,
 // chunk length, lines per wave (NL = 64 / P) and the element-to-line map fixed
-// at compile time, line offsets computed once per wave, a mask for the
-// periodic wrap, and no closure code on periodic lines.
-template <typename T, int Q, int M, int SYM, int EPI, int NL, bool PER>
+// at compile time, line offsets computed once per wave and a mask for the
+// periodic wrap.
+template <typename T, int Q, int M, int SYM, int EPI, int NL>
 __global__ void __launch_bounds__(64) k_line_xwf(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz, int ny,
                                                  int64_t nlines, EpiArgs e, LineFields mf)
 {
@@ -1811,7 +1518,7 @@ __global__ void __launch_bounds__(64) k_line_xwf(LineDev p, const T *__restrict_
 #pragma unroll
         for (int lj = 0; lj < NL; lj++)
 #pragma unroll
-            for (int q = 0; q < EPL; q++) tile[lj * TS + xw_slot(lane + 64 * q)] = tmp[lj * EPL + q];
+            for (int q = 0; q < EPL; q++) tile[lj * TS + xw_slot<XCL>(lane + 64 * q)] = tmp[lj * EPL + q];
     }
     __syncthreads();
     const int li = lane / P, k = lane % P;
@@ -1820,40 +1527,26 @@ __global__ void __launch_bounds__(64) k_line_xwf(LineDev p, const T *__restrict_
     T fv[XCL + 2 * M];
 #pragma unroll
     for (int t = -M; t < XCL + M; t++) {
-        int r = s + t;
-        if constexpr (PER) {
-            fv[t + M] = trow[xw_slot(r & (N - 1))];
-        } else {
-            fv[t + M] = (r >= 0 && r < N) ? trow[xw_slot(r < 0 ? 0 : (r >= N ? N - 1 : r))] : T(0);
-        }
+        fv[t + M] = trow[xw_slot<XCL>((s + t) & (N - 1))];
     }
-    T fe[8];
-#pragma unroll
-    for (int kap = 0; kap < 8; kap++) fe[kap] = PER ? T(0) : trow[xw_slot(N - 1 - kap)];
-    Chunk<T, Q, M, SYM, XCL> ch;
-    if constexpr (PER) {
+    T d[XCL];
+    {
         const T *cf = coefp<T>(p);
         T ci[M];
 #pragma unroll
-        for (int m = 0; m < M; m++) ci[m] = cf[COEF_CI + m];
-        const T a0 = cf[COEF_A0];
+        for (int m = 0; m < M; m++) ci[m] = cload(cf + COEF_CI + m);
+        const T a0 = cload(cf + COEF_A0);
 #pragma unroll
-        for (int t = 0; t < XCL; t++) ch.d[t] = rhs_row<T, M, SYM>(fv, t + M, ci, a0);
-    } else {
-        ch.rhs(p, k, XCL, fv, fe);
+        for (int t = 0; t < XCL; t++) d[t] = rhs_row<T, M, SYM>(fv, t + M, ci, a0);
     }
-    const int rs = PER ? 0 : s;
-    const int kc = PER ? 0 : k;
-    ch.solve(p, rs, XCL);
+    const int blk = cload(p.blk);
+    solve_padded<T, Q, XCL, 8>(d, Rows<T, XCL, true>{rowsp<T>(p) + blk});
     double r[2 * Q], tp[Q], hn[Q];
-    ch.ends(XCL, r);
-    reduced_solve_wave<Q>(p, k, kc, li * P, r, tp, hn);
-    T res[XCL];
-#pragma unroll
-    for (int t = 0; t < XCL; t++) res[t] = (T)corrected<T, Q>(p, rs + t, ch.d[t], tp, hn);
+    chunk_ends<T, Q, XCL, true, XCL>(d, XCL, r);
+    reduced_solve_wave<Q, false, true>(p, k, 0, li * P, r, tp, hn);
     __syncthreads();   // all window reads done before the tile is overwritten
-#pragma unroll
-    for (int t = 0; t < XCL; t++) trow[xw_slot(s + t)] = res[t];
+    correct_padded<T, Q, XCL, 8>(d, Rows<double, XCL, true>{p.rows64 + blk}, tp, hn,
+                                 [&](int t, T v) { trow[xw_slot<XCL>(s + t)] = v; });
     __syncthreads();
 #pragma unroll
     for (int lj = 0; lj < NL; lj++) {
@@ -1869,7 +1562,7 @@ __global__ void __launch_bounds__(64) k_line_xwf(LineDev p, const T *__restrict_
                 const int x = lane + 64 * (q < EPL ? q : 0);
                 ok[i] = in;
                 o[i] = loff[lj] + x;
-                v[i] = tile[lj * TS + xw_slot(x)];
+                v[i] = tile[lj * TS + xw_slot<XCL>(x)];
             }
             epilogue_batch<T, EPI, 8>(e, o, v, ok);
         }
@@ -1910,17 +1603,13 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
     const int B = 2 * Q;
     const size_t lim = lds_limit();
     const int maxNT = Q == 1 ? 1024 : 512;
-    if (dim == 1 && p.extra == 0 && p.m == XCL && P == 16 && (p.periodic || p.closed)) {
+    if (dim == 1 && p.extra == 0 && p.m == XCL && P == 16 && p.periodic) {
         // 256-point lines: four per wave
         const int64_t nlines = v.n[1] * v.n[2];
         const int64_t nblk = (nlines + 3) / 4;
-        if (p.periodic)
-            hipLaunchKernelGGL((k_line_xwf<T, Q, M, SYM, EPI, 4, true>), dim3((unsigned)nblk, nf), dim3(64), 0, st, p, f,
-                               v.s[1], v.s[2], (int)v.n[1], nlines, e, mf);
-        else
-            hipLaunchKernelGGL((k_line_xwf<T, Q, M, SYM, EPI, 4, false>), dim3((unsigned)nblk, nf), dim3(64), 0, st, p, f,
-                               v.s[1], v.s[2], (int)v.n[1], nlines, e, mf);
-    } else if (dim == 1 && P <= 64 && p.m + (p.extra ? 1 : 0) <= XCL) {
+        hipLaunchKernelGGL((k_line_xwf<T, Q, M, SYM, EPI, 4>), dim3((unsigned)nblk, nf), dim3(64), 0, st, p, f,
+                           v.s[1], v.s[2], (int)v.n[1], nlines, e, mf);
+    } else if (dim == 1 && P <= 64 && p.cap <= XCL) {
         const int64_t nlines = v.n[1] * v.n[2];
         const int nl = 64 / P;
         const int64_t nblk = (nlines + nl - 1) / nl;
@@ -1945,40 +1634,33 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         if (p.cap == 8) pick(std::integral_constant<int, 8>{});
         else pick(std::integral_constant<int, XCL>{});
     } else if (dim == 1) {
-        const size_t tile_row = (size_t)(p.n + 1) * sizeof(T);
         const int64_t nlines = v.n[1] * v.n[2];
-        auto shm_of = [&](int Lt) {
-            return (((size_t)Lt * tile_row + 7) / 8) * 8 + (size_t)2 * B * Lt * P * sizeof(double);
+        const int y = p.n + 2 * M + p.cap;
+        const int TS = y + y / p.cap + 1;
+        auto shm_of = [&](int Lt, bool over = false) {
+            const size_t tile = (((size_t)Lt * TS * sizeof(T) + 7) / 8) * 8;
+            const size_t bufs = (size_t)2 * B * Lt * P * sizeof(double);
+            return over ? std::max(tile, bufs) : tile + bufs;
         };
-        if (64 * P <= maxNT && shm_of(64) <= lim && nlines >= 64) {
-            const int Lt = 64, NT = 64 * P;
-            const size_t shm = shm_of(Lt);
-            auto kern = k_line_x<T, Q, M, SYM, EPI, true>;
+        int Lt = 1;
+        while (Lt * 2 * P <= 512 && shm_of(Lt * 2) <= 48 * 1024 && Lt < 32) Lt *= 2;
+        const bool overlay = shm_of(Lt) > lim;
+        if (Lt * P > 512 || shm_of(Lt, overlay) > lim)
+            throw Error{CLES_ERR_UNSUPPORTED, "line too long for the x-sweep kernel"};
+        const int NT = Lt * P;
+        const size_t shm = shm_of(Lt, overlay);
+        const int64_t nblk = (nlines + Lt - 1) / Lt;
+        auto go = [&](auto kern) {
             allow_lds(kern, shm);
-            const int64_t nblk = (nlines + Lt - 1) / Lt;
             hipLaunchKernelGGL(kern, dim3((unsigned)nblk, nf), dim3(NT), shm, st, p, f, v.s[1], v.s[2], (int)v.n[1],
-                               nlines, Lt, e, mf);
-        } else {
-            int Lt = 1;
-            while (Lt * 2 * P <= 512 && shm_of(Lt * 2) <= 48 * 1024 && Lt < 32) Lt *= 2;
-            if (Lt * P > 512 || shm_of(Lt) > lim)
-                throw Error{CLES_ERR_UNSUPPORTED, "line too long for the x-sweep kernel"};
-            const int NT = Lt * P;
-            const size_t shm = shm_of(Lt);
-            const int64_t nblk = (nlines + Lt - 1) / Lt;
-            const int cl = p.m + (p.extra ? 1 : 0);
-            auto go = [&](auto kern) {
-                allow_lds(kern, shm);
-                hipLaunchKernelGGL(kern, dim3((unsigned)nblk, nf), dim3(NT), shm, st, p, f, v.s[1], v.s[2],
-                                   (int)v.n[1], nlines, Lt, e, mf);
-            };
-            if (cl <= 8)
-                go(k_line_x<T, Q, M, SYM, EPI, false, 8>);
-            else if (cl <= 16)
-                go(k_line_x<T, Q, M, SYM, EPI, false, 16>);
-            else
-                go(k_line_x<T, Q, M, SYM, EPI, false, MC>);
-        }
+                               nlines, Lt, TS, overlay, e, mf);
+        };
+        if (p.cap == 8)
+            go(k_line_x<T, Q, M, SYM, EPI, 8>);
+        else if (p.cap == 16)
+            go(k_line_x<T, Q, M, SYM, EPI, 16>);
+        else
+            go(k_line_x<T, Q, M, SYM, EPI, MC>);
     } else {
         const int64_t nlane = v.n[0];
         const int64_t sd = dim == 2 ? v.s[1] : v.s[2];
@@ -2040,11 +1722,10 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             const int NT = Lx * P;
             const int nxb = (int)((nlane + Lx - 1) / Lx);
             const size_t shm = (size_t)2 * B * NT * sizeof(double);
-            const int cl = p.m + (p.extra ? 1 : 0);
-            if (cl <= 8)
+            if (p.cap == 8)
                 hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 8>), dim3((unsigned)(nxb * nouter), nf),
                                    dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
-            else if (cl <= 16)
+            else if (p.cap == 16)
                 hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 16>), dim3((unsigned)(nxb * nouter), nf),
                                    dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
             else

@@ -14,43 +14,32 @@
 
 namespace cles {
 
-// a pad slot after every CL points (the chunk capacity) spreads the
-// chunk-strided reads over the banks
-template <int CL>
-__device__ __forceinline__ int rag_slot(int x) { return x + x / CL; }
-
 // Blocks are dispatched round-robin over the 8 XCDs; renumbering them so that
 // each XCD takes one contiguous range keeps the nf blocks of one work item
-// (same lines and tables, different fields) on one XCD's L2.
+// (same lines, different fields) on one XCD's L2.
 __device__ __forceinline__ unsigned rag_block(unsigned b, unsigned nb)
 {
     const unsigned nfull = nb & ~7u;
     return b < nfull ? (b & 7u) * (nfull >> 3) + (b >> 3) : b;
 }
 
-template <typename T> __device__ __forceinline__ const T *rowtp(const LineDev &p);
-template <> __device__ __forceinline__ const double *rowtp<double>(const LineDev &p) { return p.rowt64; }
-template <> __device__ __forceinline__ const float *rowtp<float>(const LineDev &p) { return p.rowt32; }
-
-// The chunk-major plan rows of chunk k (RAG_MAX_CHUNK zero-padded rows per
-// chunk, so every t < RAG_MAX_CHUNK is in bounds): the P lanes of a line read
-// consecutive words for each (field, t).
-template <typename T>
-struct RowsRag {
-    const T *base;
-    int P;
-    __device__ __forceinline__ T operator()(int f, int t) const
-    {
-        return gload(base + ((size_t)f * RAG_MAX_CHUNK + t) * P);
-    }
-    template <typename D> __device__ __forceinline__ void fence(const D &dep)
-    {
-        asm volatile("" : "+v"(base) : "v"(dep));
-    }
-};
+// Tile row of a line of at most CL P points with its halo, a pad slot after
+// every CL points (xw_slot) and room for the last chunk's window overrun.
+template <int CL, int M> __host__ __device__ constexpr int rag_row(int P)
+{
+    return (CL * P + 2 * M + CL) + (CL * P + 2 * M + CL) / CL + 1;
+}
 
 // CL: chunk capacity of the launch's items (RAG_SHORT_CHUNK for the short
-// class, RAG_MAX_CHUNK otherwise); the plan rows keep RAG_MAX_CHUNK per chunk.
+// class, RAG_MAX_CHUNK otherwise).
+//
+// Bound: the latency of one wave's chain (a few thousand lines fill the chip
+// less than twice over), so what is waited for counts: the row constants of
+// all instances share one pool of distinct chunk blocks (LineDev::rows64), a
+// few KB that stay in the nearest cache instead of 40 bytes of tables per
+// point; each tile row carries the halo points, so window reads have no wrap
+// tests; the sweeps run on zero-padded rows.  96 steps of 512 tubes and their
+// states FP64, tables per instance / shared: 163.8 / 133.5 ms.
 template <typename T, int Q, int M, int SYM, int EPI, int CL>
 __global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict__ f, EpiArgs e)
 {
@@ -63,13 +52,14 @@ __global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict
     f += fo;
     if constexpr (EPI == EPI_ART_MULTI) e = e.multi[fld];   // its own outputs: no field offset
     const int *it = r.items + 3 * item;
-    const int P = it[0], start = it[1], count = it[2];
-    const int TS = (CL + 1) * P;   // rag_slot<CL>(CL P - 1) < (CL + 1) P
+    const int P = cload(it), start = cload(it + 1), count = cload(it + 2);
+    const int TS = rag_row<CL, M>(P);
 
     // stage the item's lines
     for (int lj = 0; lj < count; lj++) {
-        const int inst = r.order[start + lj];
+        const int inst = cload(r.order + start + lj);
         const int n = r.plans[inst].n;
+        const bool per = r.plans[inst].periodic;
         const T *src = f + r.off[inst];
         T *row = tile + lj * TS;
         // a line of up to 64 CL points in one round of CL loads per lane (the
@@ -84,8 +74,12 @@ __global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict
 #pragma unroll
             for (int i = 0; i < CL; i++) {
                 const int x = x0 + lane + 64 * i;
-                if (x < n) row[rag_slot<CL>(x)] = v[i];
+                if (x < n) row[xw_slot<CL>(x + M)] = v[i];
             }
+        }
+        if (lane < 2 * M) {   // the halo: wrapped copies, or zeros
+            const T v = per ? src[lane < M ? n - M + lane : lane - M] : T(0);
+            row[xw_slot<CL>(lane < M ? lane : lane + n)] = v;
         }
     }
     __syncthreads();
@@ -99,42 +93,30 @@ __global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict
     const int s = k * p.m + min(k, p.extra);
     const int len = p.m + (k < p.extra ? 1 : 0);
     T *trow = tile + (live ? li : 0) * TS;
-    T fv[CL + 2 * M];
+    constexpr int TMIN = 1;   // a line may be one chunk of a few points
+    T d[CL];
+    {
+        T fv[CL + 2 * M], fe[8];
 #pragma unroll
-    for (int t = -M; t < CL + M; t++) {
-        T val = T(0);
-        if (t < len + M) {
-            int rr = s + t;
-            bool ok = true;
-            if (rr < 0) {
-                if (p.periodic) rr += n; else ok = false;
-            } else if (rr >= n) {
-                if (p.periodic) rr -= n; else ok = false;
-            }
-            if (ok) val = trow[rag_slot<CL>(rr)];
-        }
-        fv[t + M] = val;
+        for (int t = 0; t < CL + 2 * M; t++) fv[t] = trow[xw_slot<CL>(s + t)];
+#pragma unroll
+        for (int kap = 0; kap < 8; kap++)
+            fe[kap] = (p.closed && kap < n) ? trow[xw_slot<CL>(n - 1 - kap + M)] : T(0);
+        chunk_rhs<T, M, SYM, CL, false, false, TMIN>(p, fv, fe, k == 0, k == P - 1, len, d);
     }
-    T fe[8];
-#pragma unroll
-    for (int kap = 0; kap < 8; kap++) fe[kap] = (p.closed && kap < n) ? trow[rag_slot<CL>(n - 1 - kap)] : T(0);
-    Chunk<T, Q, M, SYM, CL> ch;
-    ch.rhs(p, k, len, fv, fe);
-    solve_grouped<T, Q, CL, 8>(ch.d, len, RowsRag<T>{rowtp<T>(p) + k, p.P});
+    const int blk = p.blk[k];
+    solve_padded<T, Q, CL, 8>(d, Rows<T, CL, false>{rowsp<T>(p) + blk});
     double ends[2 * Q], tp[Q], hn[Q];
-    ch.ends(len, ends);
+    chunk_ends<T, Q, CL, false, TMIN>(d, len, ends);
     reduced_solve_wave<Q, Q == 1>(p, k, k, li * P, ends, tp, hn);
-    correct_grouped<T, Q, CL, 8>(ch.d, len, RowsRag<double>{p.rowt64 + k, p.P}, tp, hn);
     __syncthreads();   // every window read is done before the tile is overwritten
-    if (live) {
-#pragma unroll
-        for (int t = 0; t < CL; t++)
-            if (t < len) trow[rag_slot<CL>(s + t)] = ch.d[t];
-    }
+    correct_padded<T, Q, CL, 8>(d, Rows<double, CL, false>{p.rows64 + blk}, tp, hn, [&](int t, T v) {
+        if (live && t < len) trow[xw_slot<CL>(s + t + M)] = v;
+    });
     __syncthreads();
 
     for (int lj = 0; lj < count; lj++) {
-        const int ij = r.order[start + lj];
+        const int ij = cload(r.order + start + lj);
         if (r.mask && !r.mask[ij]) continue;
         const int nj = r.plans[ij].n;
         const int64_t oj = r.off[ij];
@@ -151,16 +133,16 @@ __global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict
         constexpr int NB = CL > 16 ? 16 : 8;
         for (int x0 = 0; x0 < nj; x0 += 64 * NB) {
             int64_t o[NB];
-            T v[NB];
+            T v[1][NB];
             bool ok[NB];
 #pragma unroll
             for (int i = 0; i < NB; i++) {
                 const int x = x0 + lane + 64 * i;
                 ok[i] = x < nj;
                 o[i] = oj + (ok[i] ? x : 0);
-                v[i] = ok[i] ? row[rag_slot<CL>(x)] : T(0);
+                v[0][i] = row[xw_slot<CL>((ok[i] ? x : 0) + M)];
             }
-            epilogue_batch<T, EPI, NB>(ej, o, v, ok);
+            epilogue_rows<T, EPI, NB, 1, false>(ej, o, v, ok);
         }
     }
 }
@@ -181,14 +163,14 @@ void launch_rag_variant(const RagLines &r, const T *f, const EpiArgs &e, hipStre
     rl.items = r.items + 3 * r.nshort;
     rl.nitems = r.nitems - r.nshort;
     if (rs.nitems > 0) {
-        const size_t shm = (size_t)64 * (RAG_SHORT_CHUNK + 1) * sizeof(T);
+        const size_t shm = (size_t)(64 / r.pmin[0]) * rag_row<RAG_SHORT_CHUNK, M>(r.pmin[0]) * sizeof(T);
         const int64_t nb = (int64_t)rs.nitems * r.nf;
         hipLaunchKernelGGL((k_line_rag<T, Q, M, SYM, EPI, RAG_SHORT_CHUNK>), dim3((unsigned)nb), dim3(64), shm, st, rs, f,
                            e);
         CLES_HIP(hipGetLastError());
     }
     if (rl.nitems > 0) {
-        const size_t shm = (size_t)64 * (RAG_MAX_CHUNK + 1) * sizeof(T);
+        const size_t shm = (size_t)(64 / r.pmin[1]) * rag_row<RAG_MAX_CHUNK, M>(r.pmin[1]) * sizeof(T);
         const int64_t nb = (int64_t)rl.nitems * r.nf;
         hipLaunchKernelGGL((k_line_rag<T, Q, M, SYM, EPI, RAG_MAX_CHUNK>), dim3((unsigned)nb), dim3(64), shm, st, rl, f,
                            e);

@@ -163,7 +163,7 @@ void chunk_solve(const ChunkFactor &F, std::vector<double> &x)
 }  // namespace
 
 void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int periodic, double h, int max_chunk,
-                       int dim, bool chunk_major, int lo_fold, int hi_fold)
+                       int dim, RowPool *pool, int lo_fold, int hi_fold)
 {
     const int q = s.q, M = s.M, nc = s.nclosure;
     if (q < 1 || q > 2) throw Error{CLES_ERR_UNSUPPORTED, "scheme LHS half-bandwidth q must be 1 or 2"};
@@ -406,74 +406,50 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
         }
     }
 
-    // chunk-major copy of the row constants for the ragged kernel
-    std::vector<double> rowt;
-    if (chunk_major) {
-        if (max_chunk > RAG_MAX_CHUNK) throw Error{CLES_ERR_INVALID, "chunk-major tables hold chunks of at most 32 points"};
-        rowt.assign((size_t)nrow * RAG_MAX_CHUNK * P, 0.0);
-        for (int f = 0; f < nrow; f++)
-            for (int k = 0; k < P; k++)
-                for (int t = 0; t < clen(k); t++)
-                    rowt[((size_t)f * RAG_MAX_CHUNK + t) * P + k] = row[(size_t)f * n + cstart(k) + t];
-    }
-
-    // per-chunk blocks padded to the kernels' capacity (LineDev::rowu64); the
-    // ragged plans do not use them
+    // the distinct chunk blocks, padded to the kernels' capacity
     const int longest = m + (extra ? 1 : 0);
-    const int cap = longest <= 8 ? 8 : longest <= 16 ? 16 : 32;
-    std::vector<double> rowu, rowv;
-    if (!chunk_major) {
-        rowu.assign((size_t)P * nrow * cap, 0.0);
-        rowv.assign((size_t)P * nrow * cap, 0.0);
-        for (int k = 0; k < P; k++)
-            for (int f = 0; f < nrow; f++)
-                for (int t = 0; t < clen(k); t++) {
-                    if (q == 1 && f == R1_C && t == clen(k) - 1) continue;
-                    const double c = row[(size_t)f * n + cstart(k) + t];
-                    rowu[((size_t)k * nrow + f) * cap + t] = c;
-                    rowv[((size_t)f * cap + t) * P + k] = c;
-                }
+    const int cap = longest <= 8 && !pool ? 8 : longest <= 16 ? 16 : 32;
+    if (longest > cap) throw Error{CLES_ERR_INVALID, "chunks of more than 32 points"};
+    RowPool own;
+    RowPool &rp = pool ? *pool : own;
+    std::vector<int> blk(P);
+    std::vector<double> block((size_t)nrow * cap);
+    for (int k = 0; k < P; k++) {
+        std::fill(block.begin(), block.end(), 0.0);
+        for (int f = 0; f < nrow; f++)
+            for (int t = 0; t < clen(k); t++)
+                if (!(q == 1 && f == R1_C && t == clen(k) - 1))
+                    block[(size_t)f * cap + t] = row[(size_t)f * n + cstart(k) + t];
+        const std::string key((const char *)block.data(), block.size() * sizeof(double));
+        auto it = rp.at.find(key);
+        if (it == rp.at.end()) {
+            it = rp.at.emplace(key, (int)rp.rows.size()).first;
+            rp.rows.insert(rp.rows.end(), block.begin(), block.end());
+        }
+        blk[k] = it->second;
     }
 
-    // host image: coef64 | coef32 | row64 | row32 | pcr | rowu64 | rowu32 | rowv64 | rowv32 | rowt64 | rowt32
-    // (256-byte aligned parts)
-    size_t b_coef64 = COEF_N * sizeof(double), b_coef32 = COEF_N * sizeof(float);
-    size_t b_row64 = row.size() * sizeof(double), b_row32 = row.size() * sizeof(float);
-    size_t b_pcr = pcr.size() * sizeof(double);
-    size_t b_rowt64 = rowt.size() * sizeof(double), b_rowt32 = rowt.size() * sizeof(float);
+    // host image: coef64 | coef32 | pcr | blk | rows64 | rows32 (256-byte aligned parts)
+    const size_t b_coef64 = COEF_N * sizeof(double), b_coef32 = COEF_N * sizeof(float);
+    const size_t b_pcr = pcr.size() * sizeof(double), b_blk = blk.size() * sizeof(int);
+    const size_t b_rows64 = own.rows.size() * sizeof(double), b_rows32 = own.rows.size() * sizeof(float);
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     out.o_coef32 = al(b_coef64);
-    out.o_row64 = out.o_coef32 + al(b_coef32);
-    out.o_row32 = out.o_row64 + al(b_row64);
-    out.o_pcr = out.o_row32 + al(b_row32);
-    const size_t b_rowu64 = rowu.size() * sizeof(double), b_rowu32 = rowu.size() * sizeof(float);
-    out.o_rowu64 = out.o_pcr + al(std::max<size_t>(b_pcr, 8));
-    out.o_rowu32 = out.o_rowu64 + al(b_rowu64);
-    out.o_rowv64 = out.o_rowu32 + al(b_rowu32);
-    out.o_rowv32 = out.o_rowv64 + al(b_rowu64);
-    out.o_rowt64 = out.o_rowv32 + al(b_rowu32);
-    out.o_rowt32 = out.o_rowt64 + al(b_rowt64);
-    const size_t total = out.o_rowt32 + al(b_rowt32);
-    out.image.assign(total, 0);
-    if (!rowu.empty()) {
-        std::vector<float> rowu32(rowu.begin(), rowu.end());
-        std::memcpy(out.image.data() + out.o_rowu64, rowu.data(), b_rowu64);
-        std::memcpy(out.image.data() + out.o_rowu32, rowu32.data(), b_rowu32);
-        std::vector<float> rowv32(rowv.begin(), rowv.end());
-        std::memcpy(out.image.data() + out.o_rowv64, rowv.data(), b_rowu64);
-        std::memcpy(out.image.data() + out.o_rowv32, rowv32.data(), b_rowu32);
-    }
-    if (!rowt.empty()) {
-        std::vector<float> rowt32(rowt.begin(), rowt.end());
-        std::memcpy(out.image.data() + out.o_rowt64, rowt.data(), b_rowt64);
-        std::memcpy(out.image.data() + out.o_rowt32, rowt32.data(), b_rowt32);
-    }
-    std::memcpy(out.image.data(), coef.data(), b_coef64);
-    std::vector<float> coef32(coef.begin(), coef.end()), row32(row.begin(), row.end());
-    std::memcpy(out.image.data() + out.o_coef32, coef32.data(), b_coef32);
-    std::memcpy(out.image.data() + out.o_row64, row.data(), b_row64);
-    std::memcpy(out.image.data() + out.o_row32, row32.data(), b_row32);
-    if (b_pcr) std::memcpy(out.image.data() + out.o_pcr, pcr.data(), b_pcr);
+    out.o_pcr = out.o_coef32 + al(b_coef32);
+    out.o_blk = out.o_pcr + al(std::max<size_t>(b_pcr, 8));
+    out.o_rows64 = out.o_blk + al(b_blk);
+    out.o_rows32 = out.o_rows64 + al(b_rows64);
+    out.image.assign(out.o_rows32 + al(b_rows32), 0);
+    const std::vector<float> coef32(coef.begin(), coef.end()), rows32(own.rows.begin(), own.rows.end());
+    auto put = [&](size_t o, const void *src, size_t bytes) {
+        if (bytes) std::memcpy(out.image.data() + o, src, bytes);
+    };
+    put(0, coef.data(), b_coef64);
+    put(out.o_coef32, coef32.data(), b_coef32);
+    put(out.o_pcr, pcr.data(), b_pcr);
+    put(out.o_blk, blk.data(), b_blk);
+    put(out.o_rows64, own.rows.data(), b_rows64);
+    put(out.o_rows32, rows32.data(), b_rows32);
     LineDev &L0 = out.dev;
     L0 = LineDev{};
     L0.n = n; L0.q = q; L0.M = M; L0.sym = s.symmetric ? 1 : 0; L0.nc = closed ? nc : 0;
@@ -487,22 +463,17 @@ void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base)
     dev = t.dev;
     dev.coef64 = (const double *)base;
     dev.coef32 = (const float *)(base + t.o_coef32);
-    dev.row64 = (const double *)(base + t.o_row64);
-    dev.row32 = (const float *)(base + t.o_row32);
     dev.pcr = (const double *)(base + t.o_pcr);
-    dev.rowu64 = (const double *)(base + t.o_rowu64);
-    dev.rowu32 = (const float *)(base + t.o_rowu32);
-    dev.rowv64 = (const double *)(base + t.o_rowv64);
-    dev.rowv32 = (const float *)(base + t.o_rowv32);
-    dev.rowt64 = t.o_rowt64 != t.o_rowt32 ? (const double *)(base + t.o_rowt64) : nullptr;
-    dev.rowt32 = t.o_rowt64 != t.o_rowt32 ? (const float *)(base + t.o_rowt32) : nullptr;
+    dev.blk = (const int *)(base + t.o_blk);
+    dev.rows64 = (const double *)(base + t.o_rows64);
+    dev.rows32 = (const float *)(base + t.o_rows32);
 }
 
 void build_line_plan(HostPlan &hp, const cles_scheme_desc &s, int n, int periodic, double h, int max_chunk,
                      int lo_fold, int hi_fold)
 {
     LineTables t;
-    build_line_tables(t, s, n, periodic, h, max_chunk, hp.dim, false, lo_fold, hi_fold);
+    build_line_tables(t, s, n, periodic, h, max_chunk, hp.dim, nullptr, lo_fold, hi_fold);
     void *d = nullptr;
     CLES_HIP(hipMalloc(&d, t.image.size()));
     hipError_t e = hipMemcpy(d, t.image.data(), t.image.size(), hipMemcpyHostToDevice);

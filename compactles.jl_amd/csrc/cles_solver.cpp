@@ -1292,10 +1292,10 @@ int cles_solver_footprint(const cles_solver_desc *desc, size_t *bytes)
             N *= (double)d.n_global[k];
             if (d.n_global[k] > 1) {
                 nact++;
-                // three line plans at most per dimension: row tables (<= 9 values of 8 + 4
-                // bytes per node, and two padded copies of the chunk blocks, each
-                // at most twice that), PCR blocks and 256-byte-aligned parts
-                plans += 3.0 * ((double)d.n_global[k] * 12.0 * 60.0 + 64.0 * 1024.0);
+                // three line plans at most per dimension: chunk blocks (at most one per
+                // chunk: <= 9 values of 8 + 4 bytes per row, rows padded to at most twice
+                // the points), PCR blocks and 256-byte-aligned parts
+                plans += 3.0 * ((double)d.n_global[k] * 12.0 * 20.0 + 64.0 * 1024.0);
                 for (int sd = 0; sd < 2; sd++)
                     nscbc = nscbc || d.bc[k][sd] == CLES_BC_NSCBC_IN || d.bc[k][sd] == CLES_BC_NSCBC_OUT;
             }

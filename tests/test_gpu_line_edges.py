@@ -64,3 +64,37 @@ def test_wave_local_x(ctx, dtype, bar, periodic, line):  # noqa: F811
             ref = _oracle_apply(name, 1, n, periodic, 0.1, f)
             got = _gpu_apply(ctx, name, 1, n, periodic, 0.1, f, dtype=dtype, padded=padded)
             assert Hh.relerr(got, ref) <= bar, (name, n)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("line", [1025, 1100, 2048, 4000])
+def test_block_x(ctx, dtype, bar, periodic, line):  # noqa: F811
+    """The block-wide x sweep: lines of more than 64 chunks, whole and uneven
+    chunks, blocks with missing lines, padded and unpadded rows."""
+    for name in ("lele_d1_6", "lele_d1_10", "compact_filter"):
+        for ny, nz, padded in ((5, 3, True), (1, 1, False), (3, 1, False)):
+            n = (line, ny, nz)
+            f = Hh.random_field(n, seed=51)
+            if dtype == np.float32:
+                f = f.astype(np.float32).astype(np.float64)
+            ref = _oracle_apply(name, 1, n, periodic, 0.1, f)
+            got = _gpu_apply(ctx, name, 1, n, periodic, 0.1, f, dtype=dtype, padded=padded)
+            assert Hh.relerr(got, ref) <= bar, (name, n)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("lanes,line", [(1, 40), (3, 9), (8, 16), (17, 33), (47, 64), (47, 100), (20, 700), (64, 600)])
+def test_narrow_yz(ctx, dtype, bar, periodic, lanes, line):  # noqa: F811
+    """The narrow-block y / z sweeps: few lanes, or more chunks than 64 lanes
+    leave room for; every chunk capacity, whole and uneven chunks."""
+    for name in ("lele_d1_6", "lele_d1_10", "compact_filter"):
+        for dim in (2, 3):
+            n = (lanes, line, 3) if dim == 2 else (lanes, 2, line)
+            f = Hh.random_field(n, seed=61)
+            if dtype == np.float32:
+                f = f.astype(np.float32).astype(np.float64)
+            ref = _oracle_apply(name, dim, n, periodic, 0.1, f)
+            got = _gpu_apply(ctx, name, dim, n, periodic, 0.1, f, dtype=dtype)
+            assert Hh.relerr(got, ref) <= bar, (name, dim, n)
