@@ -176,6 +176,7 @@ void build_plan_set(PlanSet &ps, std::vector<unsigned char> &blob, const cles_sc
             d.coef64 = (const double *)(uintptr_t)(base);
             d.coef32 = (const float *)(uintptr_t)(base + t.o_coef32);
             d.pcr = (const double *)(uintptr_t)(base + t.o_pcr);
+            d.pidx = (const int *)(uintptr_t)(base + t.o_pidx);
             d.blk = (const int *)(uintptr_t)(base + t.o_blk);
             it = cache.emplace(key, std::make_pair(d, base)).first;
         }
@@ -229,6 +230,7 @@ void rebase(std::vector<LineDev> &v, unsigned char *base)
         d.coef64 = (const double *)(base + (uintptr_t)d.coef64);
         d.coef32 = (const float *)(base + (uintptr_t)d.coef32);
         d.pcr = (const double *)(base + (uintptr_t)d.pcr);
+        d.pidx = (const int *)(base + (uintptr_t)d.pidx);
         d.blk = (const int *)(base + (uintptr_t)d.blk);
         d.rows64 = (const double *)(base + (uintptr_t)d.rows64);
         d.rows32 = (const float *)(base + (uintptr_t)d.rows32);

@@ -70,8 +70,10 @@ struct LineDev {
     int extra;      // first `extra` chunks have length m + 1
     const double *coef64;  // [0..8) ci, [8] a0, [16..80) clo[8][8], [80..144) chi[8][8]
     const float *coef32;
-    const double *pcr;     // per step s, chunk k: alpha, beta (B*B each, row-major);
-                           // then per chunk the final inverse block
+    const double *pcr;     // the distinct coefficient blocks: alpha, beta (B*B each, row-major) of a
+                           // step, or a final inverse block
+    const int *pidx;       // [s * P + k]: offset in pcr of chunk k's block of step s < nsteps, and of
+                           // its final block (s = nsteps)
     int cap;               // chunk capacity of the kernels: 8, 16 or 32 >= the longest chunk (ragged: 16 or 32)
     // Row constants: one block [field * cap + t] per distinct chunk, rows past
     // the chunk's length zero and its last row's coupling C zero (q = 1); chunk
@@ -102,7 +104,7 @@ struct HostPlan {
 struct LineTables {
     LineDev dev{};
     std::vector<unsigned char> image;
-    size_t o_coef32 = 0, o_pcr = 0, o_blk = 0, o_rows64 = 0, o_rows32 = 0;
+    size_t o_coef32 = 0, o_pcr = 0, o_pidx = 0, o_blk = 0, o_rows64 = 0, o_rows32 = 0;
 };
 // Distinct chunk blocks, shared by the plans that are built with one pool.
 struct RowPool {
@@ -239,9 +241,8 @@ inline constexpr double LSRK_C[5] = {0.0, 1432997174477.0 / 9575080441755.0, 252
 // (1..3): the line-tile table entry for this descriptor when one exists
 // (*tuned = true), otherwise default_line_chunk.
 int line_chunk(int dim, const cles_solver_desc &d, bool *tuned = nullptr);
-// The largest chunk length (x: <= 16, y/z: <= 32, >= 8) that still gives a
-// launch of at least 131072 threads.
-int default_line_chunk(int dim, int64_t n_line, int64_t lines);
+// Chunk length by line length, line count and periodicity (cles_tune.cpp).
+int default_line_chunk(int dim, int64_t n_line, int64_t lines, bool periodic);
 
 // Ragged batch of independent lines (one line per instance, each with its own
 // length and plan), laid end to end: instance i occupies [off[i], off[i]+n).

@@ -113,7 +113,7 @@ __device__ __forceinline__ void epilogue(const EpiArgs &e, int64_t o, double v)
         const T *acc = (const T *)e.a0;
         const double dq = acc ? (double)(acc[o] - (T)v) : -v;
         const double dt = EPI == EPI_LSRK_DEV ? e.dtp[ii] : e.dt;
-        double nv = fma(dt, dq, e.c0 * e.du[o]);
+        double nv = fma(dt, dq, e.c0 != 0.0 ? e.c0 * e.du[o] : 0.0);
         e.du[o] = nv;
         e.Q[o] = fma(e.c1, nv, e.Q[o]);
     } else if constexpr (EPI == EPI_ART_MUBETA) {
@@ -198,7 +198,7 @@ __device__ __forceinline__ void epilogue_batch(const EpiArgs &e, const int64_t (
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             a[i] = (okk[i] && acc) ? acc[o[i]] : T(0);
-            du[i] = okk[i] ? e.du[o[i]] : 0.0;
+            du[i] = okk[i] && e.c0 != 0.0 ? e.du[o[i]] : 0.0;
             q[i] = okk[i] ? e.Q[o[i]] : 0.0;
         }
 #pragma unroll
@@ -492,7 +492,9 @@ __device__ __forceinline__ void correct_padded(T (&d)[CL], R64 R, const double (
 // PF: each step's coefficient blocks are loaded one step ahead, before the
 // exchange through LDS (the barriers wait for LDS traffic only), so their
 // latency overlaps the exchange; for per-lane chunk indices (the x sweep).
-template <int Q, bool PF = false>
+// UNI: k is wave-uniform (scalar loads).  The blocks of inner chunks are the
+// same block of the table (LineDev::pcr), so the lanes of a wave read a few.
+template <int Q, bool PF = false, bool UNI = false>
 __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int NT, int nl, int k, int li,
                                               double (&r)[2 * Q], double (&tp)[Q], double (&hn)[Q])
 {
@@ -500,16 +502,25 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
     const int P = p.P;
     const int slot = k * nl + li;
     const double *pc = p.pcr;
+    auto ld = [](const auto *q) {
+        if constexpr (UNI) return cload(q);
+        else return gload(q);
+    };
+    // offsets of this chunk's blocks, one per step and the final one
+    const int *ix = p.pidx + k;
+    const int last = p.nsteps - 1;
+    int at = ld(ix);
     if constexpr (PF) {
         constexpr int C = 2 * B * B;
         // one PCR step: multiplies by the blocks in cur and loads the next
         // step's into nxt (this step's again on the last step: in bounds, unused)
         auto step = [&](int st, double (&cur)[C], double (&nxt)[C]) {
             const int dd = 1 << st;
-            const int sn = st + 1 < p.nsteps ? st + 1 : st;
-            const double *an = pc + ((size_t)(sn * P + k) * 2) * B * B;
+            // at: the next step's block (this step's again on the last step)
+            const double *an = pc + at;
 #pragma unroll
-            for (int c = 0; c < C; c++) nxt[c] = gload(an + c);
+            for (int c = 0; c < C; c++) nxt[c] = ld(an + c);
+            at = ld(ix + (st + 2 < last ? st + 2 : last) * P);
             double *bf = buf + (st & 1) * B * NT;
 #pragma unroll
             for (int c = 0; c < B; c++) bf[c * NT + slot] = r[c];
@@ -542,9 +553,10 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
         };
         double ca[C], cb[C];
         if (p.nsteps > 0) {
-            const double *a0 = pc + (size_t)k * 2 * B * B;
+            const double *a0 = pc + at;
 #pragma unroll
-            for (int c = 0; c < C; c++) ca[c] = gload(a0 + c);
+            for (int c = 0; c < C; c++) ca[c] = ld(a0 + c);
+            at = ld(ix + (last > 0 ? 1 : 0) * P);
         }
         // two steps per trip, so the prefetch buffers alternate without copies
         for (int st = 0; st < p.nsteps; st += 2) {
@@ -572,27 +584,28 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
                 rm[c] = hm ? bf[c * NT + km * nl + li] : 0.0;
                 rp[c] = hp ? bf[c * NT + kp * nl + li] : 0.0;
             }
-            const double *al = pc + ((size_t)(st * P + k) * 2) * B * B;
+            const double *al = pc + at;
             const double *be = al + B * B;
+            at = ld(ix + (st + 1) * P);
 #pragma unroll
             for (int i = 0; i < B; i++) {
                 double acc = r[i];
 #pragma unroll
                 for (int j = 0; j < B; j++) {
-                    acc = fma(al[i * B + j], rm[j], acc);
-                    acc = fma(be[i * B + j], rp[j], acc);
+                    acc = fma(ld(al + i * B + j), rm[j], acc);
+                    acc = fma(ld(be + i * B + j), rp[j], acc);
                 }
                 r[i] = acc;
             }
         }
     }
-    const double *mi = pc + (size_t)p.nsteps * P * 2 * B * B + (size_t)k * B * B;
+    const double *mi = pc + (PF ? ld(ix + p.nsteps * P) : at);
     double z[B];
 #pragma unroll
     for (int i = 0; i < B; i++) {
         double acc = 0.0;
 #pragma unroll
-        for (int j = 0; j < B; j++) acc = fma(mi[i * B + j], r[j], acc);
+        for (int j = 0; j < B; j++) acc = fma(ld(mi + i * B + j), r[j], acc);
         z[i] = acc;
     }
     double *bf = buf + (p.nsteps & 1) * B * NT;
@@ -719,7 +732,12 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             if (acc) vload<V>(acc + o[i], a[i]);
-            vload<V>((const double *)e.du + o[i], du[i]);
+            if (e.c0 != 0.0) {
+                vload<V>((const double *)e.du + o[i], du[i]);
+            } else {   // the first stage (A = 0) does not read the register
+#pragma unroll
+                for (int j = 0; j < V; j++) du[i][j] = 0.0;
+            }
             vload<V>((const double *)e.Q + o[i], q[i]);
         }
 #pragma unroll
@@ -954,7 +972,7 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
                 r[Q + i] = (double)x;
             }
         }
-        reduced_solve<Q>(p, smem + (size_t)j * 2 * B * NT, NT, 64, k, lane, r, tp[j], hn[j]);
+        reduced_solve<Q, false, true>(p, smem + (size_t)j * 2 * B * NT, NT, 64, k, lane, r, tp[j], hn[j]);
     }
     if (!valid) return;
 
@@ -1214,20 +1232,25 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
     constexpr int B = 2 * Q;
     const int P = p.P;
     const double *pc = p.pcr;
-    auto ld = [](const double *q) {
+    auto ld = [](const auto *q) {
         if constexpr (UNI) return cload(q);
         else return gload(q);
     };
+    // offsets of this chunk's blocks, one per step and the final one
+    const int *ix = p.pidx + kc;
+    const int last = p.nsteps - 1;
+    int at = ld(ix);
     if constexpr (PF) {
         constexpr int C = 2 * B * B;
         // one PCR step: multiplies by the blocks in cur and loads the next
         // step's into nxt (this step's again on the last step: in bounds, unused)
         auto step = [&](int st, double (&cur)[C], double (&nxt)[C]) {
             const int dd = 1 << st;
-            const int sn = st + 1 < p.nsteps ? st + 1 : st;
-            const double *an = pc + ((size_t)(sn * P + kc) * 2) * B * B;
+            // at: the next step's block (this step's again on the last step)
+            const double *an = pc + at;
 #pragma unroll
-            for (int c = 0; c < C; c++) nxt[c] = gload(an + c);
+            for (int c = 0; c < C; c++) nxt[c] = ld(an + c);
+            at = ld(ix + (st + 2 < last ? st + 2 : last) * P);
             int km = k - dd, kp = k + dd;
             bool hm = true, hp = true;
             if (p.periodic) {
@@ -1260,9 +1283,10 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
         };
         double ca[C], cb[C];
         if (p.nsteps > 0) {
-            const double *a0 = pc + (size_t)kc * 2 * B * B;
+            const double *a0 = pc + at;
 #pragma unroll
-            for (int c = 0; c < C; c++) ca[c] = gload(a0 + c);
+            for (int c = 0; c < C; c++) ca[c] = ld(a0 + c);
+            at = ld(ix + (last > 0 ? 1 : 0) * P);
         }
         // two steps per trip, so the prefetch buffers alternate without copies
         for (int st = 0; st < p.nsteps; st += 2) {
@@ -1290,8 +1314,9 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
                 if (!hm) rm[c] = 0.0;
                 if (!hp) rp[c] = 0.0;
             }
-            const double *al = pc + ((size_t)(st * P + kc) * 2) * B * B;
+            const double *al = pc + at;
             const double *be = al + B * B;
+            at = ld(ix + (st + 1) * P);
 #pragma unroll
             for (int i = 0; i < B; i++) {
                 double acc = r[i];
@@ -1304,7 +1329,7 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
             }
         }
     }
-    const double *mi = pc + (size_t)p.nsteps * P * 2 * B * B + (size_t)kc * B * B;
+    const double *mi = pc + (PF ? ld(ix + p.nsteps * P) : at);
     double z[B];
 #pragma unroll
     for (int i = 0; i < B; i++) {

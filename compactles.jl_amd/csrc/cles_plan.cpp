@@ -318,7 +318,6 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     constexpr long double PCR_DROP = 1e-20L;
     std::vector<Mat> D(P, mat_eye(B)), L = Lb, U = Ub;
     std::vector<double> pcr;
-    pcr.reserve((size_t)(nsteps * P * 2 + P) * B * B);
     std::vector<double> steps((size_t)nsteps * P * 2 * B * B, 0.0);
     bool decoupled = false;
     for (int st = 0, d = 1; st < nsteps; st++, d *= 2) {
@@ -353,11 +352,30 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
         }
         D = D2; L = L2; U = U2;
     }
-    pcr = steps;
-    for (int k = 0; k < P; k++) {
-        Mat Mk = periodic && !decoupled ? mat_add(mat_add(D[k], L[k]), U[k]) : D[k];
-        Mat inv = mat_inv(Mk, B);
-        for (int i = 0; i < B * B; i++) pcr.push_back((double)inv[i]);
+    // the distinct blocks of the steps, then the final ones: inner chunks have
+    // the same neighbourhood and hence the same blocks
+    std::vector<int> pidx((size_t)(nsteps + 1) * P);
+    {
+        std::map<std::string, int> at;
+        auto place = [&](const double *v, size_t count) {
+            const std::string key((const char *)v, count * sizeof(double));
+            auto it = at.find(key);
+            if (it == at.end()) {
+                it = at.emplace(key, (int)pcr.size()).first;
+                pcr.insert(pcr.end(), v, v + count);
+            }
+            return it->second;
+        };
+        for (int st = 0; st < nsteps; st++)
+            for (int k = 0; k < P; k++)
+                pidx[(size_t)st * P + k] = place(&steps[((size_t)st * P + k) * 2 * B * B], (size_t)2 * B * B);
+        for (int k = 0; k < P; k++) {
+            Mat Mk = periodic && !decoupled ? mat_add(mat_add(D[k], L[k]), U[k]) : D[k];
+            Mat inv = mat_inv(Mk, B);
+            std::vector<double> v(B * B);
+            for (int i = 0; i < B * B; i++) v[i] = (double)inv[i];
+            pidx[(size_t)nsteps * P + k] = place(v.data(), v.size());
+        }
     }
 
     // coefficients (src/operators.jl:87-92): derivative RHS prescaled by 1/h,
@@ -429,14 +447,15 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
         blk[k] = it->second;
     }
 
-    // host image: coef64 | coef32 | pcr | blk | rows64 | rows32 (256-byte aligned parts)
+    // host image: coef64 | coef32 | pcr | pidx | blk | rows64 | rows32 (256-byte aligned parts)
     const size_t b_coef64 = COEF_N * sizeof(double), b_coef32 = COEF_N * sizeof(float);
-    const size_t b_pcr = pcr.size() * sizeof(double), b_blk = blk.size() * sizeof(int);
+    const size_t b_pcr = pcr.size() * sizeof(double), b_pidx = pidx.size() * sizeof(int), b_blk = blk.size() * sizeof(int);
     const size_t b_rows64 = own.rows.size() * sizeof(double), b_rows32 = own.rows.size() * sizeof(float);
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     out.o_coef32 = al(b_coef64);
     out.o_pcr = out.o_coef32 + al(b_coef32);
-    out.o_blk = out.o_pcr + al(std::max<size_t>(b_pcr, 8));
+    out.o_pidx = out.o_pcr + al(b_pcr);
+    out.o_blk = out.o_pidx + al(b_pidx);
     out.o_rows64 = out.o_blk + al(b_blk);
     out.o_rows32 = out.o_rows64 + al(b_rows64);
     out.image.assign(out.o_rows32 + al(b_rows32), 0);
@@ -447,6 +466,7 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     put(0, coef.data(), b_coef64);
     put(out.o_coef32, coef32.data(), b_coef32);
     put(out.o_pcr, pcr.data(), b_pcr);
+    put(out.o_pidx, pidx.data(), b_pidx);
     put(out.o_blk, blk.data(), b_blk);
     put(out.o_rows64, own.rows.data(), b_rows64);
     put(out.o_rows32, rows32.data(), b_rows32);
@@ -464,6 +484,7 @@ void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base)
     dev.coef64 = (const double *)base;
     dev.coef32 = (const float *)(base + t.o_coef32);
     dev.pcr = (const double *)(base + t.o_pcr);
+    dev.pidx = (const int *)(base + t.o_pidx);
     dev.blk = (const int *)(base + t.o_blk);
     dev.rows64 = (const double *)(base + t.o_rows64);
     dev.rows32 = (const float *)(base + t.o_rows32);

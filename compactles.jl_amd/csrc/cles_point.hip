@@ -718,7 +718,7 @@ __global__ void __launch_bounds__(TPB) k_lsrk(double *__restrict__ Q, double *__
     const unsigned ii = ipts ? (unsigned)(I % N) / ipts : 0u;
     if (gate && !gate[ii]) return;
     if (dtp) dt = dtp[ii];
-    const double v = fma(dt, (double)dQ[I], A * du[I]);
+    const double v = fma(dt, (double)dQ[I], A != 0.0 ? A * du[I] : 0.0);   // stage 1 (A = 0) does not read du
     du[I] = v;
     Q[I] += B * v;
 }

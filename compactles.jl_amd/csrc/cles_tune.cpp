@@ -43,18 +43,47 @@ TuneKey key_of(int dim, const cles_solver_desc &d)
                    d.filt.M};
 }
 
-constexpr int64_t TARGET_THREADS = 131072;   // 2048 waves: eight per CU
+// The rule for shapes the table does not hold (default_line_chunk): long chunks
+// do less work per point, short ones give more waves and shorter dependency
+// chains.  Measured on Taylor-Green steps of one field per launch:
+//  * 32-point chunks (y, z) from 131072 threads on: 190 x 160 x 170 FP64 (161k
+//    threads) 8.62 ms per step against 8.94 with 16; 128^3 (66k) 2.93 / 2.85;
+//  * 16-point chunks in y and z from 24576 threads on: 75 x 83 x 70 FP64 (27k)
+//    1.11 / 1.30 with 8, 80^3 (33k) 1.07 / 1.27; 64^3 (16k) 0.62 / 0.60; only
+//    on three-dimensional grids (many lines: 400 x 200 loses, 0.56 / 0.53);
+//  * in x, whose wave-local kernel runs equal chunks of a periodic line on
+//    scalar constants: 16 from 131072 threads on, or from 24576 where 16 gives
+//    equal chunks and 8 does not (120 x 97 x 81 FP64 1.63 / 1.70; 96^3, equal
+//    either way, 1.59 / 1.52).
+constexpr int64_t MANY_THREADS = 131072;   // 2048 waves: eight per CU
+constexpr int64_t SOME_THREADS = 24576;
+constexpr int64_t SOME_LINES = 4096;
 
 int cap_of(int dim) { return dim == 1 ? 16 : 32; }
 constexpr int MAX_TILE = 32;   // the kernels' per-thread chunk capacity
 
 }  // namespace
 
-int default_line_chunk(int dim, int64_t n_line, int64_t lines)
+int default_line_chunk(int dim, int64_t n_line, int64_t lines, bool periodic)
 {
-    for (int c = cap_of(dim); c >= 8; c /= 2)
-        if (lines * ((n_line + c - 1) / c) >= TARGET_THREADS) return c;
-    return 8;
+    auto chunks = [&](int c) {
+        int64_t P = 1;
+        while ((n_line + P - 1) / P > c) P *= 2;
+        return P;
+    };
+    auto threads = [&](int c) { return lines * ((n_line + c - 1) / c); };
+    const bool some = lines >= SOME_LINES && threads(16) >= SOME_THREADS;
+    int c = 8;
+    if (dim == 1) {
+        const bool even16 = periodic && n_line % chunks(16) == 0, even8 = periodic && n_line % chunks(8) == 0;
+        if (threads(16) >= MANY_THREADS || (some && even16 && !even8)) c = 16;
+    } else {
+        if (threads(32) >= MANY_THREADS) c = 32;
+        else if (threads(16) >= MANY_THREADS || some) c = 16;
+    }
+    // a block holds at most 512 chunks of a line
+    while (c < cap_of(dim) && chunks(c) > 512) c *= 2;
+    return c;
 }
 
 int line_chunk(int dim, const cles_solver_desc &d, bool *tuned)
@@ -71,7 +100,7 @@ int line_chunk(int dim, const cles_solver_desc &d, bool *tuned)
     int64_t N = 1;
     for (int k = 0; k < 3; k++) N *= d.n_global[k];
     const int64_t n = d.n_global[dim - 1];
-    return default_line_chunk(dim, n, N / n);
+    return default_line_chunk(dim, n, N / n, d.bc[dim - 1][0] == CLES_BC_PERIODIC);
 }
 
 }  // namespace cles

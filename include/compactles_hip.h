@@ -565,8 +565,10 @@ int cles_server_stats(cles_server *server, size_t *in_use, int *running, int *qu
  * cles_solver_create takes it from a process-wide table keyed by the grid,
  * precision, periodicity and scheme shapes; shapes the table does not hold
  * get the largest length (x <= 16, y/z <= 32, >= 8) that still launches
- * 131072 threads.  Nothing is tuned implicitly, so a table always gives the
- * same plans and the same results.
+ * 131072 threads, or 16 where that launches 24576 threads over 4096 lines or
+ * more (in x: only where 16 splits a periodic line evenly and 8 does not).
+ * Nothing is tuned implicitly, so a table always gives the same plans and the
+ * same results.
  *
  * cles_tune_solver times every candidate length (x: 16, 8, 4; y/z: 32, 16,
  * 8, 4) on the descriptor's grid (one four-field derivative launch and two

@@ -85,7 +85,7 @@ def test_block_x(ctx, dtype, bar, periodic, line):  # noqa: F811
 
 @pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
 @pytest.mark.parametrize("periodic", [True, False])
-@pytest.mark.parametrize("lanes,line", [(1, 40), (3, 9), (8, 16), (17, 33), (47, 64), (47, 100), (20, 700), (64, 600)])
+@pytest.mark.parametrize("lanes,line", [(1, 40), (3, 9), (8, 16), (17, 33), (47, 64), (47, 100), (20, 700), (64, 600), (2, 9000)])
 def test_narrow_yz(ctx, dtype, bar, periodic, lanes, line):  # noqa: F811
     """The narrow-block y / z sweeps: few lanes, or more chunks than 64 lanes
     leave room for; every chunk capacity, whole and uneven chunks."""
