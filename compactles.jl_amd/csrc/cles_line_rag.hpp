@@ -23,6 +23,12 @@ __device__ __forceinline__ unsigned rag_block(unsigned b, unsigned nb)
     return b < nfull ? (b & 7u) * (nfull >> 3) + (b >> 3) : b;
 }
 
+// One launch for both classes up to this many blocks (waves), twice what the
+// long class's registers let run at once: 512 tubes FP64, 1392 to 2784 blocks
+// per launch, 131.0 ms per 96 steps with two launches and 105.8 with one for up
+// to 2048 blocks.
+constexpr int64_t RAG_BOTH_BLOCKS = 4096;
+
 // Tile row of a line of at most CL P points with its halo, a pad slot after
 // every CL points (xw_slot) and room for the last chunk's window overrun.
 template <int CL, int M> __host__ __device__ constexpr int rag_row(int P)
@@ -41,12 +47,10 @@ template <int CL, int M> __host__ __device__ constexpr int rag_row(int P)
 // tests; the sweeps run on zero-padded rows.  96 steps of 512 tubes and their
 // states FP64, tables per instance / shared: 163.8 / 133.5 ms.
 template <typename T, int Q, int M, int SYM, int EPI, int CL>
-__global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict__ f, EpiArgs e)
+__device__ __forceinline__ void rag_item(const RagLines &r, unsigned logical, const T *__restrict__ f, EpiArgs e,
+                                         T *tile)
 {
-    extern __shared__ double smem[];
-    T *tile = (T *)smem;
     const int lane = threadIdx.x;
-    const unsigned logical = rag_block(blockIdx.x, gridDim.x);
     const int item = (int)(logical / (unsigned)r.nf), fld = (int)(logical % (unsigned)r.nf);
     const int64_t fo = (int64_t)fld * r.fstride;
     f += fo;
@@ -147,6 +151,28 @@ __global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict
     }
 }
 
+template <typename T, int Q, int M, int SYM, int EPI, int CL>
+__global__ void __launch_bounds__(64) k_line_rag(RagLines r, const T *__restrict__ f, EpiArgs e)
+{
+    extern __shared__ double smem[];
+    rag_item<T, Q, M, SYM, EPI, CL>(r, rag_block(blockIdx.x, gridDim.x), f, e, (T *)smem);
+}
+
+// Both classes in one launch, the longer lines' blocks first (they take
+// longest): batches too small to fill the chip with one class at a time run the
+// two side by side instead of one after the other.  The short class then has
+// the long one's registers and LDS, which is why large batches keep two launches.
+template <typename T, int Q, int M, int SYM, int EPI>
+__global__ void __launch_bounds__(64) k_line_rag_both(RagLines rs, RagLines rl, const T *__restrict__ f, EpiArgs e)
+{
+    extern __shared__ double smem[];
+    const unsigned nbl = (unsigned)rl.nitems * (unsigned)rl.nf;
+    if (blockIdx.x < nbl)
+        rag_item<T, Q, M, SYM, EPI, RAG_MAX_CHUNK>(rl, rag_block(blockIdx.x, nbl), f, e, (T *)smem);
+    else
+        rag_item<T, Q, M, SYM, EPI, RAG_SHORT_CHUNK>(rs, rag_block(blockIdx.x - nbl, gridDim.x - nbl), f, e, (T *)smem);
+}
+
 template <typename T, int Q, int M, int SYM, int EPI>
 void launch_rag_variant(const RagLines &r, const T *f, const EpiArgs &e, hipStream_t st)
 {
@@ -162,17 +188,24 @@ void launch_rag_variant(const RagLines &r, const T *f, const EpiArgs &e, hipStre
     rs.nitems = r.nshort;
     rl.items = r.items + 3 * r.nshort;
     rl.nitems = r.nitems - r.nshort;
+    const size_t shm_s = (size_t)(64 / r.pmin[0]) * rag_row<RAG_SHORT_CHUNK, M>(r.pmin[0]) * sizeof(T);
+    const size_t shm_l = (size_t)(64 / r.pmin[1]) * rag_row<RAG_MAX_CHUNK, M>(r.pmin[1]) * sizeof(T);
+    const int64_t blocks = (int64_t)r.nitems * r.nf;
+    if (rs.nitems > 0 && rl.nitems > 0 && blocks <= RAG_BOTH_BLOCKS) {
+        hipLaunchKernelGGL((k_line_rag_both<T, Q, M, SYM, EPI>), dim3((unsigned)blocks), dim3(64),
+                           std::max(shm_s, shm_l), st, rs, rl, f, e);
+        CLES_HIP(hipGetLastError());
+        return;
+    }
     if (rs.nitems > 0) {
-        const size_t shm = (size_t)(64 / r.pmin[0]) * rag_row<RAG_SHORT_CHUNK, M>(r.pmin[0]) * sizeof(T);
         const int64_t nb = (int64_t)rs.nitems * r.nf;
-        hipLaunchKernelGGL((k_line_rag<T, Q, M, SYM, EPI, RAG_SHORT_CHUNK>), dim3((unsigned)nb), dim3(64), shm, st, rs, f,
+        hipLaunchKernelGGL((k_line_rag<T, Q, M, SYM, EPI, RAG_SHORT_CHUNK>), dim3((unsigned)nb), dim3(64), shm_s, st, rs, f,
                            e);
         CLES_HIP(hipGetLastError());
     }
     if (rl.nitems > 0) {
-        const size_t shm = (size_t)(64 / r.pmin[1]) * rag_row<RAG_MAX_CHUNK, M>(r.pmin[1]) * sizeof(T);
         const int64_t nb = (int64_t)rl.nitems * r.nf;
-        hipLaunchKernelGGL((k_line_rag<T, Q, M, SYM, EPI, RAG_MAX_CHUNK>), dim3((unsigned)nb), dim3(64), shm, st, rl, f,
+        hipLaunchKernelGGL((k_line_rag<T, Q, M, SYM, EPI, RAG_MAX_CHUNK>), dim3((unsigned)nb), dim3(64), shm_l, st, rl, f,
                            e);
         CLES_HIP(hipGetLastError());
     }

@@ -925,7 +925,11 @@ template <typename W, bool CART = false>
 __device__ __forceinline__ double rate_at(const RateArgs<W> &a, int64_t I, int64_t N, double &rQ)
 {
     rQ = 0.0;
-    for (int sp = 0; sp < a.Ns; sp++) rQ += a.Q[(int64_t)sp * N + I];
+    // species loops are unrolled to the bound: a loop over the pointer arrays
+    // would copy them to scratch memory
+#pragma unroll
+    for (int sp = 0; sp < CLES_MAXSP; sp++)
+        if (sp < a.Ns) rQ += a.Q[(int64_t)sp * N + I];
     const double rho = a.rho[I];
     const double ri = 1 / rho;
     const double c = a.c[I];
@@ -964,8 +968,9 @@ __device__ __forceinline__ double rate_at(const RateArgs<W> &a, int64_t I, int64
         }
     }
     double Dmax = a.mu0 / (a.Sc * rho);
-    for (int sp = 0; sp < a.Ns; sp++)
-        if (a.D_art[sp]) Dmax = d_max(Dmax, a.mu0 / (a.Sc * rho) + (double)a.D_art[sp][I]);
+#pragma unroll
+    for (int sp = 0; sp < CLES_MAXSP; sp++)
+        if (sp < a.Ns && a.D_art[sp]) Dmax = d_max(Dmax, a.mu0 / (a.Sc * rho) + (double)a.D_art[sp][I]);
     const double mua = a.mu_art ? (double)a.mu_art[I] : 0.0;
     const double bea = a.beta_art ? (double)a.beta_art[I] : 0.0;
     const double kaa = a.kappa_art ? (double)a.kappa_art[I] : 0.0;
@@ -1153,12 +1158,17 @@ __global__ void __launch_bounds__(TPB) k_extrapolate(PlaneArgs a, double *__rest
 // density) derivatives come from full-field line operators run beforehand.
 // Arithmetic is FP64 in the reference's operation order for every precision.
 // ---------------------------------------------------------------------------
-template <typename W>
-__device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
+//
+// A face is a few hundred points, on x faces each in a cache line of its own, so
+// the launch lasts as long as one point's chain of memory round trips: every
+// input, the corrected dQ included, is loaded before anything is computed or
+// stored, the face's dimension is a template argument (the pointer arrays are
+// then indexed by constants) and blocks are one wave, to spread over the CUs.
+// Both x faces of 1024 x 512: 15.3 us before, 11.5 us so.
+template <typename W, int d>
+__device__ __forceinline__ void nscbc_face(const NscbcArgs<W> &a, int64_t t)
 {
-    if (t >= a.count) return;
-    const int d = a.dim;
-    const int oa = d == 0 ? 1 : 0, ob = d == 2 ? 1 : 2;
+    constexpr int oa = d == 0 ? 1 : 0, ob = d == 2 ? 1 : 2;
     int64_t idx[3];
     idx[d] = a.side == 0 ? 0 : a.n[d] - 1;
     idx[oa] = t % a.n[oa];
@@ -1167,10 +1177,23 @@ __device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
     const int64_t N = a.N;
     const double rho = a.rho[I], c = a.c[I], p = a.p[I], Tp = a.T[I], cpm = a.cp[I];
     const double uv[3] = {a.vel[0][I], a.vel[1][I], a.vel[2][I]};
+    double Yv[CLES_MAXSP], gYv[CLES_MAXSP], dq[CLES_MAXSP + 4];
+#pragma unroll
+    for (int k = 0; k < CLES_MAXSP; k++) {
+        Yv[k] = k < a.Ns ? (double)a.Y[k][I] : 0.0;
+        gYv[k] = k < a.Ns && a.gY[k] ? (double)a.gY[k][I] : 0.0;
+        dq[k] = k < a.Ns ? (double)a.dQ[(int64_t)k * N + I] : 0.0;
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) dq[CLES_MAXSP + m] = (double)a.dQ[(int64_t)(a.Ns + m) * N + I];
+    const double dpl = (double)a.dpn[I], dt1l = a.dt1 ? (double)a.dt1[I] : 0.0, dt2l = a.dt2 ? (double)a.dt2[I] : 0.0;
+    auto G = [&](int m) -> double { return a.gu[m] ? (double)a.gu[m][I] : 0.0; };
+    constexpr int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
+    const double gnn = G(d * 3 + d), g11 = G(t1 * 3 + t1), g1n = G(t1 * 3 + d), g22 = G(t2 * 3 + t2),
+                 g2n = G(t2 * 3 + d), gn1 = G(d * 3 + t1), gn2 = G(d * 3 + t2);
     const double un = uv[d];
     const double Ma = fabs(un) / c;
     if (!(Ma < 1)) return;   // supersonic point: every wave leaves
-    const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
     const int im = a.Ns;
     // inv_h of the face's dimensions (nscbc.jl:108,125,130,257); 1 on unit geometry
     double ih[3] = {1.0, 1.0, 1.0};
@@ -1183,21 +1206,21 @@ __device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
     const double Rm = p / (rho * Tp);
     const double phi = a.sg_phi > 0 ? a.sg_phi : cpm / Rm - 1;
     const double ke = 0.5 * (uv[0] * uv[0] + uv[1] * uv[1] + uv[2] * uv[2]);
-    const double dpn = ih[d] * (double)a.dpn[I];
-    const double dun = a.gu[d * 3 + d][I];
+    const double dpn = ih[d] * dpl;
+    const double dun = gnn;
     if (!a.inflow) {
         const double sgn = a.side == 1 ? -1.0 : 1.0;
         const double Lcomp = a.side == 1 ? (un - c) * (dpn - rho * c * dun) : (un + c) * (dpn + rho * c * dun);
         double tin = 0.0;
         if (a.act1) {
             const double ut = uv[t1];
-            tin += ut * ih[t1] * (double)a.dt1[I] + rho * c * c * (double)a.gu[t1 * 3 + t1][I] +
-                   sgn * rho * c * ut * (double)a.gu[t1 * 3 + d][I];
+            tin += ut * ih[t1] * dt1l + rho * c * c * g11 +
+                   sgn * rho * c * ut * g1n;
         }
         if (a.act2) {
             const double ut = uv[t2];
-            tin += ut * ih[t2] * (double)a.dt2[I] + rho * c * c * (double)a.gu[t2 * 3 + t2][I] +
-                   sgn * rho * c * ut * (double)a.gu[t2 * 3 + d][I];
+            tin += ut * ih[t2] * dt2l + rho * c * c * g22 +
+                   sgn * rho * c * ut * g2n;
         }
         const double bt = a.beta_t < 0 ? Ma : a.beta_t;
         const double K = a.sigma * (1 - Ma * Ma) * c / a.Lref;
@@ -1205,20 +1228,17 @@ __device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
         const double dd1 = dL / (2 * c * c);
         const double dd2 = dL / 2;
         const double dd3 = sgn * dL / (2 * rho * c);
-        for (int k = 0; k < a.Ns; k++) {
-            W *q = a.dQ + (int64_t)k * N + I;
-            *q = (W)((double)*q - (double)a.Y[k][I] * dd1);
-        }
+#pragma unroll
+        for (int k = 0; k < CLES_MAXSP; k++)
+            if (k < a.Ns) a.dQ[(int64_t)k * N + I] = (W)(dq[k] - Yv[k] * dd1);
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            W *q = a.dQ + (int64_t)(im + m) * N + I;
-            *q = (W)((double)*q - (uv[m] * dd1 + (m == d ? rho * dd3 : 0.0)));
+            a.dQ[(int64_t)(im + m) * N + I] = (W)(dq[CLES_MAXSP + m] - (uv[m] * dd1 + (m == d ? rho * dd3 : 0.0)));
         }
-        W *qe = a.dQ + (int64_t)(im + 3) * N + I;
-        *qe = (W)((double)*qe - (ke * dd1 + phi * dd2 + rho * un * dd3));
+        a.dQ[(int64_t)(im + 3) * N + I] = (W)(dq[CLES_MAXSP + 3] - (ke * dd1 + phi * dd2 + rho * un * dd3));
         return;
     }
-    const double drn = ih[d] * (double)a.dt1[I];
+    const double drn = ih[d] * dt1l;
     const double K = c / a.Lref;
     const double L1c = (un - c) * (dpn - rho * c * dun);
     const double L5c = (un + c) * (dpn + rho * c * dun);
@@ -1232,16 +1252,17 @@ __device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
     const double dd1 = dL2 / (c * c) + (dL5 + dL1) / (2 * c * c);
     const double dd2 = (dL5 + dL1) / 2;
     const double dd3 = (dL5 - dL1) / (2 * rho * c);
-    const double dd4 = a.eta_t * K * (uv[t1] - a.ut[t1]) - un * (double)a.gu[d * 3 + t1][I];
-    const double dd5 = a.eta_t * K * (uv[t2] - a.ut[t2]) - un * (double)a.gu[d * 3 + t2][I];
+    const double dd4 = a.eta_t * K * (uv[t1] - a.ut[t1]) - un * gn1;
+    const double dd5 = a.eta_t * K * (uv[t2] - a.ut[t2]) - un * gn2;
     const double cvm = cpm - Rm;
     double sphiY = 0.0;
-    for (int k = 0; k < a.Ns; k++) {
-        const double Yk = a.Y[k][I];
-        const double gYk = a.gY[k] ? (double)a.gY[k][I] : 0.0;
+#pragma unroll
+    for (int k = 0; k < CLES_MAXSP; k++) {
+        if (k >= a.Ns) continue;
+        const double Yk = Yv[k];
+        const double gYk = gYv[k];
         const double dLs = a.eta_Y * K * (Yk - a.Yt[k]) - un * gYk;
-        W *q = a.dQ + (int64_t)k * N + I;
-        *q = (W)((double)*q - (Yk * dd1 + rho * dLs));
+        a.dQ[(int64_t)k * N + I] = (W)(dq[k] - (Yk * dd1 + rho * dLs));
         // physics.jl:148-152 eos_dphi_dY; a Nasa9Mixture takes cv_k(T) (physics.jl:504-510)
         const double cvk = a.n9 ? n9_cp(*a.n9, k, Tp) - a.Rk[k] : a.cvk[k];
         if (!(a.sg_phi > 0)) sphiY += (cvk * Rm - a.Rk[k] * cvm) / (Rm * Rm) * dLs;   // :212: 0 for a stiffened gas
@@ -1249,26 +1270,35 @@ __device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
 #pragma unroll
     for (int m = 0; m < 3; m++) {
         const double extra = m == d ? rho * dd3 : m == t1 ? rho * dd4 : rho * dd5;
-        W *q = a.dQ + (int64_t)(im + m) * N + I;
-        *q = (W)((double)*q - (uv[m] * dd1 + extra));
+        a.dQ[(int64_t)(im + m) * N + I] = (W)(dq[CLES_MAXSP + m] - (uv[m] * dd1 + extra));
     }
-    W *qe = a.dQ + (int64_t)(im + 3) * N + I;
-    *qe = (W)((double)*qe - (ke * dd1 + phi * dd2 + p * sphiY + rho * (un * dd3 + uv[t1] * dd4 + uv[t2] * dd5)));
+    a.dQ[(int64_t)(im + 3) * N + I] = (W)(dq[CLES_MAXSP + 3] - (ke * dd1 + phi * dd2 + p * sphiY + rho * (un * dd3 + uv[t1] * dd4 + uv[t2] * dd5)));
 }
 
 template <typename W>
-__global__ void __launch_bounds__(TPB) k_nscbc(NscbcArgs<W> a)
+__device__ __forceinline__ void nscbc_point(const NscbcArgs<W> &a, int64_t t)
 {
-    nscbc_point(a, (int64_t)blockIdx.x * TPB + threadIdx.x);
+    if (t >= a.count) return;
+    if (a.dim == 0) nscbc_face<W, 0>(a, t);
+    else if (a.dim == 1) nscbc_face<W, 1>(a, t);
+    else nscbc_face<W, 2>(a, t);
+}
+
+constexpr int NSCBC_TPB = 64;
+
+template <typename W>
+__global__ void __launch_bounds__(NSCBC_TPB) k_nscbc(NscbcArgs<W> a)
+{
+    nscbc_point(a, (int64_t)blockIdx.x * NSCBC_TPB + threadIdx.x);
 }
 
 // Both faces of one dimension in one launch (grid y = side): their planes are
 // disjoint (n >= 2 along the normal), and each thread updates dQ at its own
 // face point only, so the result is that of the two launches in order.
 template <typename W>
-__global__ void __launch_bounds__(TPB) k_nscbc_pair(NscbcArgs<W> a0, NscbcArgs<W> a1)
+__global__ void __launch_bounds__(NSCBC_TPB) k_nscbc_pair(NscbcArgs<W> a0, NscbcArgs<W> a1)
 {
-    const int64_t t = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * NSCBC_TPB + threadIdx.x;
     if (blockIdx.y == 0)
         nscbc_point(a0, t);
     else
@@ -1733,7 +1763,7 @@ template <typename W>
 void launch_nscbc(const NscbcArgs<W> &a, hipStream_t st)
 {
     if (a.count <= 0) return;
-    hipLaunchKernelGGL((k_nscbc<W>), dim3(nblocks(a.count)), dim3(TPB), 0, st, a);
+    hipLaunchKernelGGL((k_nscbc<W>), dim3(nblocks(a.count, NSCBC_TPB)), dim3(NSCBC_TPB), 0, st, a);
     CHECK_LAUNCH();
 }
 template void launch_nscbc<double>(const NscbcArgs<double> &, hipStream_t);
@@ -1745,7 +1775,7 @@ void launch_nscbc_pair(const NscbcArgs<W> &a0, const NscbcArgs<W> &a1, hipStream
     if (a0.dim != a1.dim || a0.side == a1.side || a0.n[a0.dim] < 2 || a0.count != a1.count)
         throw Error{CLES_ERR_INVALID, "an NSCBC face pair is the two faces of one dimension"};
     if (a0.count <= 0) return;
-    hipLaunchKernelGGL((k_nscbc_pair<W>), dim3(nblocks(a0.count), 2), dim3(TPB), 0, st, a0, a1);
+    hipLaunchKernelGGL((k_nscbc_pair<W>), dim3(nblocks(a0.count, NSCBC_TPB), 2), dim3(NSCBC_TPB), 0, st, a0, a1);
     CHECK_LAUNCH();
 }
 template void launch_nscbc_pair<double>(const NscbcArgs<double> &, const NscbcArgs<double> &, hipStream_t);
