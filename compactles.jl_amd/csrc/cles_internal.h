@@ -154,8 +154,8 @@ struct PinnedBuf {
     void *get(size_t bytes);
     void release();
 };
-// Pinned staging of one owner (at most 6 x 2 buffers of 4 MB, or of a row that
-// is longer), freed with it; transfers of one stage run one at a time.
+// Pinned staging of one owner (at most 6 x 8 MB, or two rows where those are
+// longer), freed with it; transfers of one stage run one at a time.
 struct HostStage {
     ~HostStage();
     // Moves ncomp components of contiguous device rows (component c, plane k,
@@ -167,7 +167,7 @@ struct HostStage {
 
 private:
     struct Lane {
-        PinnedBuf buf[2];
+        PinnedBuf buf;
         hipEvent_t ev[2] = {nullptr, nullptr};
     };
     std::mutex mu;
@@ -224,9 +224,21 @@ struct LineFields {
     int64_t eoff[LINE_MF] = {};
 };
 
+// The z direction of a launch that does y and z (store epilogue; fields nf ..
+// 2 nf - 1 of LineFields are its inputs and outputs).
+struct LineSecond {
+    LineDev p;
+    int64_t so;
+    int sd, slabs;
+    int nouter1, nouter;    // outer extents of the two directions
+};
+
 // Launch one line operator along `dim` (1..3) over the view (mf: more fields).
-void launch_line(const HostPlan &hp, int dim, const View3 &v, const void *f,
-                 const EpiArgs &epi, hipStream_t st, const LineFields *mf = nullptr);
+// hp2: dim is 2, and the same launch applies hp2 along z to fields mf->nf ..
+// 2 mf->nf - 1 (pairable_lines must hold).
+void launch_line(const HostPlan &hp, int dim, const View3 &v, const void *f, const EpiArgs &epi, hipStream_t st,
+                 const LineFields *mf = nullptr, const HostPlan *hp2 = nullptr);
+bool pairable_lines(const HostPlan &a, const HostPlan &b, const View3 &v, int nf);
 
 // timestep.jl:5-21 LSRK(5,4) coefficient tables (Carpenter & Kennedy)
 inline constexpr double LSRK_A[5] = {0.0, -567301805773.0 / 1357537059087.0, -2404267990393.0 / 2016746695238.0,

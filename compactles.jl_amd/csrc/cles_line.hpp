@@ -253,7 +253,9 @@ __device__ __forceinline__ void epilogue_batch(const EpiArgs &e, const int64_t (
 template <typename T, int EPI>
 __device__ __forceinline__ void select_field(const LineFields &mf, const T *__restrict__ &f, EpiArgs &e)
 {
-    const int i = blockIdx.y;
+    // grid z = 1: the second direction of a paired launch, whose outputs follow
+    // the first direction's in the table (its inputs are the same fields)
+    const int i = EPI == EPI_STORE ? blockIdx.y + gridDim.y * blockIdx.z : blockIdx.y;
     if constexpr (EPI == EPI_ART_MULTI) e = e.multi[i];
     if (i == 0) return;
     f = (const T *)mf.in[i];
@@ -819,17 +821,32 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
 
 template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V, bool NTS>
 __global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
-k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
-           LineFields mf)
+k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
+           LineFields mf, LineSecond two)
 {
     select_field<T, EPI>(mf, f, e);
     extern __shared__ double smem[];
     constexpr int B = 2 * Q;
+    const bool second = EPI == EPI_STORE && blockIdx.z;
+    LineDev p = p1;
+    unsigned nb = gridDim.x;
+    if constexpr (EPI == EPI_STORE) {
+        if (gridDim.z > 1) {   // the two directions may differ in lines, hence in blocks
+            nb = (unsigned)nxb * (unsigned)(second ? two.nouter : two.nouter1);
+            if (second) {
+                p = two.p;
+                sd = two.sd;
+                so = two.so;
+                slabs = two.slabs;
+            }
+            if (blockIdx.x >= nb) return;
+        }
+    }
     const int P = p.P, n = p.n;
     const int NT = 64 * P;
     const int lane = (int)(threadIdx.x & 63);
     const int k = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const unsigned blk = slabs ? xcd_slab(blockIdx.x, gridDim.x) : blockIdx.x;
+    const unsigned blk = slabs ? xcd_slab(blockIdx.x, nb) : blockIdx.x;
     const int xb = blk % nxb;
     const int64_t ob = blk / nxb;
     const int x0 = (xb * 64 + lane) * V;
@@ -1017,10 +1034,22 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
 // with too many chunks for 64 lanes.
 // ---------------------------------------------------------------------------
 template <typename T, int Q, int M, int SYM, int EPI, int CL>
-__global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restrict__ f, int sd, int64_t so,
-                                                  int nlane, int nxb, int Lx, EpiArgs e, LineFields mf)
+__global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p1, const T *__restrict__ f, int sd, int64_t so,
+                                                  int nlane, int nxb, int Lx, EpiArgs e, LineFields mf, LineSecond two)
 {
     select_field<T, EPI>(mf, f, e);
+    const bool second = EPI == EPI_STORE && blockIdx.z;
+    LineDev p = p1;
+    if constexpr (EPI == EPI_STORE) {
+        if (gridDim.z > 1) {
+            if (second) {
+                p = two.p;
+                sd = two.sd;
+                so = two.so;
+            }
+            if (blockIdx.x >= (unsigned)nxb * (unsigned)(second ? two.nouter : two.nouter1)) return;
+        }
+    }
     extern __shared__ double smem[];
     const int NT = Lx * p.P;
     const int lane = (int)(threadIdx.x % Lx);
@@ -1619,7 +1648,7 @@ inline void allow_lds(K kern, size_t shm)
 
 template <typename T, int Q, int M, int SYM, int EPI>
 void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, const EpiArgs &e,
-                           hipStream_t st, const LineFields &mf)
+                           hipStream_t st, const LineFields &mf, const HostPlan *hp2)
 {
     const unsigned nf = (unsigned)mf.nf;
     const LineDev &p = hp.dev;
@@ -1690,7 +1719,19 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         const int64_t nlane = v.n[0];
         const int64_t sd = dim == 2 ? v.s[1] : v.s[2];
         const int64_t so = dim == 2 ? v.s[2] : v.s[1];
-        const int64_t nouter = dim == 2 ? v.n[2] : v.n[1];
+        // hp2: the z direction (dim is 2) in the same launch, grid z = 1
+        // (pairable_lines has checked that it takes the same kernel)
+        LineSecond two{};
+        if (hp2) {
+            two.p = hp2->dev;
+            two.sd = (int)v.s[2];
+            two.so = v.s[1];
+            two.slabs = 0;
+            two.nouter = (int)v.n[1];
+            two.nouter1 = (int)v.n[2];
+        }
+        const unsigned nz = hp2 ? 2 : 1;
+        const int64_t nouter = dim == 2 ? (hp2 ? std::max(v.n[1], v.n[2]) : v.n[2]) : v.n[1];
         if ((int64_t)(p.n - 1) * sd > INT32_MAX) throw Error{CLES_ERR_UNSUPPORTED, "array too large for 32-bit line offsets"};
         if (nlane >= 48 && 64 * P <= maxNT) {
             const int NT = 64 * P;
@@ -1700,12 +1741,12 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             // faster without it.
             const bool nts = dim == 3 && (EPI == EPI_STORE || EPI == EPI_STORE_NEG) &&
                              (double)v.n[0] * v.n[1] * v.n[2] * sizeof(T) * nf > 256.0 * 1024 * 1024;
-            const bool full = p.extra == 0 && p.m == p.cap;
+            const bool full = p.extra == 0 && p.m == p.cap && (!hp2 || (two.p.extra == 0 && two.p.m == two.p.cap));
             auto go = [&](auto kern, int V) {
                 const int nxb = (int)((nlane + 64 * V - 1) / (64 * V));
                 const size_t shm = (size_t)2 * B * NT * V * sizeof(double);
-                hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf), dim3(NT), shm, st, p, f, (int)sd, so,
-                                   (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf);
+                hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf, nz), dim3(NT), shm, st, p, f, (int)sd, so,
+                                   (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf, two);
             };
             auto pick = [&](auto cl, auto vv, auto nt) {
                 if (full) go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, true, vv.value, nt.value>, vv.value);
@@ -1719,22 +1760,22 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             };
             // two lines per lane in FP32 where the launch still has two blocks
             // per CU (the row width must be even)
-            bool two = false;
+            bool pairs = false;
             if constexpr (sizeof(T) == 4 && Q == 1)
-                two = nlane % 2 == 0 && ((nlane + 127) / 128) * nouter * (int64_t)nf >= 512;
+                pairs = nlane % 2 == 0 && ((nlane + 127) / 128) * nouter * (int64_t)nf * nz >= 512;
             if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_NEG) {
                 if (nts) {
                     if constexpr (sizeof(T) == 4 && Q == 1) {
-                        if (two) capd(integral_constant<int, 2>{}, std::true_type{});
+                        if (pairs) capd(integral_constant<int, 2>{}, std::true_type{});
                     }
-                    if (!two) capd(integral_constant<int, 1>{}, std::true_type{});
+                    if (!pairs) capd(integral_constant<int, 1>{}, std::true_type{});
                 }
             }
             if (!nts) {
                 if constexpr (sizeof(T) == 4 && Q == 1) {
-                    if (two) capd(integral_constant<int, 2>{}, std::false_type{});
+                    if (pairs) capd(integral_constant<int, 2>{}, std::false_type{});
                 }
-                if (!two) capd(integral_constant<int, 1>{}, std::false_type{});
+                if (!pairs) capd(integral_constant<int, 1>{}, std::false_type{});
             }
         } else {
             int Lx = 64;
@@ -1742,20 +1783,20 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             while (Lx / 2 >= nlane && Lx > 1) Lx /= 2;   // narrow x extents (2-D / 1-D grids)
             // few lines (2-D grids): narrower blocks, down to 8 lanes (64-byte
             // rows), until the launch has two blocks per CU
-            while (Lx > 8 && ((nlane + Lx - 1) / Lx) * nouter * (int64_t)nf < 512) Lx /= 2;
+            while (Lx > 8 && ((nlane + Lx - 1) / Lx) * nouter * (int64_t)nf * nz < 512) Lx /= 2;
             if (Lx * P > 512) throw Error{CLES_ERR_UNSUPPORTED, "line too long for the y/z-sweep kernel"};
             const int NT = Lx * P;
             const int nxb = (int)((nlane + Lx - 1) / Lx);
             const size_t shm = (size_t)2 * B * NT * sizeof(double);
             if (p.cap == 8)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 8>), dim3((unsigned)(nxb * nouter), nf),
-                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
+                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 8>), dim3((unsigned)(nxb * nouter), nf, nz),
+                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf, two);
             else if (p.cap == 16)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 16>), dim3((unsigned)(nxb * nouter), nf),
-                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
+                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 16>), dim3((unsigned)(nxb * nouter), nf, nz),
+                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf, two);
             else
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, MC>), dim3((unsigned)(nxb * nouter), nf),
-                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf);
+                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, MC>), dim3((unsigned)(nxb * nouter), nf, nz),
+                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf, two);
         }
     }
     CLES_HIP(hipGetLastError());
@@ -1763,25 +1804,25 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
 
 template <typename T, int Q, int M, int SYM>
 void launch_epi(const HostPlan &hp, int dim, const View3 &v, const T *f, const EpiArgs &e, hipStream_t st,
-                const LineFields &mf)
+                const LineFields &mf, const HostPlan *hp2)
 {
     if constexpr (SYM) {
         switch (e.kind) {
-        case EPI_STORE: return launch_variant<T, Q, M, SYM, EPI_STORE>(hp, dim, v, f, e, st, mf);
-        case EPI_STORE_GATE: return launch_variant<T, Q, M, SYM, EPI_STORE_GATE>(hp, dim, v, f, e, st, mf);
-        case EPI_ART_MUBETA: return launch_variant<T, Q, M, SYM, EPI_ART_MUBETA>(hp, dim, v, f, e, st, mf);
-        case EPI_ART_KAPPA: return launch_variant<T, Q, M, SYM, EPI_ART_KAPPA>(hp, dim, v, f, e, st, mf);
-        case EPI_ART_D: return launch_variant<T, Q, M, SYM, EPI_ART_D>(hp, dim, v, f, e, st, mf);
-        case EPI_ART_MULTI: return launch_variant<T, Q, M, SYM, EPI_ART_MULTI>(hp, dim, v, f, e, st, mf);
+        case EPI_STORE: return launch_variant<T, Q, M, SYM, EPI_STORE>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_STORE_GATE: return launch_variant<T, Q, M, SYM, EPI_STORE_GATE>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_ART_MUBETA: return launch_variant<T, Q, M, SYM, EPI_ART_MUBETA>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_ART_KAPPA: return launch_variant<T, Q, M, SYM, EPI_ART_KAPPA>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_ART_D: return launch_variant<T, Q, M, SYM, EPI_ART_D>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_ART_MULTI: return launch_variant<T, Q, M, SYM, EPI_ART_MULTI>(hp, dim, v, f, e, st, mf, hp2);
         default: break;
         }
     } else {
         switch (e.kind) {
-        case EPI_STORE: return launch_variant<T, Q, M, SYM, EPI_STORE>(hp, dim, v, f, e, st, mf);
-        case EPI_STORE_NEG: return launch_variant<T, Q, M, SYM, EPI_STORE_NEG>(hp, dim, v, f, e, st, mf);
-        case EPI_SUB: return launch_variant<T, Q, M, SYM, EPI_SUB>(hp, dim, v, f, e, st, mf);
-        case EPI_LSRK: return launch_variant<T, Q, M, SYM, EPI_LSRK>(hp, dim, v, f, e, st, mf);
-        case EPI_LSRK_DEV: return launch_variant<T, Q, M, SYM, EPI_LSRK_DEV>(hp, dim, v, f, e, st, mf);
+        case EPI_STORE: return launch_variant<T, Q, M, SYM, EPI_STORE>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_STORE_NEG: return launch_variant<T, Q, M, SYM, EPI_STORE_NEG>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_SUB: return launch_variant<T, Q, M, SYM, EPI_SUB>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_LSRK: return launch_variant<T, Q, M, SYM, EPI_LSRK>(hp, dim, v, f, e, st, mf, hp2);
+        case EPI_LSRK_DEV: return launch_variant<T, Q, M, SYM, EPI_LSRK_DEV>(hp, dim, v, f, e, st, mf, hp2);
         default: break;
         }
     }

@@ -26,8 +26,8 @@ __device__ __forceinline__ unsigned rag_block(unsigned b, unsigned nb)
 // One launch for both classes up to this many blocks (waves), twice what the
 // long class's registers let run at once: 512 tubes FP64, 1392 to 2784 blocks
 // per launch, 131.0 ms per 96 steps with two launches and 105.8 with one for up
-// to 2048 blocks.
-constexpr int64_t RAG_BOTH_BLOCKS = 4096;
+// to 2048 blocks; 1024 tubes 1.76 / 1.73 ms per step, 4096 tubes 6.34 / 6.36.
+constexpr int64_t RAG_BOTH_BLOCKS = 8192;
 
 // Tile row of a line of at most CL P points with its halo, a pad slot after
 // every CL points (xw_slot) and room for the last chunk's window overrun.

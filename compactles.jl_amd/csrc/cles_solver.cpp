@@ -434,51 +434,80 @@ struct Impl {
     // every field of one direction in one launch
     void velocity_gradients(bool scalars = false) const
     {
-        for (int k = 0; k < s.nact; k++) gradients_along(k, scalars);
+        // y and z in one launch where they take the same kernel
+        const bool yz = s.nact >= 2 && s.active[1] && s.active[2] && !s.fold[1].on && !s.fold[2].on;
+        for (int k = 0; k < s.nact; k++) {
+            const int d = s.adim[k];
+            if (d == 1 && yz) {
+                GradList y = grad_list(1, scalars);
+                const GradList z = grad_list(2, scalars);
+                if (y.nf == z.nf && pairable_lines(s.dplan[1], s.dplan[2], view(), y.nf)) {
+                    LineFields mf;
+                    mf.nf = y.nf;
+                    for (int i = 0; i < y.nf; i++) {
+                        mf.in[i] = y.in[i];
+                        mf.out[i] = y.out[i];
+                        mf.in[y.nf + i] = z.in[i];
+                        mf.out[y.nf + i] = z.out[i];
+                    }
+                    s.timed(PH_DERIV + 1, line_bytes(s.dplan[1], EPI_STORE) * (double)s.N * 2 * y.nf, [&] {
+                        launch_line(s.dplan[1], 2, view(), mf.in[0], store(mf.out[0]), s.st(), &mf, &s.dplan[2]);
+                    });
+                    for (int dd = 1; dd <= 2; dd++) {
+                        GradList g = dd == 1 ? y : z;
+                        if (s.met.m[dd] || s.curv) metric(g.out, g.nf, 0, dd);
+                    }
+                    break;
+                }
+            }
+            gradients_along(k, scalars);
+        }
         if (s.curv) {   // rhs.jl:604 metric_correct_gradients!
             const CurvArgs<W> a = curv_args();
             s.timed(PH_OTHER, sizeof(W) * 10.0 * (double)s.N, [&] { launch_metric_grad<W>(a, s.st()); });
         }
     }
+    // the fields of the gradients along dimension d
+    struct GradList {
+        int nf = 3;
+        const void *in[LINE_MF] = {};
+        void *out[LINE_MF] = {};
+        int par[LINE_MF] = {};
+    };
+    GradList grad_list(int d, bool scalars) const
+    {
+        GradList g;
+        const void *vel[3] = {s.u, s.v, s.w};
+        for (int j = 0; j < 3; j++) {
+            g.in[j] = vel[j];
+            g.out[j] = s.gu[d * 3 + j];
+            g.par[j] = vel_parity(d, j);
+        }
+        auto add = [&](const void *in, void *out) {
+            g.par[g.nf] = 1;
+            g.in[g.nf] = in;
+            g.out[g.nf++] = out;
+        };
+        if (!scalars) return g;
+        add(s.T, s.gT[d]);
+        if (s.Ns > 1)
+            for (int sp = 0; sp < s.Ns; sp++) add(s.Y[sp], s.gY[d][sp]);
+        if (s.nscbc && s.nsd_merged) {   // the NSCBC faces' full-field derivatives
+            bool np[3], nr[3];
+            nscbc_needs(np, nr);
+            if (np[d]) add(s.p, s.nsdp[d]);
+            if (nr[d]) add(s.rho, s.nsdr[d]);
+        }
+        return g;
+    }
     // the gradients along the k-th active dimension
     void gradients_along(int k, bool scalars) const
     {
-        {
-            const int d = s.adim[k];
-            const void *in[LINE_MF] = {s.u, s.v, s.w};
-            void *out[LINE_MF] = {s.gu[d * 3], s.gu[d * 3 + 1], s.gu[d * 3 + 2]};
-            int par[LINE_MF] = {vel_parity(d, 0), vel_parity(d, 1), vel_parity(d, 2)};
-            int nf = 3;
-            if (scalars) {
-                par[nf] = 1;
-                in[nf] = s.T;
-                out[nf++] = s.gT[d];
-                if (s.Ns > 1)
-                    for (int sp = 0; sp < s.Ns; sp++) {
-                        par[nf] = 1;
-                        in[nf] = s.Y[sp];
-                        out[nf++] = s.gY[d][sp];
-                    }
-                if (s.nscbc && s.nsd_merged) {   // the NSCBC faces' full-field derivatives
-                    bool np[3], nr[3];
-                    nscbc_needs(np, nr);
-                    if (np[d]) {
-                        par[nf] = 1;
-                        in[nf] = s.p;
-                        out[nf++] = s.nsdp[d];
-                    }
-                    if (nr[d]) {
-                        par[nf] = 1;
-                        in[nf] = s.rho;
-                        out[nf++] = s.nsdr[d];
-                    }
-                }
-            }
-            lines_par(DERIV, d, nf, in, out, par, store(out[0]), PH_DERIV);
-            if (s.met.m[d] || s.curv) metric(out, nf, 0, d);   // rhs.jl:599,631,634 _scale_grad!
-        }
+        const int d = s.adim[k];
+        const GradList g = grad_list(d, scalars);
+        lines_par(DERIV, d, g.nf, g.in, g.out, g.par, store(g.out[0]), PH_DERIV);
+        if (s.met.m[d] || s.curv) metric(g.out, g.nf, 0, d);   // rhs.jl:599,631,634 _scale_grad!
     }
-
 
     CurvArgs<W> curv_args() const
     {

@@ -90,9 +90,10 @@ void HostStage::transfer(bool down, int device, hipStream_t st, double *dev, con
         auto first = [&](int64_t i) { return (w + i * nlane) * per; };
         auto rows = [&](int64_t i) { return std::min<int64_t>(per, nrows - first(i)); };
         const int64_t mine = (nchunk - w + nlane - 1) / nlane;
-        auto buf = [&](int64_t i) {
-            return (char *)l.buf[i & 1].get(row * (size_t)std::min<int64_t>(per, nrows));
-        };
+        // both buffers in one allocation (each costs about 0.1 ms to pin)
+        const size_t half = row * (size_t)std::min<int64_t>(per, nrows);
+        char *const base = (char *)l.buf.get(half * (size_t)std::min<int64_t>(2, mine));
+        auto buf = [&](int64_t i) { return base + half * (size_t)(i & 1); };
         auto issue = [&](int64_t i) {
             char *b = buf(i);
             double *d = dev + first(i) * n0;

@@ -3,5 +3,5 @@
 
 namespace cles {
 template void launch_epi<double, 1, 4, 1>(const HostPlan &, int, const View3 &, const double *, const EpiArgs &,
-                                            hipStream_t, const LineFields &);
+                                            hipStream_t, const LineFields &, const HostPlan *);
 }  // namespace cles

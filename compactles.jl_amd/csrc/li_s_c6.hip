@@ -3,5 +3,5 @@
 
 namespace cles {
 template void launch_epi<float, 1, 2, 0>(const HostPlan &, int, const View3 &, const float *, const EpiArgs &,
-                                            hipStream_t, const LineFields &);
+                                            hipStream_t, const LineFields &, const HostPlan *);
 }  // namespace cles

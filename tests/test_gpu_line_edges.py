@@ -7,6 +7,7 @@ import pytest
 
 import helpers as Hh
 from test_gpu_operators import _gpu_apply, _oracle_apply, ctx  # noqa: F401
+from test_gpu_solver import _compare_rhs
 
 pytestmark = pytest.mark.gpu
 
@@ -98,3 +99,31 @@ def test_narrow_yz(ctx, dtype, bar, periodic, lanes, line):  # noqa: F811
             ref = _oracle_apply(name, dim, n, periodic, 0.1, f)
             got = _gpu_apply(ctx, name, dim, n, periodic, 0.1, f, dtype=dtype)
             assert Hh.relerr(got, ref) <= bar, (name, dim, n)
+
+
+@pytest.mark.parametrize("n,species", [((24, 20, 20), 1), ((24, 33, 20), 1), ((64, 17, 19), 1), ((50, 40, 36), 2),
+                                       ((12, 9, 24), 1)])
+def test_paired_gradients(ctx, n, species):  # noqa: F811
+    """The y and z gradients of one launch (equal chunk counts, unequal outer
+    extents, more fields for two species) and, where the directions differ too
+    much, of two: against the oracle's RHS."""
+    import cases
+    L = (2 * np.pi,) * 3
+    X, Y, Z = cases.grid(n, L)
+    kw = {}
+    if species == 2:
+        th = 0.5 * (1 + 0.5 * np.sin(X + Y) * np.cos(Z))
+        q = cases.conserved(cases.smooth_prim(X, Y, Z), species=cases.HE_CO2, Y=[1 - th, th])
+        kw["species"] = cases.HE_CO2
+    else:
+        q = cases.conserved(cases.smooth_prim(X, Y, Z))
+    gs = cases.gpu_solver(ctx, n, L, q, **kw)
+    os_ = cases.oracle_solver(n, L, q, art=True, **kw)
+    gs.compute_rhs(False)
+    os_.compute_rhs(False)
+    _compare_rhs(gs, os_, n)
+    for d in (1, 2, 3):
+        for j in (1, 2, 3):
+            name = f"grad_u[{d}{j}]"
+            assert Hh.relerr(gs.field(name), os_.interior(os_.field(name))) <= 1e-12, name
+    gs.close()
