@@ -74,7 +74,8 @@ struct LineDev {
                            // step, or a final inverse block
     const int *pidx;       // [s * P + k]: offset in pcr of chunk k's block of step s < nsteps, and of
                            // its final block (s = nsteps)
-    int cap;               // chunk capacity of the kernels: 8, 16 or 32 >= the longest chunk (ragged: 16 or 32)
+    int cap;               // chunk capacity of the kernel: 8, 12, 16, 24 or 32 >= the longest chunk
+                           // (12 and 24 only in some kernels; ragged: 16 or 32)
     // Row constants: one block [field * cap + t] per distinct chunk, rows past
     // the chunk's length zero and its last row's coupling C zero (q = 1); chunk
     // k has the block at rows64 + blk[k].  Chunks inside a line factorise alike,
@@ -120,9 +121,10 @@ struct RowPool {
 // interior column -j-1 with sign sigma_g, and the low-edge RHS rows read the
 // mirror f(-j-1) sigma_f of each ghost (sigma_f = sigma_g for filters, -sigma_g
 // for derivatives), carried as synthesised closure rows.
+// lanes: extent along x (which y / z kernel the plan goes to).
 // hi_fold does the same at the high edge (ghost n + j mirrors n - 1 - j).
 void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int periodic, double h, int max_chunk,
-                       int dim, RowPool *pool = nullptr, int lo_fold = 0, int hi_fold = 0);
+                       int dim, RowPool *pool = nullptr, int lo_fold = 0, int hi_fold = 0, int64_t lanes = 0);
 void bind_line_tables(LineDev &dev, const LineTables &t, unsigned char *base);
 
 // Builds the device tables for one (scheme, n, periodic, h).  Throws Error.

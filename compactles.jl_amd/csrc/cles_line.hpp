@@ -651,7 +651,9 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
 // (2375 with uneven chunks).  Measured before / after, one pass: C6 gradient of
 // 384^3 FP32 665 / 578 us, in-place C8 filter of 256 x 255 x 257 FP64 185 / 176
 // us, C10 gradient of 250 x 199 x 180 FP32 256 / 224 us; 40 Taylor-Green steps
-// at 64^3 FP64 31.9 / 28.7 ms, 120 x 97 x 81 FP32 81.8 / 73.4 ms.
+// at 64^3 FP64 31.9 / 28.7 ms, 120 x 97 x 81 FP32 81.8 / 73.4 ms.  The capacities 12 and 24 (LineDev::cap)
+// between 8, 16 and 32 save the steps and registers of half-empty chunks: C6
+// gradient of 384^3 FP32 (24-point chunks) 384 / 342 us.
 // ---------------------------------------------------------------------------
 // Blocks are dispatched round-robin over the 8 XCDs, each with its own L2;
 // renumbered so that every XCD sweeps one contiguous slab.  For y sweeps, whose
@@ -819,7 +821,7 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
     }
 }
 
-template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V, bool NTS>
+template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V>
 __global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
 k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
            LineFields mf, LineSecond two)
@@ -997,7 +999,7 @@ k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, i
     const double *rv = p.rows64 + rows;
     // the Runge-Kutta epilogues hold three inputs per point: four rows at a
     // time where eight would spill
-    constexpr int NB = (EPI == EPI_LSRK || EPI == EPI_LSRK_DEV) && (CL > 16 || V > 1) ? 4 : 8;
+    constexpr int NB = CL % 8 != 0 || ((EPI == EPI_LSRK || EPI == EPI_LSRK_DEV) && (CL > 16 || V > 1)) ? 4 : 8;
 #pragma unroll
     for (int b = 0; b < CL; b += NB) {
         int64_t o[NB];
@@ -1023,7 +1025,7 @@ k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, i
                 v[j][i] = (T)((double)d[j][t] - acc);
             }
         }
-        epilogue_rows<T, EPI, NB, V, NTS>(e, o, v, ok);
+        epilogue_rows<T, EPI, NB, V, false>(e, o, v, ok);
     }
 }
 
@@ -1389,7 +1391,7 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
 
 // One wave per block, 64/P lines staged in LDS (a pad slot after every XC
 // points keeps the chunk-strided reads conflict-free), so global loads and
-// stores are contiguous.  XC is the chunk capacity (8 or 16).
+// stores are contiguous.  XC is the chunk capacity (8, 12 or 16).
 //
 // Bound: instruction issue before HBM, so every row costs as few instructions
 // as it can.  A line's points are dealt to LPL = 8..64 lanes (the power of two
@@ -1493,7 +1495,7 @@ __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restric
     T *trow = tile + li * TS;
     // slot of window point t (halo included), t = 0 .. XC + 2 M - 1
     auto slot = [&](int t) { return FULL ? k * (XC + 1) + t + t / XC : xw_slot<XC>(s + t); };
-    constexpr int TMIN = XC == 8 ? 1 : XC / 2;
+    constexpr int TMIN = XC <= 12 ? 1 : 8;   // the next smaller capacity is 12 (8 for other plans)
     T d[XC];
     {
         T fv[XC + 2 * M], fe[8];
@@ -1507,7 +1509,7 @@ __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restric
         chunk_rhs<T, M, SYM, XC, FULL, true, TMIN>(pr, fv, fe, k == 0, k == P - 1, len, d);
     }
     // rows per group of per-lane loads: four where two groups of eight spill
-    constexpr int G = !UNIROW && XC > 8 && (Q == 2 || sizeof(T) == 8) ? 4 : 8;
+    constexpr int G = XC == 12 || (!UNIROW && XC > 8 && (Q == 2 || sizeof(T) == 8)) ? 4 : 8;
     const int blk = UNIROW ? cload(p.blk) : p.blk[k];
     solve_padded<T, Q, XC, G>(d, Rows<T, XC, UNIROW>{rowsp<T>(p) + blk});
     double r[2 * Q], tp[Q], hn[Q];
@@ -1521,20 +1523,21 @@ __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restric
     });
     __syncthreads();
     Walk w{0, lsub};
+    constexpr int NB = XC % 8 == 0 ? 8 : 4;
 #pragma unroll
-    for (int b = 0; b < XC; b += 8) {
-        int64_t o[8];
-        T v[1][8];
-        bool ok[8];
+    for (int b = 0; b < XC; b += NB) {
+        int64_t o[NB];
+        T v[1][NB];
+        bool ok[NB];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < NB; i++) {
             const int x = xl + w.q * lpl, xc = x < n ? x : n - 1;
             ok[i] = w.lj < left && x < n;
             o[i] = line_off(w.lj) + xc;
             v[0][i] = tile[(w.lj < nl ? w.lj : 0) * TS + xw_slot<XC>(xc + M)];
             next(w);
         }
-        epilogue_rows<T, EPI, 8, 1, false>(e, o, v, ok);
+        epilogue_rows<T, EPI, NB, 1, false>(e, o, v, ok);
     }
 }
 
@@ -1686,6 +1689,7 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             else go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, false>, XC);
         };
         if (p.cap == 8) pick(std::integral_constant<int, 8>{});
+        else if (p.cap == 12) pick(std::integral_constant<int, 12>{});
         else pick(std::integral_constant<int, XCL>{});
     } else if (dim == 1) {
         const int64_t nlines = v.n[1] * v.n[2];
@@ -1735,12 +1739,6 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         if ((int64_t)(p.n - 1) * sd > INT32_MAX) throw Error{CLES_ERR_UNSUPPORTED, "array too large for 32-bit line offsets"};
         if (nlane >= 48 && 64 * P <= maxNT) {
             const int NT = 64 * P;
-            // The z sweep's plain stores take the non-temporal hint when the launch
-            // writes more than the 256 MB Infinity Cache holds (the outputs are
-            // evicted before they are read again); the x and y sweeps measured
-            // faster without it.
-            const bool nts = dim == 3 && (EPI == EPI_STORE || EPI == EPI_STORE_NEG) &&
-                             (double)v.n[0] * v.n[1] * v.n[2] * sizeof(T) * nf > 256.0 * 1024 * 1024;
             const bool full = p.extra == 0 && p.m == p.cap && (!hp2 || (two.p.extra == 0 && two.p.m == two.p.cap));
             auto go = [&](auto kern, int V) {
                 const int nxb = (int)((nlane + 64 * V - 1) / (64 * V));
@@ -1748,35 +1746,28 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
                 hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf, nz), dim3(NT), shm, st, p, f, (int)sd, so,
                                    (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf, two);
             };
-            auto pick = [&](auto cl, auto vv, auto nt) {
-                if (full) go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, true, vv.value, nt.value>, vv.value);
-                else go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, false, vv.value, nt.value>, vv.value);
+            auto pick = [&](auto cl, auto vv) {
+                if (full) go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, true, vv.value>, vv.value);
+                else go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, false, vv.value>, vv.value);
             };
             using std::integral_constant;
-            auto capd = [&](auto vv, auto nt) {
-                if (p.cap == 8) pick(integral_constant<int, 8>{}, vv, nt);
-                else if (p.cap == 16) pick(integral_constant<int, 16>{}, vv, nt);
-                else pick(integral_constant<int, MC>{}, vv, nt);
+            auto capd = [&](auto vv) {
+                switch (p.cap) {
+                case 8: return pick(integral_constant<int, 8>{}, vv);
+                case 12: return pick(integral_constant<int, 12>{}, vv);
+                case 16: return pick(integral_constant<int, 16>{}, vv);
+                case 24: return pick(integral_constant<int, 24>{}, vv);
+                default: return pick(integral_constant<int, MC>{}, vv);
+                }
             };
             // two lines per lane in FP32 where the launch still has two blocks
             // per CU (the row width must be even)
             bool pairs = false;
-            if constexpr (sizeof(T) == 4 && Q == 1)
+            if constexpr (sizeof(T) == 4 && Q == 1) {
                 pairs = nlane % 2 == 0 && ((nlane + 127) / 128) * nouter * (int64_t)nf * nz >= 512;
-            if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_NEG) {
-                if (nts) {
-                    if constexpr (sizeof(T) == 4 && Q == 1) {
-                        if (pairs) capd(integral_constant<int, 2>{}, std::true_type{});
-                    }
-                    if (!pairs) capd(integral_constant<int, 1>{}, std::true_type{});
-                }
+                if (pairs) capd(integral_constant<int, 2>{});
             }
-            if (!nts) {
-                if constexpr (sizeof(T) == 4 && Q == 1) {
-                    if (pairs) capd(integral_constant<int, 2>{}, std::false_type{});
-                }
-                if (!pairs) capd(integral_constant<int, 1>{}, std::false_type{});
-            }
+            if (!pairs) capd(integral_constant<int, 1>{});
         } else {
             int Lx = 64;
             while (Lx * P > 512 && Lx > 1) Lx /= 2;
@@ -1785,6 +1776,7 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             // rows), until the launch has two blocks per CU
             while (Lx > 8 && ((nlane + Lx - 1) / Lx) * nouter * (int64_t)nf * nz < 512) Lx /= 2;
             if (Lx * P > 512) throw Error{CLES_ERR_UNSUPPORTED, "line too long for the y/z-sweep kernel"};
+            if (p.cap == 12 || p.cap == 24) throw Error{CLES_ERR_INVALID, "plan built for another line kernel"};
             const int NT = Lx * P;
             const int nxb = (int)((nlane + Lx - 1) / Lx);
             const size_t shm = (size_t)2 * B * NT * sizeof(double);

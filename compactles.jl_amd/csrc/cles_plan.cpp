@@ -11,6 +11,7 @@
 //      (src/tridiag.jl:100-124 generalised from a dense LU to a cyclic
 //      reduction whose blocks are fixed by the scheme).
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <sstream>
@@ -21,9 +22,9 @@ namespace cles {
 
 namespace {
 
-using Mat = std::vector<long double>;   // small dense B x B, row-major
+using Mat = std::array<long double, 16>;   // small dense B x B (B <= 4), row-major
 
-Mat mat_zero(int B) { return Mat(B * B, 0.0L); }
+Mat mat_zero(int) { return Mat{}; }
 Mat mat_eye(int B)
 {
     Mat m = mat_zero(B);
@@ -163,7 +164,7 @@ void chunk_solve(const ChunkFactor &F, std::vector<double> &x)
 }  // namespace
 
 void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int periodic, double h, int max_chunk,
-                       int dim, RowPool *pool, int lo_fold, int hi_fold)
+                       int dim, RowPool *pool, int lo_fold, int hi_fold, int64_t lanes)
 {
     const int q = s.q, M = s.M, nc = s.nclosure;
     if (q < 1 || q > 2) throw Error{CLES_ERR_UNSUPPORTED, "scheme LHS half-bandwidth q must be 1 or 2"};
@@ -322,15 +323,16 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     bool decoupled = false;
     for (int st = 0, d = 1; st < nsteps; st++, d *= 2) {
         long double largest = 0.0L;
-        std::vector<Mat> D2(P), L2(P), U2(P);
+        std::vector<Mat> D2(P), L2(P), U2(P), Di(P);
+        for (int k = 0; k < P; k++) Di[k] = k > 0 && D[k] == D[k - 1] ? Di[k - 1] : mat_inv(D[k], B);
         for (int k = 0; k < P; k++) {
             int km = k - d, kp = k + d;
             bool hm = true, hp2 = true;
             if (periodic) { km = ((km % P) + P) % P; kp = kp % P; }
             else { hm = km >= 0; hp2 = kp < P; }
             Mat alpha = mat_zero(B), beta = mat_zero(B);
-            if (hm) alpha = mat_neg(mat_mul(L[k], mat_inv(D[km], B), B));
-            if (hp2) beta = mat_neg(mat_mul(U[k], mat_inv(D[kp], B), B));
+            if (hm) alpha = mat_neg(mat_mul(L[k], Di[km], B));
+            if (hp2) beta = mat_neg(mat_mul(U[k], Di[kp], B));
             Mat Dn = D[k];
             if (hm) Dn = mat_add(Dn, mat_mul(alpha, U[km], B));
             if (hp2) Dn = mat_add(Dn, mat_mul(beta, L[kp], B));
@@ -426,7 +428,13 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
 
     // the distinct chunk blocks, padded to the kernels' capacity
     const int longest = m + (extra ? 1 : 0);
-    const int cap = longest <= 8 && !pool ? 8 : longest <= 16 ? 16 : 32;
+    // the wave-local x sweep and the one-chunk-per-wave y / z sweeps also come in
+    // the capacities 12 and 24 (a sweep runs cap steps however short its chunks); in
+    // x from 16 chunks on, below which a wave stages up to 16 values per lane
+    const bool fine = !pool && (dim == 1 ? P >= 16 && P <= 64 && longest <= 16 : lanes >= 48 && 64 * P <= (q == 1 ? 1024 : 512));
+    int cap = longest <= 8 && !pool ? 8 : longest <= 16 ? 16 : 32;
+    if (fine && cap == 16 && longest <= 12) cap = 12;
+    if (fine && cap == 32 && longest <= 24) cap = 24;
     if (longest > cap) throw Error{CLES_ERR_INVALID, "chunks of more than 32 points"};
     RowPool own;
     RowPool &rp = pool ? *pool : own;
@@ -494,7 +502,7 @@ void build_line_plan(HostPlan &hp, const cles_scheme_desc &s, int n, int periodi
                      int lo_fold, int hi_fold)
 {
     LineTables t;
-    build_line_tables(t, s, n, periodic, h, max_chunk, hp.dim, nullptr, lo_fold, hi_fold);
+    build_line_tables(t, s, n, periodic, h, max_chunk, hp.dim, nullptr, lo_fold, hi_fold, hp.nloc[0]);
     void *d = nullptr;
     CLES_HIP(hipMalloc(&d, t.image.size()));
     hipError_t e = hipMemcpy(d, t.image.data(), t.image.size(), hipMemcpyHostToDevice);
