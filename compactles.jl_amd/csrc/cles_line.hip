@@ -42,7 +42,7 @@ static void launch_typed(const HostPlan &hp, int dim, const View3 &v, const T *f
 
 // The same kernel serves both directions: equal chunk counts and capacities
 // (then also equal block shapes), offsets within the kernels' 32 bits.  Paired
-// only while a launch is short: up to 2^21 points the two save a launch's
+// only while a launch is short: up to 2^20 points the two save a launch's
 // latency (64^3 FP64, 7 us of 604 per step and stage); on larger grids they are
 // bound by bandwidth and sweep better one after the other.
 bool pairable_lines(const HostPlan &a, const HostPlan &b, const View3 &v, int nf)

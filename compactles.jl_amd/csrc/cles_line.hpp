@@ -4,7 +4,7 @@
 // registers: it forms the compact RHS from a register window of f
 // (src/operators.jl:113-174 fill), runs the chunk-local Thomas / banded LU
 // sweeps (src/tridiag.jl:46-57, src/banded.jl:63-80), exchanges its 2q end
-// values with the other chunks of the same line through LDS, solves the
+// values with the other chunks of the same line, solves the
 // reduced interface system by block parallel cyclic reduction (coefficients
 // precomputed by the plan), and applies the spike correction
 // x = y - V tail_prev - W head_next (src/tridiag.jl:159-168,
@@ -12,9 +12,9 @@
 //
 //  * y/z sweeps: 64 (or fewer) consecutive x-lanes per chunk row; every load
 //    and store of a row is a contiguous 512-byte segment; no transposes.
-//  * x sweep: the block stages Lt whole lines in LDS with coalesced loads,
-//    each thread reads its chunk window from LDS, results return through the
-//    same tile for coalesced stores.
+//  * x sweeps: a wave (lines of at most 64 chunks) or a block (longer ones)
+//    stages whole lines in LDS with coalesced loads, each lane reads its chunk
+//    window from LDS, results return through the same tile for coalesced stores.
 // No MFMA: the work is banded and HBM-bound.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -79,16 +79,13 @@ template <typename T, int CAP, bool UNI> struct Rows {
 // ---------------------------------------------------------------------------
 // Epilogues
 // ---------------------------------------------------------------------------
-// NT: plain stores carry the non-temporal hint (a compile-time choice: a
-// run-time branch between two otherwise identical stores is merged into one
-// plain store by the compiler)
-template <typename T, int EPI, bool NT = false>
+template <typename T, int EPI>
 __device__ __forceinline__ void epilogue(const EpiArgs &e, int64_t o, double v)
 {
     if constexpr (EPI == EPI_ART_MULTI) {   // e is the field's own ART_* epilogue (select_field)
-        if (e.kind == EPI_ART_MUBETA) epilogue<T, EPI_ART_MUBETA, NT>(e, o, v);
-        else if (e.kind == EPI_ART_KAPPA) epilogue<T, EPI_ART_KAPPA, NT>(e, o, v);
-        else epilogue<T, EPI_ART_D, NT>(e, o, v);
+        if (e.kind == EPI_ART_MUBETA) epilogue<T, EPI_ART_MUBETA>(e, o, v);
+        else if (e.kind == EPI_ART_KAPPA) epilogue<T, EPI_ART_KAPPA>(e, o, v);
+        else epilogue<T, EPI_ART_D>(e, o, v);
         return;
     }
     // gated kinds: one flag and dt, or (ipts > 0: instances of ipts points side
@@ -99,11 +96,7 @@ __device__ __forceinline__ void epilogue(const EpiArgs &e, int64_t o, double v)
         if (!e.gate[ii]) return;
     }
     if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_GATE || EPI == EPI_STORE_NEG) {
-        const T val = EPI == EPI_STORE_NEG ? (T)(-v) : (T)v;
-        if constexpr (NT)
-            __builtin_nontemporal_store(val, (T *)e.out + o);
-        else
-            ((T *)e.out)[o] = val;
+        ((T *)e.out)[o] = EPI == EPI_STORE_NEG ? (T)(-v) : (T)v;
     } else if constexpr (EPI == EPI_SUB) {
         T *out = (T *)e.out;
         out[o] = out[o] - (T)v;
@@ -142,14 +135,14 @@ __device__ __forceinline__ void epilogue(const EpiArgs &e, int64_t o, double v)
 // Batched epilogue: every input of NB points is loaded before any output is
 // stored, so the loads of a batch are in flight together (the compiler cannot
 // reorder them across stores through pointers that may alias).
-template <typename T, int EPI, int NB, bool NT = false>
+template <typename T, int EPI, int NB>
 __device__ __forceinline__ void epilogue_batch(const EpiArgs &e, const int64_t (&o)[NB], const T (&v)[NB],
                                                const bool (&ok)[NB])
 {
     if constexpr (EPI == EPI_ART_MULTI) {
-        if (e.kind == EPI_ART_MUBETA) epilogue_batch<T, EPI_ART_MUBETA, NB, NT>(e, o, v, ok);
-        else if (e.kind == EPI_ART_KAPPA) epilogue_batch<T, EPI_ART_KAPPA, NB, NT>(e, o, v, ok);
-        else epilogue_batch<T, EPI_ART_D, NB, NT>(e, o, v, ok);
+        if (e.kind == EPI_ART_MUBETA) epilogue_batch<T, EPI_ART_MUBETA, NB>(e, o, v, ok);
+        else if (e.kind == EPI_ART_KAPPA) epilogue_batch<T, EPI_ART_KAPPA, NB>(e, o, v, ok);
+        else epilogue_batch<T, EPI_ART_D, NB>(e, o, v, ok);
         return;
     }
     // gated kinds: one flag and dt for the launch, or (ipts > 0) those of
@@ -182,7 +175,7 @@ __device__ __forceinline__ void epilogue_batch(const EpiArgs &e, const int64_t (
         constexpr int E1 = EPI == EPI_STORE_GATE ? (int)EPI_STORE : EPI;   // the gate is applied
 #pragma unroll
         for (int i = 0; i < NB; i++)
-            if (okk[i]) epilogue<T, E1, NT>(e, o[i], (double)v[i]);
+            if (okk[i]) epilogue<T, E1>(e, o[i], (double)v[i]);
     } else if constexpr (EPI == EPI_SUB) {
         T *out = (T *)e.out;
         T a[NB];
@@ -651,9 +644,10 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
 // (2375 with uneven chunks).  Measured before / after, one pass: C6 gradient of
 // 384^3 FP32 665 / 578 us, in-place C8 filter of 256 x 255 x 257 FP64 185 / 176
 // us, C10 gradient of 250 x 199 x 180 FP32 256 / 224 us; 40 Taylor-Green steps
-// at 64^3 FP64 31.9 / 28.7 ms, 120 x 97 x 81 FP32 81.8 / 73.4 ms.  The capacities 12 and 24 (LineDev::cap)
-// between 8, 16 and 32 save the steps and registers of half-empty chunks: C6
-// gradient of 384^3 FP32 (24-point chunks) 384 / 342 us.
+// at 64^3 FP64 31.9 / 28.7 ms, 120 x 97 x 81 FP32 81.8 / 73.4 ms.  The
+// capacities 12 and 24 (LineDev::cap) between 8, 16 and 32 save the steps and
+// registers of half-empty chunks: C6 gradient of 384^3 FP32 (24-point chunks)
+// 384 / 342 us.
 // ---------------------------------------------------------------------------
 // Blocks are dispatched round-robin over the 8 XCDs, each with its own L2;
 // renumbered so that every XCD sweeps one contiguous slab.  For y sweeps, whose
@@ -682,31 +676,29 @@ template <int V, typename T> __device__ __forceinline__ void vload(const T *ptr,
         for (int i = 0; i < V; i++) v[i] = x[i];
     }
 }
-template <int V, bool NT, typename T> __device__ __forceinline__ void vstore(T *ptr, const T (&v)[V])
+template <int V, typename T> __device__ __forceinline__ void vstore(T *ptr, const T (&v)[V])
 {
     if constexpr (V == 1) {
-        if constexpr (NT) __builtin_nontemporal_store(v[0], ptr);
-        else *ptr = v[0];
+        *ptr = v[0];
     } else {
         typename Pack<T, V>::type x;
 #pragma unroll
         for (int i = 0; i < V; i++) x[i] = v[i];
-        if constexpr (NT) __builtin_nontemporal_store(x, (typename Pack<T, V>::type *)ptr);
-        else *(typename Pack<T, V>::type *)ptr = x;
+        *(typename Pack<T, V>::type *)ptr = x;
     }
 }
 
 // The epilogue of NB rows of V adjacent points: element o[i] .. o[i] + V - 1
 // takes v[.][i].  Every input is loaded before any output is stored.  Row i is
 // stored where ok[i] (wave-uniform); the offsets of other rows are in bounds.
-template <typename T, int EPI, int NB, int V, bool NT>
+template <typename T, int EPI, int NB, int V>
 __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&o)[NB], const T (&v)[V][NB],
                                               const bool (&ok)[NB])
 {
     if constexpr (EPI == EPI_ART_MULTI) {
-        if (e.kind == EPI_ART_MUBETA) epilogue_rows<T, EPI_ART_MUBETA, NB, V, NT>(e, o, v, ok);
-        else if (e.kind == EPI_ART_KAPPA) epilogue_rows<T, EPI_ART_KAPPA, NB, V, NT>(e, o, v, ok);
-        else epilogue_rows<T, EPI_ART_D, NB, V, NT>(e, o, v, ok);
+        if (e.kind == EPI_ART_MUBETA) epilogue_rows<T, EPI_ART_MUBETA, NB, V>(e, o, v, ok);
+        else if (e.kind == EPI_ART_KAPPA) epilogue_rows<T, EPI_ART_KAPPA, NB, V>(e, o, v, ok);
+        else epilogue_rows<T, EPI_ART_D, NB, V>(e, o, v, ok);
         return;
     }
     if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_NEG) {
@@ -716,7 +708,7 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
             T x[V];
 #pragma unroll
             for (int j = 0; j < V; j++) x[j] = EPI == EPI_STORE_NEG ? -v[j][i] : v[j][i];
-            vstore<V, NT>((T *)e.out + o[i], x);
+            vstore<V>((T *)e.out + o[i], x);
         }
     } else if constexpr (EPI == EPI_SUB) {
         T a[NB][V];
@@ -727,7 +719,7 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
             if (!ok[i]) continue;
 #pragma unroll
             for (int j = 0; j < V; j++) a[i][j] = a[i][j] - v[j][i];
-            vstore<V, false>((T *)e.out + o[i], a[i]);
+            vstore<V>((T *)e.out + o[i], a[i]);
         }
     } else if constexpr (EPI == EPI_LSRK) {
         const T *acc = (const T *)e.a0;
@@ -753,8 +745,8 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
                 du[i][j] = fma(e.dt, dq, e.c0 * du[i][j]);
                 q[i][j] = fma(e.c1, du[i][j], q[i][j]);
             }
-            vstore<V, false>(e.du + o[i], du[i]);
-            vstore<V, false>(e.Q + o[i], q[i]);
+            vstore<V>(e.du + o[i], du[i]);
+            vstore<V>(e.Q + o[i], q[i]);
         }
     } else if constexpr (EPI == EPI_ART_MUBETA) {
         T r[NB][V];
@@ -770,8 +762,8 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
                 mu[j] = (T)e.c0 * rs;
                 be[j] = (T)e.c1 * rs;
             }
-            vstore<V, false>((T *)e.out + o[i], mu);
-            vstore<V, false>((T *)e.out2 + o[i], be);
+            vstore<V>((T *)e.out + o[i], mu);
+            vstore<V>((T *)e.out2 + o[i], be);
         }
     } else if constexpr (EPI == EPI_ART_KAPPA) {
         T r[NB][V], cc[NB][V], tt[NB][V];
@@ -791,7 +783,7 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
                 const T scale = r[i][j] * cc[i][j] / (tt[i][j] > eps ? tt[i][j] : eps);
                 ka[j] = (T)e.c0 * scale * (v[j][i] > T(0) ? v[j][i] : T(0));
             }
-            vstore<V, false>((T *)e.out + o[i], ka);
+            vstore<V>((T *)e.out + o[i], ka);
         }
     } else if constexpr (EPI == EPI_ART_D) {
         T cc[NB][V];
@@ -803,7 +795,7 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
             T dd[V];
 #pragma unroll
             for (int j = 0; j < V; j++) dd[j] = (T)e.c0 * cc[i][j] * (v[j][i] > T(0) ? v[j][i] : T(0));
-            vstore<V, false>((T *)e.out + o[i], dd);
+            vstore<V>((T *)e.out + o[i], dd);
         }
     } else {
         // gated kinds: the flag and dt of the launch, or of each point's instance
@@ -816,7 +808,7 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
                 oj[i] = o[i] + j;
                 vj[i] = v[j][i];
             }
-            epilogue_batch<T, EPI, NB, false>(e, oj, vj, ok);
+            epilogue_batch<T, EPI, NB>(e, oj, vj, ok);
         }
     }
 }
@@ -1025,7 +1017,7 @@ k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, i
                 v[j][i] = (T)((double)d[j][t] - acc);
             }
         }
-        epilogue_rows<T, EPI, NB, V, false>(e, o, v, ok);
+        epilogue_rows<T, EPI, NB, V>(e, o, v, ok);
     }
 }
 
@@ -1120,7 +1112,7 @@ __global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p1, const T *__restr
             o[i] = off + (int64_t)(ok[i] ? s + b + i : s) * sd;
             v[0][i] = d[b + i];
         }
-        epilogue_rows<T, EPI, NB, 1, false>(e, o, v, ok);
+        epilogue_rows<T, EPI, NB, 1>(e, o, v, ok);
     }
 }
 
@@ -1237,7 +1229,7 @@ k_line_x(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz, int ny, int
             v[0][i] = tile[(w.lj < Lt ? w.lj : 0) * TS + xw_slot<CL>(xc + M)];
             next(w);
         }
-        epilogue_rows<T, EPI, 8, 1, false>(e, o, v, ok);
+        epilogue_rows<T, EPI, 8, 1>(e, o, v, ok);
     }
 }
 
@@ -1537,7 +1529,7 @@ __global__ void __launch_bounds__(64, 4) k_line_xw(LineDev p, const T *__restric
             v[0][i] = tile[(w.lj < nl ? w.lj : 0) * TS + xw_slot<XC>(xc + M)];
             next(w);
         }
-        epilogue_rows<T, EPI, NB, 1, false>(e, o, v, ok);
+        epilogue_rows<T, EPI, NB, 1>(e, o, v, ok);
     }
 }
 

@@ -23,8 +23,9 @@ __device__ __forceinline__ unsigned rag_block(unsigned b, unsigned nb)
     return b < nfull ? (b & 7u) * (nfull >> 3) + (b >> 3) : b;
 }
 
-// One launch for both classes up to this many blocks (waves), twice what the
-// long class's registers let run at once: 512 tubes FP64, 1392 to 2784 blocks
+// One launch for both classes up to this many blocks (waves), four times what
+// the long class's registers let run at once (from there on the two launches
+// fill the card by themselves and the results are equal): 512 tubes FP64, 1392 to 2784 blocks
 // per launch, 131.0 ms per 96 steps with two launches and 105.8 with one for up
 // to 2048 blocks; 1024 tubes 1.76 / 1.73 ms per step, 4096 tubes 6.34 / 6.36.
 constexpr int64_t RAG_BOTH_BLOCKS = 8192;
@@ -146,7 +147,7 @@ __device__ __forceinline__ void rag_item(const RagLines &r, unsigned logical, co
                 o[i] = oj + (ok[i] ? x : 0);
                 v[0][i] = row[xw_slot<CL>((ok[i] ? x : 0) + M)];
             }
-            epilogue_rows<T, EPI, NB, 1, false>(ej, o, v, ok);
+            epilogue_rows<T, EPI, NB, 1>(ej, o, v, ok);
         }
     }
 }

@@ -316,6 +316,8 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     // what it leaves out is at most 1e-20 of the line's largest interface
     // value, four decades below half an ulp of it.  The step it saves costs an
     // exchange through LDS (or shuffles) on the critical path of every kernel.
+    // (A NaN or an infinity in a line therefore reaches the chunks within the
+    // kept steps' reach, not always the whole line.)
     constexpr long double PCR_DROP = 1e-20L;
     std::vector<Mat> D(P, mat_eye(B)), L = Lb, U = Ub;
     std::vector<double> pcr;
