@@ -1061,12 +1061,14 @@ __global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p1, const T *__restr
     // lanes of one wave own different chunks, so branching per load
     // would diverge: every load is unconditional, from the wrapped row
     // clamped into the line (and the last lane of the row set for lanes
-    // past it), and its value selected afterwards
+    // past it), and its value selected afterwards.  Rows of the line past the
+    // chunk's own window stay: the low closure reads up to eight points from
+    // the edge, however short the first chunk is
     const T *fa = f + (int64_t)(valid ? xi : nlane - 1) + ob * so;
 #pragma unroll
     for (int t = -M; t < CL + M; t++) {
         int r = s + t;
-        bool ok = valid && t < len + M;
+        bool ok = valid;
         if (r < 0) {
             ok = ok && p.periodic;
             r += n;

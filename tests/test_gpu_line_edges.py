@@ -127,3 +127,49 @@ def test_paired_gradients(ctx, n, species):  # noqa: F811
             name = f"grad_u[{d}{j}]"
             assert Hh.relerr(gs.field(name), os_.interior(os_.field(name))) <= 1e-12, name
     gs.close()
+
+
+def _dense(scheme, n, h):
+    """The operator of a closed derivative scheme on n points as a dense matrix:
+    the left-hand band and the right-hand rows, solved together."""
+    q = getattr(scheme, "q", 1)
+    lhs = scheme.lhs if q == 2 else [scheme.alpha]
+    A, B = np.eye(n), np.zeros((n, n))
+    nc = len(scheme.closures)
+    for i in range(nc, n - nc):
+        for s, a in enumerate(lhs, 1):
+            A[i, i - s] = A[i, i + s] = a
+        for m, c in enumerate(scheme.coeffs, 1):
+            B[i, i + m], B[i, i - m] = c, -c
+    for j, row in enumerate(scheme.closures):
+        for s in range(-q, q + 1):
+            if 0 <= j + s < n:
+                A[j, j + s] = A[n - 1 - j, n - 1 - j - s] = row.lhs[q + s]
+        for t, w in enumerate(row.rhs):
+            B[j, t], B[n - 1 - j, n - 1 - t] = w, -w
+    return np.linalg.solve(A, B / h)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("half", [1, 2])
+@pytest.mark.parametrize("lanes", [6, 50])
+def test_long_closures_on_short_chunks(ctx, half, lanes, dtype, bar):  # noqa: F811
+    """Closure rows of eight weights reach past the first chunk (four or five
+    points on lines of 17 to 20 and 33 to 40) and, for these stencils, past its
+    window; every direction, against a dense solve."""
+    import compactles_hip as ch
+    g = np.random.default_rng(8)
+    base = ch.pade_d1_4() if half == 1 else ch.lele_d1_6()
+    rows = [ch.ClosureRow(lhs, list(g.uniform(-1, 1, 8))) for lhs in ((0.0, 1.0, 0.5), (0.25, 1.0, 0.25))]
+    scheme = ch.CompactScheme("long closures", base.alpha, 0.0, base.coeffs, False, rows)
+    for line in (9, 16, 17, 18, 19, 20, 33, 36, 39, 40):
+        D = _dense(scheme, line, 0.1)
+        for dim in (1, 2, 3):
+            n = {1: (line, lanes, 2), 2: (lanes, line, 3), 3: (lanes, 2, line)}[dim]
+            f = Hh.random_field(n, seed=71).astype(dtype).astype(np.float64)
+            dec = ch.Decomp(n, (False,) * 3)
+            plan = ch.plan_direction(ctx, dec, scheme, dim, 0.1, dtype=dtype)
+            out = ch.field(ctx, dec, dtype)
+            ch.apply_along_(out, plan, ch.DeviceArray.from_numpy(ctx, Hh.pad(f, n), dtype), dec)
+            ref = np.moveaxis(np.tensordot(D, f, (1, dim - 1)), 0, dim - 1)
+            assert Hh.relerr(Hh.interior(out.numpy().astype(np.float64), n), ref) <= bar, (line, dim)
