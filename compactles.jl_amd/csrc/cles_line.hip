@@ -48,7 +48,7 @@ static void launch_typed(const HostPlan &hp, int dim, const View3 &v, const T *f
 bool pairable_lines(const HostPlan &a, const HostPlan &b, const View3 &v, int nf)
 {
     const LineDev &p = a.dev, &q = b.dev;
-    return a.dtype == b.dtype && p.P == q.P && p.cap == q.cap && p.q == q.q && p.M == q.M && p.sym == q.sym &&
+    return a.dtype == b.dtype && p.P == q.P && p.cap == q.cap && p.q == q.q && p.M == q.M && !p.sym && !q.sym &&
            2 * nf <= LINE_MF && v.n[0] * v.n[1] * v.n[2] <= PAIR_POINTS && (int64_t)(p.n - 1) * v.s[1] <= INT32_MAX &&
            (int64_t)(q.n - 1) * v.s[2] <= INT32_MAX;
 }

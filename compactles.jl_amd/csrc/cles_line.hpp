@@ -243,12 +243,12 @@ __device__ __forceinline__ void epilogue_batch(const EpiArgs &e, const int64_t (
 
 // Field of a multi-field launch (grid y): field 0 keeps the launch's own input
 // and epilogue, field i >= 1 takes its input and output from the table.
-template <typename T, int EPI>
+// PAIR: grid z = 1 is the second direction of a paired launch, whose fields
+// follow the first direction's in the table.
+template <typename T, int EPI, bool PAIR = false>
 __device__ __forceinline__ void select_field(const LineFields &mf, const T *__restrict__ &f, EpiArgs &e)
 {
-    // grid z = 1: the second direction of a paired launch, whose outputs follow
-    // the first direction's in the table (its inputs are the same fields)
-    const int i = EPI == EPI_STORE ? blockIdx.y + gridDim.y * blockIdx.z : blockIdx.y;
+    const int i = PAIR ? blockIdx.y + gridDim.y * blockIdx.z : blockIdx.y;
     if constexpr (EPI == EPI_ART_MULTI) e = e.multi[i];
     if (i == 0) return;
     f = (const T *)mf.in[i];
@@ -813,29 +813,14 @@ __device__ __forceinline__ void epilogue_rows(const EpiArgs &e, const int64_t (&
     }
 }
 
+//
+// One block; nb: the blocks of its direction.
 template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V>
-__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
-k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
-           LineFields mf, LineSecond two)
+__device__ __forceinline__ void line_yzu(const LineDev &p, const T *__restrict__ f, int sd, int64_t so, int nlane,
+                                         int nxb, int slabs, unsigned nb, const EpiArgs &e)
 {
-    select_field<T, EPI>(mf, f, e);
     extern __shared__ double smem[];
     constexpr int B = 2 * Q;
-    const bool second = EPI == EPI_STORE && blockIdx.z;
-    LineDev p = p1;
-    unsigned nb = gridDim.x;
-    if constexpr (EPI == EPI_STORE) {
-        if (gridDim.z > 1) {   // the two directions may differ in lines, hence in blocks
-            nb = (unsigned)nxb * (unsigned)(second ? two.nouter : two.nouter1);
-            if (second) {
-                p = two.p;
-                sd = two.sd;
-                so = two.so;
-                slabs = two.slabs;
-            }
-            if (blockIdx.x >= nb) return;
-        }
-    }
     const int P = p.P, n = p.n;
     const int NT = 64 * P;
     const int lane = (int)(threadIdx.x & 63);
@@ -1021,6 +1006,39 @@ k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, i
     }
 }
 
+template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V>
+__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
+k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
+           LineFields mf)
+{
+    select_field<T, EPI>(mf, f, e);
+    line_yzu<T, Q, M, SYM, EPI, CL, FULL, V>(p, f, sd, so, nlane, nxb, slabs, gridDim.x, e);
+}
+
+// The y (grid z = 0) and z (1) directions in one launch, store epilogue.  A
+// kernel of its own, so that plain launches carry neither the second plan's
+// arguments nor the choice between the plans (C6 gradient of 33 x 29 x 31 FP64,
+// three plain launches: 21.2 us a pass with one kernel for both, 20.5 so).
+template <typename T, int Q, int M, int SYM, int CL, bool FULL, int V>
+__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
+k_line_yzu_pair(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
+                LineFields mf, LineSecond two)
+{
+    select_field<T, EPI_STORE, true>(mf, f, e);
+    const bool second = blockIdx.z;
+    // the two directions may differ in lines, hence in blocks
+    const unsigned nb = (unsigned)nxb * (unsigned)(second ? two.nouter : two.nouter1);
+    if (blockIdx.x >= nb) return;
+    LineDev p = p1;
+    if (second) {
+        p = two.p;
+        sd = two.sd;
+        so = two.so;
+        slabs = two.slabs;
+    }
+    line_yzu<T, Q, M, SYM, EPI_STORE, CL, FULL, V>(p, f, sd, so, nlane, nxb, slabs, nb, e);
+}
+
 // ---------------------------------------------------------------------------
 // y / z sweeps on narrow blocks: lanes along x.
 // Line dimension stride sd, outer dimension stride so; block = Lx lanes x P
@@ -1028,22 +1046,9 @@ k_line_yzu(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, i
 // with too many chunks for 64 lanes.
 // ---------------------------------------------------------------------------
 template <typename T, int Q, int M, int SYM, int EPI, int CL>
-__global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p1, const T *__restrict__ f, int sd, int64_t so,
-                                                  int nlane, int nxb, int Lx, EpiArgs e, LineFields mf, LineSecond two)
+__device__ __forceinline__ void line_yz(const LineDev &p, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb,
+                                        int Lx, const EpiArgs &e)
 {
-    select_field<T, EPI>(mf, f, e);
-    const bool second = EPI == EPI_STORE && blockIdx.z;
-    LineDev p = p1;
-    if constexpr (EPI == EPI_STORE) {
-        if (gridDim.z > 1) {
-            if (second) {
-                p = two.p;
-                sd = two.sd;
-                so = two.so;
-            }
-            if (blockIdx.x >= (unsigned)nxb * (unsigned)(second ? two.nouter : two.nouter1)) return;
-        }
-    }
     extern __shared__ double smem[];
     const int NT = Lx * p.P;
     const int lane = (int)(threadIdx.x % Lx);
@@ -1116,6 +1121,32 @@ __global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p1, const T *__restr
         }
         epilogue_rows<T, EPI, NB, 1>(e, o, v, ok);
     }
+}
+
+template <typename T, int Q, int M, int SYM, int EPI, int CL>
+__global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane,
+                                                    int nxb, int Lx, EpiArgs e, LineFields mf)
+{
+    select_field<T, EPI>(mf, f, e);
+    line_yz<T, Q, M, SYM, EPI, CL>(p, f, sd, so, nlane, nxb, Lx, e);
+}
+
+// The y and z directions in one launch, as k_line_yzu_pair.
+template <typename T, int Q, int M, int SYM, int CL>
+__global__ void __launch_bounds__(512, 3) k_line_yz_pair(LineDev p1, const T *__restrict__ f, int sd, int64_t so,
+                                                         int nlane, int nxb, int Lx, EpiArgs e, LineFields mf,
+                                                         LineSecond two)
+{
+    select_field<T, EPI_STORE, true>(mf, f, e);
+    const bool second = blockIdx.z;
+    if (blockIdx.x >= (unsigned)nxb * (unsigned)(second ? two.nouter : two.nouter1)) return;
+    LineDev p = p1;
+    if (second) {
+        p = two.p;
+        sd = two.sd;
+        so = two.so;
+    }
+    line_yz<T, Q, M, SYM, EPI_STORE, CL>(p, f, sd, so, nlane, nxb, Lx, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -1734,13 +1765,17 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         if (nlane >= 48 && 64 * P <= maxNT) {
             const int NT = 64 * P;
             const bool full = p.extra == 0 && p.m == p.cap && (!hp2 || (two.p.extra == 0 && two.p.m == two.p.cap));
-            auto go = [&](auto kern, int V) {
+            auto go = [&](auto kern, int V, auto... second) {
                 const int nxb = (int)((nlane + 64 * V - 1) / (64 * V));
                 const size_t shm = (size_t)2 * B * NT * V * sizeof(double);
                 hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf, nz), dim3(NT), shm, st, p, f, (int)sd, so,
-                                   (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf, two);
+                                   (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf, second...);
             };
             auto pick = [&](auto cl, auto vv) {
+                if constexpr (EPI == EPI_STORE && !SYM) {
+                    if (hp2 && full) return go(k_line_yzu_pair<T, Q, M, SYM, cl.value, true, vv.value>, vv.value, two);
+                    if (hp2) return go(k_line_yzu_pair<T, Q, M, SYM, cl.value, false, vv.value>, vv.value, two);
+                }
                 if (full) go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, true, vv.value>, vv.value);
                 else go(k_line_yzu<T, Q, M, SYM, EPI, cl.value, false, vv.value>, vv.value);
             };
@@ -1774,15 +1809,19 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             const int NT = Lx * P;
             const int nxb = (int)((nlane + Lx - 1) / Lx);
             const size_t shm = (size_t)2 * B * NT * sizeof(double);
-            if (p.cap == 8)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 8>), dim3((unsigned)(nxb * nouter), nf, nz),
-                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf, two);
-            else if (p.cap == 16)
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, 16>), dim3((unsigned)(nxb * nouter), nf, nz),
-                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf, two);
-            else
-                hipLaunchKernelGGL((k_line_yz<T, Q, M, SYM, EPI, MC>), dim3((unsigned)(nxb * nouter), nf, nz),
-                                   dim3(NT), shm, st, p, f, (int)sd, so, (int)nlane, nxb, Lx, e, mf, two);
+            auto go = [&](auto kern, auto... second) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf, nz), dim3(NT), shm, st, p, f, (int)sd, so,
+                                   (int)nlane, nxb, Lx, e, mf, second...);
+            };
+            auto pick = [&](auto cl) {
+                if constexpr (EPI == EPI_STORE && !SYM) {
+                    if (hp2) return go(k_line_yz_pair<T, Q, M, SYM, cl.value>, two);
+                }
+                go(k_line_yz<T, Q, M, SYM, EPI, cl.value>);
+            };
+            if (p.cap == 8) pick(std::integral_constant<int, 8>{});
+            else if (p.cap == 16) pick(std::integral_constant<int, 16>{});
+            else pick(std::integral_constant<int, MC>{});
         }
     }
     CLES_HIP(hipGetLastError());
