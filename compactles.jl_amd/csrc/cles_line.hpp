@@ -489,9 +489,20 @@ __device__ __forceinline__ void correct_padded(T (&d)[CL], R64 R, const double (
 // latency overlaps the exchange; for per-lane chunk indices (the x sweep).
 // UNI: k is wave-uniform (scalar loads).  The blocks of inner chunks are the
 // same block of the table (LineDev::pcr), so the lanes of a wave read a few.
+//
+// The plan leaves out steps whose coefficients are below rounding, but a NaN or
+// an infinity still has to reach its whole line: a chunk whose values are not
+// finite (they reach its ends, and z[0] sums every end value) raises its line's
+// flag (*bad, which every thread cleared before the first step's barrier: a line
+// of several chunks takes one step at least), and a raised flag makes the line
+// NaN; bad[64] takes what the others write.  No branch, and nothing kept in
+// registers for it: flags per wave and a branch to look for the line cost the
+// y / z sweeps a block per CU (C6 derivative of 160^3 FP32 11.8 / 16.0 us).
+constexpr int XCH_FLAGS = 64;   // doubles of flags before a block's exchange buffers
+
 template <int Q, bool PF = false, bool UNI = false>
 __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int NT, int nl, int k, int li,
-                                              double (&r)[2 * Q], double (&tp)[Q], double (&hn)[Q])
+                                              double (&r)[2 * Q], double (&tp)[Q], double (&hn)[Q], int *bad)
 {
     constexpr int B = 2 * Q;
     const int P = p.P;
@@ -606,6 +617,7 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
     double *bf = buf + (p.nsteps & 1) * B * NT;
 #pragma unroll
     for (int c = 0; c < B; c++) bf[c * NT + slot] = z[c];
+    bad[__builtin_isfinite(z[0]) ? 64 : 0] = 1;
     __syncthreads();
     int kprev = k - 1, knext = k + 1;
     bool hasp = true, hasn = true;
@@ -621,6 +633,7 @@ __device__ __forceinline__ void reduced_solve(const LineDev &p, double *buf, int
         tp[i] = hasp ? bf[(Q + i) * NT + kprev * nl + li] : 0.0;
         hn[i] = hasn ? bf[i * NT + knext * nl + li] : 0.0;
     }
+    tp[0] = *bad ? (double)__builtin_nanf("") : tp[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -824,6 +837,8 @@ __device__ __forceinline__ void line_yzu(const LineDev &p, const T *__restrict__
     const int P = p.P, n = p.n;
     const int NT = 64 * P;
     const int lane = (int)(threadIdx.x & 63);
+#pragma unroll
+    for (int j = 0; j < V; j++) ((int *)(smem + XCH_FLAGS * j))[lane] = 0;
     const int k = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned blk = slabs ? xcd_slab(blockIdx.x, nb) : blockIdx.x;
     const int xb = blk % nxb;
@@ -949,7 +964,7 @@ __device__ __forceinline__ void line_yzu(const LineDev &p, const T *__restrict__
             }
     }
 
-    // the reduced system, each of the V lines in its own part of the buffers
+    // the reduced system, each of the V lines in its own part of the flags and buffers
     double tp[V][Q], hn[V][Q];
 #pragma unroll
     for (int j = 0; j < V; j++) {
@@ -968,7 +983,8 @@ __device__ __forceinline__ void line_yzu(const LineDev &p, const T *__restrict__
                 r[Q + i] = (double)x;
             }
         }
-        reduced_solve<Q, false, true>(p, smem + (size_t)j * 2 * B * NT, NT, 64, k, lane, r, tp[j], hn[j]);
+        reduced_solve<Q, false, true>(p, smem + XCH_FLAGS * V + (size_t)j * 2 * B * NT, NT, 64, k, lane, r, tp[j],
+                                      hn[j], (int *)(smem + XCH_FLAGS * j) + lane);
     }
     if (!valid) return;
 
@@ -1006,8 +1022,18 @@ __device__ __forceinline__ void line_yzu(const LineDev &p, const T *__restrict__
     }
 }
 
+// Waves per SIMD that a variant is held to: those of uneven 24-point chunks lie
+// at 78 to 84 registers, and 80 still let a CU take three blocks instead of two
+// (C4 derivative of 192^3 FP64: 20.0 us at 79, 22.9 at 81).
+template <typename T, int Q, int M, int EPI, int CL, bool FULL, int V> constexpr int yzu_waves()
+{
+    constexpr bool store24 = CL == 24 && !FULL && (EPI == EPI_STORE || EPI == EPI_STORE_NEG);
+    if (Q == 2) return store24 ? 6 : 4;
+    return store24 && M <= 2 && sizeof(T) * V == 8 ? 6 : 1;
+}
+
 template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V>
-__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
+__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, (yzu_waves<T, Q, M, EPI, CL, FULL, V>()))
 k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
            LineFields mf)
 {
@@ -1020,7 +1046,7 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
 // arguments nor the choice between the plans (C6 gradient of 33 x 29 x 31 FP64,
 // three plain launches: 21.2 us a pass with one kernel for both, 20.5 so).
 template <typename T, int Q, int M, int SYM, int CL, bool FULL, int V>
-__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, Q == 2 ? 4 : 1)
+__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, (yzu_waves<T, Q, M, EPI_STORE, CL, FULL, V>()))
 k_line_yzu_pair(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
                 LineFields mf, LineSecond two)
 {
@@ -1053,6 +1079,7 @@ __device__ __forceinline__ void line_yz(const LineDev &p, const T *__restrict__ 
     const int NT = Lx * p.P;
     const int lane = (int)(threadIdx.x % Lx);
     const int k = (int)(threadIdx.x / Lx);
+    ((int *)smem)[lane] = 0;
     const int xb = blockIdx.x % nxb;
     const int64_t ob = blockIdx.x / nxb;
     const int xi = xb * Lx + lane;
@@ -1102,7 +1129,7 @@ __device__ __forceinline__ void line_yz(const LineDev &p, const T *__restrict__ 
     solve_padded<T, Q, CL, G>(d, Rows<T, CL, false>{rowsp<T>(p) + blk});
     double r[2 * Q], tp[Q], hn[Q];
     chunk_ends<T, Q, CL, false, TMIN>(d, len, r);
-    reduced_solve<Q, Q == 1 && sizeof(T) == 8>(p, smem, NT, Lx, k, lane, r, tp, hn);
+    reduced_solve<Q, Q == 1 && sizeof(T) == 8>(p, smem + XCH_FLAGS, NT, Lx, k, lane, r, tp, hn, (int *)smem + lane);
     if (!valid) return;
     correct_padded<T, Q, CL, G>(d, Rows<double, CL, false>{p.rows64 + blk}, tp, hn, [](int, T) {});
     // the device-dt LSRK epilogue (per-point gate and dt beside three
@@ -1162,7 +1189,7 @@ __global__ void __launch_bounds__(512, 3) k_line_yz_pair(LineDev p1, const T *__
 template <int XC> __device__ __forceinline__ int xw_slot(int x) { return x + x / XC; }
 
 template <typename T, int Q, int M, int SYM, int EPI, int CL>
-__global__ void __launch_bounds__(512, CL <= 8 && Q == 1 ? 4 : 1)
+__global__ void __launch_bounds__(512, CL <= 8 ? 4 : 1)
 k_line_x(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz, int ny, int64_t nlines, int Lt, int TS, bool overlay,
          EpiArgs e, LineFields mf)
 {
@@ -1241,7 +1268,8 @@ k_line_x(LineDev p, const T *__restrict__ f, int64_t sy, int64_t sz, int ny, int
     double r[2 * Q], tp[Q], hn[Q];
     chunk_ends<T, Q, CL, false, TMIN>(d, len, r);
     if (overlay) __syncthreads();
-    reduced_solve<Q, Q == 1>(p, buf, NT, Lt, k, li, r, tp, hn);
+    ((int *)buf)[li] = 0;
+    reduced_solve<Q, Q == 1>(p, buf + XCH_FLAGS, NT, Lt, k, li, r, tp, hn, (int *)buf + li);
     // every thread has finished reading the tile before the reduced solve's barrier
     if (overlay) __syncthreads();
     correct_padded<T, Q, CL, G>(d, Rows<double, CL, false>{p.rows64 + blk}, tp, hn, [&](int t, T v) {
@@ -1412,6 +1440,9 @@ __device__ __forceinline__ void reduced_solve_wave(const LineDev &p, int k, int 
         tp[i] = hasp ? a : 0.0;
         hn[i] = hasn ? b : 0.0;
     }
+    // a NaN or an infinity reaches its whole line (see reduced_solve)
+    const uint64_t bad = (uint64_t)__ballot(!__builtin_isfinite(z[0]));
+    if (bad && (bad >> base & (~(uint64_t)0 >> (64 - P)))) tp[0] = __builtin_nan("");
 }
 
 // One wave per block, 64/P lines staged in LDS (a pad slot after every XC
@@ -1682,7 +1713,6 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
     const LineDev &p = hp.dev;
 
     const int P = p.P;
-    const int B = 2 * Q;
     const size_t lim = lds_limit();
     const int maxNT = Q == 1 ? 1024 : 512;
     if (dim == 1 && p.extra == 0 && p.m == XCL && P == 16 && p.periodic) {
@@ -1722,7 +1752,7 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         const int TS = y + y / p.cap + 1;
         auto shm_of = [&](int Lt, bool over = false) {
             const size_t tile = (((size_t)Lt * TS * sizeof(T) + 7) / 8) * 8;
-            const size_t bufs = (size_t)2 * B * Lt * P * sizeof(double);
+            const size_t bufs = ((size_t)4 * Q * Lt * P + XCH_FLAGS) * sizeof(double);
             return over ? std::max(tile, bufs) : tile + bufs;
         };
         int Lt = 1;
@@ -1767,7 +1797,8 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             const bool full = p.extra == 0 && p.m == p.cap && (!hp2 || (two.p.extra == 0 && two.p.m == two.p.cap));
             auto go = [&](auto kern, int V, auto... second) {
                 const int nxb = (int)((nlane + 64 * V - 1) / (64 * V));
-                const size_t shm = (size_t)2 * B * NT * V * sizeof(double);
+                const size_t shm = ((size_t)4 * Q * NT + XCH_FLAGS) * V * sizeof(double);
+                allow_lds(kern, shm);
                 hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf, nz), dim3(NT), shm, st, p, f, (int)sd, so,
                                    (int)nlane, nxb, dim == 2 ? 1 : 0, e, mf, second...);
             };
@@ -1808,7 +1839,7 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
             if (p.cap == 12 || p.cap == 24) throw Error{CLES_ERR_INVALID, "plan built for another line kernel"};
             const int NT = Lx * P;
             const int nxb = (int)((nlane + Lx - 1) / Lx);
-            const size_t shm = (size_t)2 * B * NT * sizeof(double);
+            const size_t shm = ((size_t)4 * Q * NT + XCH_FLAGS) * sizeof(double);
             auto go = [&](auto kern, auto... second) {
                 hipLaunchKernelGGL(kern, dim3((unsigned)(nxb * nouter), nf, nz), dim3(NT), shm, st, p, f, (int)sd, so,
                                    (int)nlane, nxb, Lx, e, mf, second...);

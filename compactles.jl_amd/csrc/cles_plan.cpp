@@ -316,8 +316,9 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     // what it leaves out is at most 1e-20 of the line's largest interface
     // value, four decades below half an ulp of it.  The step it saves costs an
     // exchange through LDS (or shuffles) on the critical path of every kernel.
-    // (A NaN or an infinity in a line therefore reaches the chunks within the
-    // kept steps' reach, not always the whole line.)
+    // A NaN or an infinity, which no coefficient makes small, would then stay
+    // within the kept steps' reach: the kernels spread it over its line (in
+    // blocks, by way of the first step's barrier, so that one step is kept).
     constexpr long double PCR_DROP = 1e-20L;
     std::vector<Mat> D(P, mat_eye(B)), L = Lb, U = Ub;
     std::vector<double> pcr;
@@ -348,7 +349,7 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
                 largest = std::max({largest, std::fabs(alpha[i]), std::fabs(beta[i])});
             }
         }
-        if (largest < PCR_DROP) {
+        if (largest < PCR_DROP && st > 0) {
             nsteps = st;
             decoupled = true;
             steps.resize((size_t)nsteps * P * 2 * B * B);

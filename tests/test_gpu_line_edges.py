@@ -173,3 +173,36 @@ def test_long_closures_on_short_chunks(ctx, half, lanes, dtype, bar):  # noqa: F
             ch.apply_along_(out, plan, ch.DeviceArray.from_numpy(ctx, Hh.pad(f, n), dtype), dec)
             ref = np.moveaxis(np.tensordot(D, f, (1, dim - 1)), 0, dim - 1)
             assert Hh.relerr(Hh.interior(out.numpy().astype(np.float64), n), ref) <= bar, (line, dim)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("dim,n", [(1, (256, 6, 5)), (1, (512, 6, 5)), (1, (500, 6, 5)), (1, (768, 3, 2)),
+                                   (1, (2000, 5, 3)), (2, (64, 512, 3)), (3, (50, 2, 300)), (2, (6, 900, 2)),
+                                   (3, (3, 2, 700)), (2, (128, 128, 512)), (2, (128, 500, 520))])
+def test_non_finite_value_spreads_over_its_line(ctx, dim, n, periodic, bad):  # noqa: F811
+    """Also where the reduction stops early, a NaN or an infinity leaves no
+    finite value on its line, as the sweeps over the whole line would, and
+    changes no other line."""
+    import compactles_hip as ch
+    at = [n[0] // 2, n[1] // 2, n[2] // 2]
+    at[dim - 1] = n[dim - 1] // 3
+    line = list(at)
+    line[dim - 1] = slice(None)
+    line = tuple(line)
+    f = Hh.random_field(n, seed=81)
+    g = f.copy(order="F")
+    g[tuple(at)] = bad
+    dec = ch.Decomp(n, (periodic,) * 3, n_halo=0)
+    for dtype in (np.float64, np.float32):
+        for scheme in (ch.lele_d1_6(), ch.lele_d1_10(), ch.compact_filter()):
+            plan = ch.plan_direction(ctx, dec, scheme, dim, 0.1, dtype=dtype)
+            res = []
+            for a in (f, g):
+                out = ch.field(ctx, dec, dtype)
+                ch.apply_along_(out, plan, ch.DeviceArray.from_numpy(ctx, a, dtype), dec)
+                res.append(out.numpy())
+            assert not np.isfinite(res[1][line]).any(), (dtype, scheme.name)
+            for a in res:
+                a[line] = 0
+            assert np.array_equal(res[0], res[1]), (dtype, scheme.name)
