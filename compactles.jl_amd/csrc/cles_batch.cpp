@@ -747,7 +747,7 @@ static void move_instance(cles_batch *b, int64_t i, double *Qh, const int64_t pa
     const size_t n = (size_t)b->n[i];
     double *dev = b->Q + b->off[i], *host = Qh + halo[0];
     std::lock_guard<std::mutex> lk(b->io_mu);
-    CLES_HIP(hipSetDevice(b->ctx->device));
+    cles::DeviceScope on(b->ctx->device);
     const int nmax = *std::max_element(b->n.begin(), b->n.end());
     double *buf = (double *)b->io_buf.get(sizeof(double) * (size_t)nmax * b->C);
     if (!b->io_buf.pinned) {

@@ -143,6 +143,17 @@ struct View3 {
 // ---------------------------------------------------------------------------
 // Host transfers (cles_stage.cpp)
 // ---------------------------------------------------------------------------
+// Makes `device` the calling thread's current device for the scope.
+class DeviceScope {
+    int before = -1;
+
+public:
+    explicit DeviceScope(int device);
+    ~DeviceScope();
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+};
+
 // A pinned host buffer that grows on demand (pageable where no pinned memory
 // is to be had: `pinned` tells).
 struct PinnedBuf {

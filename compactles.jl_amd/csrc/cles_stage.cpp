@@ -32,6 +32,20 @@ void check(hipError_t e, const char *what)
 }
 }  // namespace
 
+DeviceScope::DeviceScope(int device)
+{
+    int now = -1;
+    check(hipGetDevice(&now), "hipGetDevice");
+    if (now == device) return;
+    check(hipSetDevice(device), "hipSetDevice");
+    before = now;
+}
+
+DeviceScope::~DeviceScope()
+{
+    if (before >= 0) (void)hipSetDevice(before);
+}
+
 PinnedBuf::~PinnedBuf() { release(); }
 
 void PinnedBuf::release()
@@ -128,7 +142,7 @@ void HostStage::transfer(bool down, int device, hipStream_t st, double *dev, con
     std::vector<Error> failed((size_t)nlane, Error{CLES_OK, ""});
     auto guarded = [&](int w) {
         try {
-            check(hipSetDevice(device), "hipSetDevice");
+            DeviceScope on(device);   // lane 0 and lanes without a thread run on the caller's
             work(w);
         } catch (const Error &e) {
             failed[w] = e;
