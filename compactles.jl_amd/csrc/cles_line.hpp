@@ -33,6 +33,7 @@
 namespace cles {
 
 constexpr int MC = 32;     // maximum chunk length (points per thread)
+constexpr int YZU_THREADS = 1024;   // threads of a one-chunk-per-wave y / z block at most
 constexpr int NCMAX = 4;   // closure rows per edge handled by the kernels
 
 // Plan tables live in global memory; a pointer read out of memory (the ragged
@@ -1033,7 +1034,7 @@ template <typename T, int Q, int M, int EPI, int CL, bool FULL, int V> constexpr
 }
 
 template <typename T, int Q, int M, int SYM, int EPI, int CL, bool FULL, int V>
-__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, (yzu_waves<T, Q, M, EPI, CL, FULL, V>()))
+__global__ void __launch_bounds__(1024, (yzu_waves<T, Q, M, EPI, CL, FULL, V>()))
 k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
            LineFields mf)
 {
@@ -1046,7 +1047,7 @@ k_line_yzu(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane, in
 // arguments nor the choice between the plans (C6 gradient of 33 x 29 x 31 FP64,
 // three plain launches: 21.2 us a pass with one kernel for both, 20.5 so).
 template <typename T, int Q, int M, int SYM, int CL, bool FULL, int V>
-__global__ void __launch_bounds__(Q == 1 ? 1024 : 512, (yzu_waves<T, Q, M, EPI_STORE, CL, FULL, V>()))
+__global__ void __launch_bounds__(1024, (yzu_waves<T, Q, M, EPI_STORE, CL, FULL, V>()))
 k_line_yzu_pair(LineDev p1, const T *__restrict__ f, int sd, int64_t so, int nlane, int nxb, int slabs, EpiArgs e,
                 LineFields mf, LineSecond two)
 {
@@ -1150,8 +1151,12 @@ __device__ __forceinline__ void line_yz(const LineDev &p, const T *__restrict__ 
     }
 }
 
+// Waves per SIMD: three, but the pentadiagonal sweep of 32-point chunks spills 160
+// registers there and 64 at two (C10 of 100 x 2000 FP64 along y 42.7 / 28.6 us).
+template <int Q, int CL> constexpr int yz_waves() { return Q == 2 && CL > 16 ? 2 : 3; }
+
 template <typename T, int Q, int M, int SYM, int EPI, int CL>
-__global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane,
+__global__ void __launch_bounds__(512, (yz_waves<Q, CL>())) k_line_yz(LineDev p, const T *__restrict__ f, int sd, int64_t so, int nlane,
                                                     int nxb, int Lx, EpiArgs e, LineFields mf)
 {
     select_field<T, EPI>(mf, f, e);
@@ -1160,7 +1165,7 @@ __global__ void __launch_bounds__(512, 3) k_line_yz(LineDev p, const T *__restri
 
 // The y and z directions in one launch, as k_line_yzu_pair.
 template <typename T, int Q, int M, int SYM, int CL>
-__global__ void __launch_bounds__(512, 3) k_line_yz_pair(LineDev p1, const T *__restrict__ f, int sd, int64_t so,
+__global__ void __launch_bounds__(512, (yz_waves<Q, CL>())) k_line_yz_pair(LineDev p1, const T *__restrict__ f, int sd, int64_t so,
                                                          int nlane, int nxb, int Lx, EpiArgs e, LineFields mf,
                                                          LineSecond two)
 {
@@ -1714,7 +1719,6 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
 
     const int P = p.P;
     const size_t lim = lds_limit();
-    const int maxNT = Q == 1 ? 1024 : 512;
     if (dim == 1 && p.extra == 0 && p.m == XCL && P == 16 && p.periodic) {
         // 256-point lines: four per wave
         const int64_t nlines = v.n[1] * v.n[2];
@@ -1792,7 +1796,7 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         const unsigned nz = hp2 ? 2 : 1;
         const int64_t nouter = dim == 2 ? (hp2 ? std::max(v.n[1], v.n[2]) : v.n[2]) : v.n[1];
         if ((int64_t)(p.n - 1) * sd > INT32_MAX) throw Error{CLES_ERR_UNSUPPORTED, "array too large for 32-bit line offsets"};
-        if (nlane >= 48 && 64 * P <= maxNT) {
+        if (nlane >= 48 && 64 * P <= YZU_THREADS) {
             const int NT = 64 * P;
             const bool full = p.extra == 0 && p.m == p.cap && (!hp2 || (two.p.extra == 0 && two.p.m == two.p.cap));
             auto go = [&](auto kern, int V, auto... second) {

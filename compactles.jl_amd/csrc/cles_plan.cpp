@@ -434,7 +434,7 @@ void build_line_tables(LineTables &out, const cles_scheme_desc &s, int n, int pe
     // the wave-local x sweep and the one-chunk-per-wave y / z sweeps also come in
     // the capacities 12 and 24 (a sweep runs cap steps however short its chunks); in
     // x from 16 chunks on, below which a wave stages up to 16 values per lane
-    const bool fine = !pool && (dim == 1 ? P >= 16 && P <= 64 && longest <= 16 : lanes >= 48 && 64 * P <= (q == 1 ? 1024 : 512));
+    const bool fine = !pool && (dim == 1 ? P >= 16 && P <= 64 && longest <= 16 : lanes >= 48 && 64 * P <= 1024);
     int cap = longest <= 8 && !pool ? 8 : longest <= 16 ? 16 : 32;
     if (fine && cap == 16 && longest <= 12) cap = 12;
     if (fine && cap == 32 && longest <= 24) cap = 24;
