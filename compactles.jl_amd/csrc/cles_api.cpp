@@ -158,12 +158,8 @@ int cles_plan_create(cles_ctx *ctx, const cles_scheme_desc *scheme, int dim, con
         p->hp.dtype = dtype;
         for (int d = 0; d < 3; d++) p->hp.nloc[d] = n_local[d];
         try {
-            // the solver's rule, as long as a line stays within 64 chunks (one
-            // wave in x): 33 x 29 x 31 FP64 took one 29-point chunk per y line
             const int64_t n = n_local[dim - 1], lines = n_local[0] * n_local[1] * n_local[2] / n;
-            const int most = dim == 1 ? 16 : 32;
-            int chunk = cles::default_line_chunk(dim, n, lines, periodic);
-            while (chunk < most && n > (int64_t)chunk * 64) chunk *= 2;
+            const int chunk = cles::operator_line_chunk(dim, n, lines, n_local[0], periodic);
             cles::build_line_plan(p->hp, *scheme, (int)n, periodic, h, chunk, lo_fold, hi_fold);
         } catch (...) {
             delete p;

@@ -268,6 +268,9 @@ inline constexpr double LSRK_C[5] = {0.0, 1432997174477.0 / 9575080441755.0, 252
 int line_chunk(int dim, const cles_solver_desc &d, bool *tuned = nullptr);
 // Chunk length by line length, line count and periodicity (cles_tune.cpp).
 int default_line_chunk(int dim, int64_t n_line, int64_t lines, bool periodic);
+// The same for operator plans, whose launches hold one field (cles_tune.cpp);
+// lanes: extent along x.
+int operator_line_chunk(int dim, int64_t n_line, int64_t lines, int64_t lanes, bool periodic);
 
 // Ragged batch of independent lines (one line per instance, each with its own
 // length and plan), laid end to end: instance i occupies [off[i], off[i]+n).

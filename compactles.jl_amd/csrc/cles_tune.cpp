@@ -86,6 +86,27 @@ int default_line_chunk(int dim, int64_t n_line, int64_t lines, bool periodic)
     return c;
 }
 
+// Operator plans: one field per launch, any scheme, so the rule above, measured on
+// a solver's groups of C6 launches, holds for few lines only.  Per launch:
+//  * y / z, 48 lanes and 4096 lines or more: the shortest of 16 and 32 points that
+//    keeps a line of up to 256 within 8 chunks, hence a block within 512 threads.
+//    Sixteen chunks fill a 1024-thread block, of which a CU mostly holds one: C8
+//    filter of 144^3 FP32 along z 10.0 us with 32 points and 14.3 with 16, C10 of
+//    160^3 FP64 along y 18.0 / 25.1.  Up to 128 points 16 wins by less: C10 of
+//    64^3 FP64 along z 5.7 with 16, 6.5 with 32 and 6.0 with 8, of 100^3 8.6 / 9.1 /
+//    9.6;
+//  * x, periodic lines of 256 points: 16, which k_line_xwf runs (256 x 256 FP32
+//    C10 5.1 / 6.0 us with 8);
+//  * otherwise the solver's rule, with at most 64 chunks per line.
+int operator_line_chunk(int dim, int64_t n_line, int64_t lines, int64_t lanes, bool periodic)
+{
+    if (dim > 1 && lanes >= 48 && lines >= SOME_LINES) return n_line <= 128 ? 16 : 32;
+    if (dim == 1 && periodic && n_line == 256) return 16;
+    int c = default_line_chunk(dim, n_line, lines, periodic);
+    while (c < cap_of(dim) && n_line > (int64_t)c * 64) c *= 2;
+    return c;
+}
+
 int line_chunk(int dim, const cles_solver_desc &d, bool *tuned)
 {
     {

@@ -38,3 +38,19 @@ def relerr(a, ref):
 def random_field(n, seed=0):
     rng = np.random.default_rng(seed)
     return np.asfortranarray(rng.standard_normal(n))
+
+
+def run_internal(tmp_path, program, args=()):
+    """Builds a C++ program against the library's internal header, links it with
+    the library and returns what it prints (host code only)."""
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    pkg = os.path.join(root, "compactles.jl_amd")
+    src, exe = tmp_path / "program.cpp", tmp_path / "program"
+    src.write_text(program)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(root, "include"), "-I" + os.path.join(pkg, "csrc"), str(src), "-L" + pkg,
+                    "-l:libcompactles_hip.so", "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{pkg}:/opt/rocm/lib",
+                    "-o", str(exe)], check=True)
+    return subprocess.run([str(exe), *args], check=True, capture_output=True, text=True, timeout=60).stdout
