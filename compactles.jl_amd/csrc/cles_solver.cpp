@@ -434,8 +434,9 @@ struct Impl {
     // every field of one direction in one launch
     void velocity_gradients(bool scalars = false) const
     {
-        // y and z in one launch where they take the same kernel
-        const bool yz = s.nact >= 2 && s.active[1] && s.active[2] && !s.fold[1].on && !s.fold[2].on;
+        // y and z in one launch where they take the same kernel (profiling
+        // times the directions apart)
+        const bool yz = s.nact >= 2 && s.active[1] && s.active[2] && !s.fold[1].on && !s.fold[2].on && !s.prof;
         for (int k = 0; k < s.nact; k++) {
             const int d = s.adim[k];
             if (d == 1 && yz) {
@@ -450,9 +451,7 @@ struct Impl {
                         mf.in[y.nf + i] = z.in[i];
                         mf.out[y.nf + i] = z.out[i];
                     }
-                    s.timed(PH_DERIV + 1, line_bytes(s.dplan[1], EPI_STORE) * (double)s.N * 2 * y.nf, [&] {
-                        launch_line(s.dplan[1], 2, view(), mf.in[0], store(mf.out[0]), s.st(), &mf, &s.dplan[2]);
-                    });
+                    launch_line(s.dplan[1], 2, view(), mf.in[0], store(mf.out[0]), s.st(), &mf, &s.dplan[2]);
                     for (int dd = 1; dd <= 2; dd++) {
                         GradList g = dd == 1 ? y : z;
                         if (s.met.m[dd] || s.curv) metric(g.out, g.nf, 0, dd);

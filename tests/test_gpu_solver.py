@@ -210,3 +210,26 @@ def test_rhs_step_filter_256_point_x_lines(ctx, walls):
     gs.download(Qg)
     for c in range(5):
         assert Hh.relerr(Hh.interior(Qg[..., c], n), os_.interior(os_.Q[..., c])) <= 1e-12, c
+
+
+def test_profile_times_every_direction(ctx):
+    """The per-phase timing keeps the gradients' directions apart, also on grids
+    where the y and z gradients otherwise share a launch, and the step is the
+    same with and without it."""
+    import cases
+    n, L = (24, 20, 20), (2 * np.pi,) * 3
+    X, Y, Z = cases.grid(n, L)
+    q = cases.conserved(cases.smooth_prim(X, Y, Z))
+    states = []
+    for profiled in (False, True):
+        s = cases.gpu_solver(ctx, n, L, q)
+        s.profile(profiled)
+        s.step(1e-3)
+        phases = s.profile_read()
+        if profiled:
+            assert [phases[f"line_deriv_{d}"][1] for d in "xyz"] == [5, 5, 5]
+        Q = s.allocate_state()
+        s.download(Q)
+        states.append(Q)
+        s.close()
+    assert np.isfinite(states[0]).all() and np.array_equal(states[0], states[1])
