@@ -61,6 +61,16 @@ def _cpu_model():
     return "unknown"
 
 
+def read_step_traffic(n, precision):
+    """HBM bytes per point and step of all kernels, counted in the same summary
+    as read_traffic's, or None."""
+    path = os.path.join(ROOT, "profiles", f"tgv{n}_{precision}_hbm_counters.md")
+    if not os.path.exists(path):
+        return None
+    m = re.search(r"(?m)^Measured HBM traffic per step \(all kernels\): [0-9.]+ GB = ([0-9.]+) B/pt", open(path).read())
+    return float(m.group(1)) if m else None
+
+
 def cpu_baseline(n, steps=3, warmup=1):
     """The oracle (the C restatement of the reference CPU path, the checker of
     the tests, loaded only here) on the host cores: `warmup` untimed and
@@ -162,6 +172,7 @@ def measure(ch, ctx, n, precision, steps, warmup, profile_steps, run_mode="host_
     achieved = alg_per_launch / (avg_ms * 1e-3) / 1e9 if launches else 0.0
     total_ms = sum(v[0] for v in phases.values())
     step_alg = alg_bytes_per_point_step(1, 3, precision) * npts
+    counted = read_step_traffic(n, precision)   # the kernels move less than the reference's dataflow
     solver.close()
     return {
         "value": round(value, 3), "ms_per_step": round(ms_per_step, 4), "ke": ke, "enstrophy": ens,
@@ -174,7 +185,10 @@ def measure(ch, ctx, n, precision, steps, warmup, profile_steps, run_mode="host_
         "step_roofline": {"alg_bytes_per_point_step": alg_bytes_per_point_step(1, 3, precision),
                           "alg_bytes_per_step": step_alg,
                           "achieved_GBps": round(step_alg / (ms_per_step * 1e-3) / 1e9, 1),
-                          "frac": round(step_alg / (ms_per_step * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)},
+                          "frac": round(step_alg / (ms_per_step * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
+                          "counted_bytes_per_point_step": counted,
+                          "counted_frac": counted and round(counted * npts / (ms_per_step * 1e-3) / 1e9
+                                                            / HBM_PEAK_GBPS, 4)},
         "phases_ms_per_step": {k: round(v[0] / profile_steps, 3) for k, v in
                                sorted(phases.items(), key=lambda kv: -kv[1][0])},
         "phases_GBps": {k: round(v[2] / (v[0] * 1e-3) / 1e9, 1) for k, v in phases.items() if v[0] > 0},

@@ -276,13 +276,14 @@ struct Impl {
         return g;
     }
     // algorithmic bytes per point of one line operator with epilogue kind
-    double line_bytes(const HostPlan &hp, int kind) const
+    double line_bytes(const HostPlan &hp, const EpiArgs &e) const
     {
         const double w = hp.dtype == CLES_F64 ? 8.0 : 4.0;
-        switch (kind) {
+        switch (e.kind) {
         case EPI_SUB: return 3 * w;                 // read f, read-modify-write out
         case EPI_LSRK:
-        case EPI_LSRK_DEV: return 2 * w + 32;       // f, dQ; du and Q read + written
+        case EPI_LSRK_DEV:                          // f, dQ; du and Q read + written (A = 0: du not read)
+            return 2 * w + (e.c0 != 0.0 ? 32 : 24);
         case EPI_ART_MUBETA: return 4 * w;          // sensor, rho -> mu, beta
         case EPI_ART_KAPPA: return 5 * w;           // sensor, rho, c, T -> kappa
         case EPI_ART_D: return 3 * w;               // sensor, c -> D
@@ -293,7 +294,7 @@ struct Impl {
     }
     void line(const HostPlan &hp, int d, const void *in, EpiArgs e, int phase) const
     {
-        s.timed(phase + d, line_bytes(hp, e.kind) * (double)s.N,
+        s.timed(phase + d, line_bytes(hp, e) * (double)s.N,
                 [&] { launch_line(hp, d + 1, view(), in, e, s.st()); });
     }
     // one launch over nf independent fields: field i reads in[i] and writes
@@ -309,7 +310,7 @@ struct Impl {
             if (eoff) mf.eoff[i] = eoff[i];
         }
         if (out) e.out = out[0];
-        s.timed(phase + d, line_bytes(hp, e.kind) * (double)s.N * nf,
+        s.timed(phase + d, line_bytes(hp, e) * (double)s.N * nf,
                 [&] { launch_line(hp, d + 1, view(), in[0], e, s.st(), &mf); });
     }
     // equations.jl:56-66 parities across the fold of dimension d (the axis:
@@ -825,7 +826,7 @@ struct Impl {
 
     void lsrk_all(double A, double B, double dt) const
     {
-        s.timed(PH_LSRK, (32.0 + sizeof(W)) * s.C * (double)s.N,
+        s.timed(PH_LSRK, ((A != 0.0 ? 32.0 : 24.0) + sizeof(W)) * s.C * (double)s.N,
                 [&] { launch_lsrk<W>(s.Q, s.du, f(s.dQ), A, B, dt, s.dev_dt, s.dev_gate, (int64_t)s.C * s.N, s.N,
                                      s.ipts, s.st()); });
     }

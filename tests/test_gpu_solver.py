@@ -233,3 +233,18 @@ def test_profile_times_every_direction(ctx):
         states.append(Q)
         s.close()
     assert np.isfinite(states[0]).all() and np.array_equal(states[0], states[1])
+
+
+def test_profile_bytes_of_the_fused_update(ctx):
+    """The bytes booked for the divergence fused with the Runge-Kutta update: f
+    and dQ, Q twice, and the register twice but for the first stage, which only
+    writes it."""
+    import cases
+    n, L = (24, 20, 20), (2 * np.pi,) * 3
+    X, Y, Z = cases.grid(n, L)
+    s = cases.gpu_solver(ctx, n, L, cases.conserved(cases.smooth_prim(X, Y, Z)))
+    s.profile(True)
+    s.step(1e-3)
+    _, launches, moved = s.profile_read()["line_div_lsrk_z"]
+    s.close()
+    assert launches == 5 and moved == 5 * 24 * 20 * 20 * (5 * 16 + 4 * 32 + 24)
