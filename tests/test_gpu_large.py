@@ -1,9 +1,9 @@
 """The solver path at a size where launches write more than the 256 MB
-Infinity Cache holds, so the kernels take their non-temporal store variants
-(the fluxes: 15 fields; the z sweeps' four-field gradient launches): one RHS
-and one step at 210 x 208 x 206 (9.0 M points) against the oracle on the same
-inputs (dQ and the primitives 1e-12, the sensor-fed coefficients 1e-9, the
-stepped state 1e-12)."""
+Infinity Cache holds, so the pointwise kernels take their non-temporal store
+variants (the fluxes: 15 fields; the primitives: 7): one RHS and one step at
+210 x 208 x 206 (9.0 M points) against the oracle on the same inputs (dQ and
+the primitives 1e-12, the sensor-fed coefficients 1e-9, the stepped state
+1e-12)."""
 import numpy as np
 import pytest
 
@@ -25,7 +25,7 @@ def ctx():
 def test_rhs_and_step_above_cache_size(ctx):
     n, L = (210, 208, 206), (TWO_PI,) * 3
     N = n[0] * n[1] * n[2]
-    assert N * 8 * 15 > 256 * 2 ** 20 and N * 8 * 4 > 256 * 2 ** 20   # fluxes and z-sweep gradients
+    assert N * 8 * 7 > 256 * 2 ** 20   # the primitives; the fluxes write 15 fields
     X, Y, Z = cases.grid(n, L)
     q = cases.conserved(cases.smooth_prim(X, Y, Z))
     del X, Y, Z

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import helpers as Hh
+import line_shapes as S
 from test_gpu_operators import _gpu_apply, _oracle_apply, ctx  # noqa: F401
 from test_gpu_solver import _compare_rhs
 
@@ -206,3 +207,76 @@ def test_non_finite_value_spreads_over_its_line(ctx, dim, n, periodic, bad):  # 
             for a in res:
                 a[line] = 0
             assert np.array_equal(res[0], res[1]), (dtype, scheme.name)
+
+
+def _check(ctx, names, dims, n_of, periodic, dtype, bar, seed):
+    for dim in dims:
+        n = n_of(dim)
+        f = Hh.random_field(n, seed=seed).astype(dtype).astype(np.float64)
+        for name in names:
+            ref = _oracle_apply(name, dim, n, periodic, 0.1, f)
+            got = _gpu_apply(ctx, name, dim, n, periodic, 0.1, f, dtype=dtype)
+            assert Hh.relerr(got, ref) <= bar, (name, n, dim)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("line,cap,whole", S.WIDE_LINES)
+def test_wide_capacities(ctx, line, cap, whole, periodic, dtype, bar):  # noqa: F811
+    """Wide y / z launches at every chunk capacity, whole and uneven chunks, one
+    line per lane (which shapes give which: test_line_rule_host)."""
+    _check(ctx, ("lele_d1_6", "lele_d1_10", "compact_filter"), (2, 3), lambda d: S.wide(line, d), periodic, dtype, bar, 91)
+
+
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("line", [48, 60, 64, 130, 192, 256])
+def test_wide_capacities_two_lines_per_lane(ctx, line, periodic):  # noqa: F811
+    """As above in FP32 with even rows and 512 blocks: two lines per lane."""
+    _check(ctx, ("lele_d1_6", "compact_filter"), (2,), lambda d: S.wide(line, d, 48, 512), periodic, np.float32, 2e-5, 92)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("line,cap,whole", S.FEW_LINES)
+def test_few_lines_capacity_8(ctx, line, cap, whole, periodic, dtype, bar):  # noqa: F811
+    """y / z launches of few lines: 8-point chunks."""
+    _check(ctx, ("lele_d1_6", "lele_d1_10", "compact_filter"), (2, 3), lambda d: S.wide(line, d, 49, 7), periodic, dtype,
+           bar, 93)
+
+
+@pytest.mark.parametrize("dtype,bar", [(np.float64, 1e-12), (np.float32, 2e-5)])
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("line,cap,whole", S.X_LINES)
+def test_x_capacity_12(ctx, line, cap, whole, periodic, dtype, bar):  # noqa: F811
+    """x lines of 64 chunks at capacity 12: uneven, equal and whole chunks."""
+    _check(ctx, ("lele_d1_6", "pade_d1_4", "lele_d1_10", "compact_filter"), (1,), lambda d: (line, 5, 3), periodic, dtype,
+           bar, 94)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,periodic_y,species,paired", S.PAIRS)
+def test_paired_gradients_are_the_separate_ones(ctx, n, periodic_y, species, paired, precision):  # noqa: F811
+    """The y and z gradients of one launch against the same ones launched
+    direction by direction (per-phase timing on): the same bits, also where one
+    direction is closed and the other periodic and, on 64^3 FP32, with two lines
+    per lane."""
+    import cases
+    L = (2 * np.pi,) * 3
+    X, Y, Z = cases.grid(n, L)
+    kw = {} if periodic_y else {"bcs": ((0, 0), (1, 1), (0, 0))}   # slip walls in y
+    if species == 2:
+        th = 0.5 * (1 + 0.5 * np.sin(X + Y) * np.cos(Z))
+        q = cases.conserved(cases.smooth_prim(X, Y, Z), species=cases.HE_CO2, Y=[1 - th, th])
+        kw["species"] = cases.HE_CO2
+    else:
+        q = cases.conserved(cases.smooth_prim(X, Y, Z))
+    got = []
+    for apart in (False, True):
+        s = cases.gpu_solver(ctx, n, L, q, precision=precision, **kw)
+        s.profile(apart)
+        s.compute_rhs(False)
+        got.append([s.field(f"grad_u[{d}{j}]") for d in (1, 2, 3) for j in (1, 2, 3)] +
+                   [s.field(f"grad_T[{d}]") for d in (1, 2, 3)])
+        s.close()
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
