@@ -304,7 +304,10 @@ int cles_solver_switch_bc(cles_solver *solver, int dim, int side);
 int cles_solver_bc_switched(cles_solver *solver, int dim, int side, int *switched);
 
 /* Conserved state transfer in Julia's padded layout (Q[..., c], column-major,
- * extents padded[3], interior offset halo[3], n_cons components). */
+ * extents padded[3], interior offset halo[3], n_cons components).  The solver
+ * keeps pinned host buffers for it from the first transfer on (at most 48 MB
+ * unless a row is longer than 4 MB), host memory that cles_solver_footprint does
+ * not count. */
 int cles_solver_upload(cles_solver *solver, const double *Q_host,
                        const int64_t padded[3], const int halo[3]);
 int cles_solver_download(cles_solver *solver, double *Q_host,
@@ -379,7 +382,8 @@ int cles_diagnostics(cles_solver *solver, double *ke, double *enstrophy);
 
 /* Per-phase timing of the solver's launches with HIP events on its stream
  * (phases modelled on bench/phases.jl:119-193; adds a few microseconds per
- * launch, so leave it off for throughput runs).  enable = 1 starts a fresh
+ * launch and launches the y and z gradients apart, so leave it off for
+ * throughput runs).  enable = 1 starts a fresh
  * accumulation, 0 stops.  cles_solver_profile_read returns phase `index`
  * (name, total milliseconds, launches, algorithmic bytes moved) and
  * CLES_ERR_INVALID past the last phase. */
