@@ -118,3 +118,16 @@ def test_run_modes_timing_small_grids(ctx):
         print(f"\nTGV {n}^3 ms/step: " + ", ".join(f"{k} {v:.3f}" for k, v in out.items()))
         assert out["step_graph"] < 1.5 * out["host_dt"]
 
+
+
+def test_graph_of_blocks_above_64_kb(ctx):
+    """y lines of 384 points in 16 chunks, two FP32 lines per lane: the blocks'
+    exchange buffers take more than 64 KB of LDS, also in a captured launch."""
+    n = (128, 384, 128)
+    a, b = _tgv(ctx, n, "fp32"), _tgv(ctx, n, "fp32")
+    a.set_run_mode("step_graph")
+    b.set_run_mode("host_dt")
+    da = np.concatenate([a.run(1e9, 2, record=2), a.run(1e9, 5, record=3)])
+    db = b.run(1e9, 5, record=5)
+    assert np.array_equal(da, db)
+    assert np.array_equal(_state(a), _state(b))
