@@ -1742,11 +1742,13 @@ void launch_variant(const HostPlan &hp, int dim, const View3 &v, const T *f, con
         };
         auto pick = [&](auto xcv) {
             constexpr int XC = xcv.value;
+            // plans take capacity 12 from 16 chunks on, hence lines of 129 points or more
+            constexpr bool WIDE_ONLY = XC == 12;
             if (uni && lsh == 6 && p.m == XC) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, true, true>, XC);
-            else if (uni && lsh == 6) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, false, true>, XC);
-            else if (uni) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, false, false>, XC);
-            else if (lsh == 6) go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, true>, XC);
-            else go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, false>, XC);
+            else if (uni && (WIDE_ONLY || lsh == 6)) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, false, true>, XC);
+            else if (uni) go(k_line_xw<T, Q, M, SYM, EPI, true, XC, false, WIDE_ONLY>, XC);
+            else if (WIDE_ONLY || lsh == 6) go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, true>, XC);
+            else go(k_line_xw<T, Q, M, SYM, EPI, false, XC, false, WIDE_ONLY>, XC);
         };
         if (p.cap == 8) pick(std::integral_constant<int, 8>{});
         else if (p.cap == 12) pick(std::integral_constant<int, 12>{});
